@@ -317,8 +317,7 @@ def tuned_tiles(cfdx, cdef, precision, mach, prm):
 
 def graph_steps(cfdx, block, ctx, tiles=None):
     """A one-block batch around `block` whose step(n) replays a captured RK3-step graph: the
-    library's graph path for a single block (the mixed form's viscous/face overlap becomes graph
-    edges instead of stream events: 3-4 % faster mixed, FP64 unchanged). The block keeps its
+    library's graph path for a single block. The block keeps its
     state and run parameters; remove it (q.remove, q.close) to step it directly again."""
     q = cfdx.Batch(block.precision, ctx)
     q.add(block)

@@ -440,7 +440,7 @@ class Ctx:
         return f.value, t.value
 
     def set_overlap(self, on: bool) -> None:
-        """Mixed-precision stages run the viscous kernel beside the face sweeps on a second stream
+        """A stage's viscous kernel and face sweeps run together, in one launch or on two streams
         (cfdx_ctx_set_overlap; on by default)."""
         _check(_lib.cfdx_ctx_set_overlap(self.h, 1 if on else 0))
 

@@ -22,7 +22,11 @@ ARCH = os.environ.get("CFDX_ARCH", "gfx950")
 
 COMMON = ["-O3", "-std=c++17", "-fPIC", "-Wall", "-Wno-unused-function", "-Wno-address-of-packed-member"]
 HIPFLAGS = [f"--offload-arch={ARCH}", "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops",
-            "-munsafe-fp-atomics"]
+            "-munsafe-fp-atomics",
+            # products and sums are fused where they stand in one expression, never later by what the
+            # optimiser sees around them: a block's bits then do not depend on which kernel form (tile
+            # shape, bounded or periodic list, launch together or apart) computes it
+            "-ffp-contract=on"]
 
 
 def _run(cmd, verbose):

@@ -272,28 +272,21 @@ uint32_t mon_triples(const BlockDev &B, const cfdx::blk::TileCfg &t)
     return cfdx::blk::tiles_of(B, 0, t) * (uint32_t)(tx * ty / 64) + (cfdx::blk::shell_count(B) + 63) / 64;
 }
 
-// the overlap of a stage's viscous kernel with its face sweeps on a context that allows it: for
-// mixed-precision work always; for FP64 work only inside a captured graph (the FP64 sweeps hold
-// 3 waves per SIMD at ~160 VGPRs, which leaves few registers for a viscous wave beside them:
-// with stream events the overlap measured no gain, as graph edges 1 % at 128^3)
-cfdx::blk::Overlap overlap_of(const cfdx_ctx *ctx)
+// the context's second stream, for a stage's viscous kernel beside its face sweeps; null with the overlap
+// switched off (one kernel after the other)
+const cfdx::blk::Overlap *overlap_of(const cfdx_ctx *ctx, cfdx::blk::Overlap &ov)
 {
-    return cfdx::blk::Overlap{ctx->aux, ctx->fork, ctx->join, (uint32_t)std::max(ctx->n_cu, 1)};
-}
-
-const cfdx::blk::Overlap *overlap_if(const cfdx_ctx *ctx, int precision, const cfdx::blk::Overlap &ov,
-                                     bool graph = false)
-{
-    return (ctx->overlap && (precision == CFDX_MIXED || graph)) ? &ov : nullptr;
+    ov = cfdx::blk::Overlap{ctx->aux, ctx->fork, ctx->join};
+    return ctx->overlap ? &ov : nullptr;
 }
 
 int run_stage(cfdx_block *b, int mode)
 {
     const LaunchList L = single_list(b);
     if (mode == 2) b->mon_count = mon_triples(b->B, b->tiles);
-    const cfdx::blk::Overlap ov = overlap_of(b->ctx);
+    cfdx::blk::Overlap ov;
     cfdx::blk::stage(L, b->desc.precision, mode, b->ctx->stream, b->B.viscous != 0, b->timing ? b->ev : nullptr,
-                     overlap_if(b->ctx, b->desc.precision, ov));
+                     overlap_of(b->ctx, ov));
     b->launches += (b->B.viscous ? 5 : 4);
     CFDX_TRY(cfdx::check_launch("block stage"));
     if (b->timing) {
@@ -1019,11 +1012,11 @@ extern "C" int cfdx_batch_step(cfdx_batch *q, int nsteps, int use_graph)
     CFDX_TRY(upload_batch(q));
     for (cfdx_block *b : q->blocks) b->mon_count = mon_triples(b->B, q->tiles);
     hipStream_t st = q->ctx->stream;
-    const cfdx::blk::Overlap ov = overlap_of(q->ctx);
+    cfdx::blk::Overlap ov;
     if (!use_graph) {
         for (int s = 0; s < nsteps; ++s)
             for (int j = 0; j < 3; ++j)
-                cfdx::blk::stage(q->L, q->precision, j, st, q->any_visc, nullptr, overlap_if(q->ctx, q->precision, ov));
+                cfdx::blk::stage(q->L, q->precision, j, st, q->any_visc, nullptr, overlap_of(q->ctx, ov));
         return cfdx::check_launch("batch stage");
     }
     if (q->exec && q->graph_gen != q->ctx->gen.load()) drop_graph(q);   // overlap switch or stream changed
@@ -1033,7 +1026,7 @@ extern "C" int cfdx_batch_step(cfdx_batch *q, int nsteps, int use_graph)
         // the second stream joins the capture through the fork event and is joined back before
         // each update, so the graph holds the overlap too
         for (int j = 0; j < 3; ++j)
-            cfdx::blk::stage(q->L, q->precision, j, st, q->any_visc, nullptr, overlap_if(q->ctx, q->precision, ov, true));
+            cfdx::blk::stage(q->L, q->precision, j, st, q->any_visc, nullptr, overlap_of(q->ctx, ov));
         hipError_t e = hipStreamEndCapture(st, &q->graph);
         if (e != hipSuccess) { q->graph = nullptr; return cfdx::hip_fail(e, "hipStreamEndCapture"); }
         e = hipGraphInstantiate(&q->exec, q->graph, nullptr, nullptr, 0);

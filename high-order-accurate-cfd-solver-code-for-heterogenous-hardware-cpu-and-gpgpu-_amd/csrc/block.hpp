@@ -103,13 +103,12 @@ struct LaunchList {
 // kernels (block_kernels.hip)
 // ev (optional): 6 events recorded before the viscous kernel, after it, after each face sweep
 // and after the update
-// ov (optional, ignored when timing with ev): the viscous node kernel runs on ov->aux, forked
-// from st before the face sweeps and joined back before the update, with at most ov->visc_grid
-// workgroups, so that it shares the CUs with the (VALU-bound) face sweeps
+// ov (optional, ignored when timing with ev): the viscous node kernel and the face sweeps run together:
+// in one launch with the default tile shapes and grid, else the viscous kernel on ov->aux, forked from
+// st before the sweeps and joined back before the update
 struct Overlap {
     hipStream_t aux;
     hipEvent_t fork, join;
-    uint32_t visc_grid;
 };
 void stage(const LaunchList &L, int precision, int mode, hipStream_t st, bool any_visc, hipEvent_t *ev,
            const Overlap *ov = nullptr);

@@ -191,6 +191,20 @@ __device__ __forceinline__ void node_tile(const BlockDev &B, uint32_t lt, int TX
     j0 = (int)((sidx * S + q / ntx) * TY);
 }
 
+// Runs f on the tiles of a launch: one workgroup per tile, or (LOOP) a smaller grid striding over all
+// of them. The loop is a form of its own because the compiler moves everything a tile does not change
+// (constants, index arithmetic) before it and then holds it throughout: the mixed i sweep takes 96
+// registers with the loop.
+template <bool LOOP, typename F>
+__device__ __forceinline__ void each_tile(uint32_t all, const F &f)
+{
+    if constexpr (LOOP) {
+        for (uint32_t wg = blockIdx.x; wg < all; wg += gridDim.x) f(wg);
+    } else {
+        f(blockIdx.x);
+    }
+}
+
 // block of a global tile id: the largest b with prefix[b] <= t (prefix[0] = 0, prefix[nblk] = total)
 __device__ __forceinline__ uint32_t find_block(const uint32_t *__restrict__ prefix, uint32_t nblk, uint32_t t)
 {
@@ -223,58 +237,82 @@ __device__ __forceinline__ void visc_node(const BlockDev &B, int i, int j, int k
     double U[5];
 #pragma unroll
     for (int c = 0; c < 5; ++c) U[c] = PT ? tile(c, 0, 0) : ld(Uin[c], g);
-    double dU[5][3], KS[3];
     const double iU0 = pinv_(U[0]);
+    // the differences are taken in double; the flux arithmetic runs in S
+    S Uv[5];
 #pragma unroll
-    for (int d = 0; d < 3; ++d) {
-        const uint32_t m2 = shifted(B, i, j, k, d, -2), m1 = shifted(B, i, j, k, d, -1);
-        const uint32_t p1 = shifted(B, i, j, k, d, 1), p2 = shifted(B, i, j, k, d, 2);
-        double um1[5], up1[5];
-        if (LOC && near_side(B, i, j, k, d)) {
+    for (int c = 0; c < 5; ++c) Uv[c] = S(U[c]);
+    const NodeRatios<S> nr = node_ratios(Uv);
+    S m[9], G[4][3] = {}, sk[3];
+    // adds direction d from the neighbours at d -+ 1 (a, b) and the differences dU; gives the magnitude of
+    // the MTS scale-similarity term of momentum component d + 1 along d (Viscous.cl:493-495)
+    auto add = [&](int d, double Ud, const S(&dU)[5], double a0, double b0, double ad, double bd, S mx, S my, S mz) -> S {
+        const double x = (Ud * iU0) - ((0.25 * ad + 0.5 * Ud + 0.25 * bd) * pinv_(0.25 * a0 + 0.5 * U[0] + 0.25 * b0));
+        S r = S(fabs_(x));
+        pin_(r);   // or the whole term would sink, with its operands alive, to its use after the loop
+        add_gradient(dU, nr, mx, my, mz, G);
+#pragma unroll
+        for (int c = 0; c < 4; ++c)
+#pragma unroll
+            for (int e = 0; e < 3; ++e) pin_(G[c][e]);
+        return r;
+    };
+    if constexpr (LOC) {
+#pragma unroll
+        for (int d = 0; d < 3; ++d) {
+            const uint32_t m2 = shifted(B, i, j, k, d, -2), m1 = shifted(B, i, j, k, d, -1);
+            const uint32_t p1 = shifted(B, i, j, k, d, 1), p2 = shifted(B, i, j, k, d, 2);
+            const bool near = near_side(B, i, j, k, d);
             // bounded block: the loc-selected one-sided forms of Viscous.cl:285-435 near the sides
-            const uint32_t m3 = shifted(B, i, j, k, d, -3), p3 = shifted(B, i, j, k, d, 3);
+            const uint32_t m3 = near ? shifted(B, i, j, k, d, -3) : g, p3 = near ? shifted(B, i, j, k, d, 3) : g;
             const int LI = ld(B.code, g), LM2 = ld(B.code, m2), LM1 = ld(B.code, m1), LP1 = ld(B.code, p1),
                       LP2 = ld(B.code, p2);
+            S dU[5];
 #pragma unroll
             for (int c = 0; c < 5; ++c) {
                 const double *u = Uin[c];
-                um1[c] = ld(u, m1);
-                up1[c] = ld(u, p1);
-                const double f[7] = {ld(u, m3), ld(u, m2), um1[c], U[c], up1[c], ld(u, p2), ld(u, p3)};
-                dU[c][d] = loc_derivative(f, LI, LM2, LM1, LP1, LP2, false);
+                const double a = ld(u, m1), b = ld(u, p1), a2 = ld(u, m2), b2 = ld(u, p2);
+                if (near) {
+                    const double f[7] = {ld(u, m3), a2, a, U[c], b, b2, ld(u, p3)};
+                    dU[c] = S(loc_derivative(f, LI, LM2, LM1, LP1, LP2, false));
+                } else {
+                    dU[c] = S((1.0 / 12.0) * (8.0 * (b - a) - (b2 - a2)));
+                }
+                pin_(dU[c]);
             }
-        } else if (PT && d < 2) {
-#pragma unroll
-            for (int c = 0; c < 5; ++c) {
-                um1[c] = tile(c, d, -1);
-                up1[c] = tile(c, d, 1);
-                dU[c][d] = (1.0 / 12.0) * (8.0 * (up1[c] - um1[c]) - (tile(c, d, 2) - tile(c, d, -2)));
-            }
-        } else {
-#pragma unroll
-            for (int c = 0; c < 5; ++c) {
-                const double *u = Uin[c];
-                um1[c] = ld(u, m1);
-                up1[c] = ld(u, p1);
-                dU[c][d] = (1.0 / 12.0) * (8.0 * (up1[c] - um1[c]) - (ld(u, p2) - ld(u, m2)));
-            }
+            sk[d] = add(d, U[1 + d], dU, ld(Uin[0], m1), ld(Uin[0], p1), ld(Uin[1 + d], m1), ld(Uin[1 + d], p1),
+                        ld(geo<S>(B, 1 + 3 * d), g), ld(geo<S>(B, 2 + 3 * d), g), ld(geo<S>(B, 3 + 3 * d), g));
         }
-        // MTS scale-similarity term of momentum component d+1 along d (Viscous.cl:493-495)
-        const double a = (U[1 + d] * iU0) - ((0.25 * um1[1 + d] + 0.5 * U[1 + d] + 0.25 * up1[1 + d]) * pinv_(0.25 * um1[0] + 0.5 * U[0] + 0.25 * up1[0]));
-        KS[d] = a * a;
+        uint32_t g2 = g;
+        pin_(g2);   // the metrics again, not held through the gradients
+#pragma unroll
+        for (int c = 0; c < 9; ++c) m[c] = ld(geo<S>(B, 1 + c), g2);
+    } else {
+#pragma unroll
+        for (int q = 0; q < 3; ++q) {
+            const int d = 2 - q;   // k first: its neighbours come from global memory
+            const uint32_t m2 = shifted(B, i, j, k, d, -2), m1 = shifted(B, i, j, k, d, -1);
+            const uint32_t p1 = shifted(B, i, j, k, d, 1), p2 = shifted(B, i, j, k, d, 2);
+            double a0, b0, ad, bd;
+            S dU[5];
+#pragma unroll
+            for (int c = 3 * d; c < 3 * d + 3; ++c) m[c] = ldx<NT>(geo<S>(B, 1 + c), g);
+#pragma unroll
+            for (int c = 0; c < 5; ++c) {
+                const double *u = Uin[c];
+                double a, b, a2, b2;
+                if (PT && d < 2) {
+                    a = tile(c, d, -1); b = tile(c, d, 1); a2 = tile(c, d, -2); b2 = tile(c, d, 2);
+                } else {
+                    a = ld(u, m1); b = ld(u, p1); a2 = ld(u, m2); b2 = ld(u, p2);
+                }
+                dU[c] = S((1.0 / 12.0) * (8.0 * (b - a) - (b2 - a2)));
+                if (c == 0) { a0 = a; b0 = b; }
+                if (c == d + 1) { ad = a; bd = b; }
+            }
+            sk[d] = add(d, U[1 + d], dU, a0, b0, ad, bd, m[3 * d], m[3 * d + 1], m[3 * d + 2]);
+        }
     }
-    // the differences above are taken in double; the flux arithmetic runs in S
-    S dUs[5][3], Uv[5], KSs[3], m[9];
-#pragma unroll
-    for (int c = 0; c < 5; ++c) {
-        Uv[c] = S(U[c]);
-#pragma unroll
-        for (int d = 0; d < 3; ++d) dUs[c][d] = S(dU[c][d]);
-    }
-#pragma unroll
-    for (int d = 0; d < 3; ++d) KSs[d] = S(KS[d]);
-#pragma unroll
-    for (int c = 0; c < 9; ++c) m[c] = ldx<NT>(geo<S>(B, 1 + c), g);
     S fv[3][5];
     // the node velocity: away from the sides, from the stage vector already in registers (U_m /
     // U_0, the primitives of P up to rounding) instead of three more loads; near the sides the
@@ -282,8 +320,7 @@ __device__ __forceinline__ void visc_node(const BlockDev &B, int i, int j, int k
     S vel[3];
 #pragma unroll
     for (int c = 0; c < 3; ++c) vel[c] = LOC ? ld((const S *)B.P[1 + c], g) : S(U[1 + c] * iU0);
-    const S mu = viscous_node(dUs, Uv, vel[0], vel[1], vel[2], m,
-                              ldx<NT>(geo<S>(B, 0), g), KSs, B.vp, fv);
+    const S mu = viscous_fluxes(G, Uv, nr, vel[0], vel[1], vel[2], m, ldx<NT>(geo<S>(B, 0), g), sk, B.vp, fv);
 #pragma unroll
     for (int d = 0; d < 3; ++d)
 #pragma unroll
@@ -291,59 +328,75 @@ __device__ __forceinline__ void visc_node(const BlockDev &B, int i, int j, int k
     if (mode >= 2) stx<NT>(B.mu, g, (double)mu);
 }
 
+// Doubles of LDS a node tile of the viscous kernel stages: tiles of at least 4 rows hold the stage
+// vector of the tile and its in-plane halo (each state loaded once per tile instead of once per node
+// that reaches it).
+template <int TX, int TY>
+constexpr int VISC_LDS = TY >= 4 ? 5 * (TY + 4) * (TX + 4) : 1;
+
+// Viscous node fluxes of the nodes of tile lt of block B; plane: VISC_LDS<TX, TY> doubles of LDS.
+template <typename S, int TX, int TY, bool BND>
+__device__ __forceinline__ void visc_tile(const BlockDev &B, uint32_t lt, int mode, double *plane)
+{
+    constexpr int PC = TX + 4, PR = TY + 4;
+    int i0, j0, k;
+    node_tile(B, lt, TX, TY, i0, j0, k);
+    const int tx = (int)(threadIdx.x % TX), ty = (int)(threadIdx.x / TX);
+    const int i = i0 + tx, j = j0 + ty;
+    if constexpr (TY >= 4) {
+        // the stage vector of the tile and its in-plane halo (2 nodes on each side, corners
+        // left out) into LDS; points past the last node a tile node reaches are skipped
+        const double *const *Uin = (mode == 0 || mode == 3) ? B.U0 : B.Us;
+        __syncthreads();   // the LDS of the previous tile fully read
+        for (int p = (int)threadIdx.x; p < PR * PC; p += TX * TY) {
+            const int r = p / PC, q = p % PC;
+            const bool hi = q >= 2 && q < TX + 2, hj = r >= 2 && r < TY + 2;
+            if (!hi && !hj) continue;
+            if (i0 + q - 2 > B.ni + 1 || j0 + r - 2 > B.nj + 1) continue;
+            const uint32_t x = node_index(B, along_shift(B, 0, i0, q - 2, B.ni), along_shift(B, 1, j0, r - 2, B.nj), k);
+#pragma unroll
+            for (int c = 0; c < 5; ++c) plane[(c * PR + r) * PC + q] = ld(Uin[c], x);
+        }
+        __syncthreads();
+    }
+    if (i >= B.ni || j >= B.nj) return;
+    if (BND && B.code && in_shell(B, i, j, k)) return;   // a shell tile's node
+    if constexpr (TY >= 4) visc_node<S, false, !BND, true>(B, i, j, k, mode, plane, tx, ty, PC, PR);
+    else visc_node<S, false, !BND>(B, i, j, k, mode);
+}
+
+// Viscous node fluxes of 256 shell nodes: shell tile s of the list (block = s / shell_tiles).
+template <typename S>
+__device__ __forceinline__ void visc_shell_tile(const BlockDev *__restrict__ blks, uint32_t s, int mode, uint32_t shell_tiles)
+{
+    const BlockDev &B = blks[s / shell_tiles];
+    const uint32_t t = (s % shell_tiles) * 256 + threadIdx.x;
+    if (!B.viscous || t >= shell_count(B)) return;
+    int i, j, k;
+    shell_node(B, t, i, j, k);
+    visc_node<S, true, false>(B, i, j, k, mode);
+}
+
 // Node tiles of the list first (tile ids through the XCD remap), then, for lists with bounded
 // blocks, nblk x shell_tiles shell tiles of TX * TY shell nodes each (block = id / shell_tiles),
 // dispatched last in plain order so that they spread over the XCDs at the end of the launch.
-// Tiles of at least 4 rows stage the in-plane stencil states of the tile in LDS (PLANE): each
-// state is loaded once per tile instead of once per node that reaches it.
-template <typename S, int TX, int TY, bool BND>
-__global__ void __launch_bounds__(TX *TY) k_visc(const BlockDev *__restrict__ blks, const uint32_t *__restrict__ prefix,
-                                                           uint32_t nblk, uint32_t total, int mode, uint32_t shell_tiles)
+template <typename S, int TX, int TY, bool BND, bool LOOP>
+__global__ void __launch_bounds__(TX *TY, ((TY >= 4 && !(LOOP && BND)) || sizeof(S) == 4 ? 4 : 3))
+    k_visc(const BlockDev *__restrict__ blks, const uint32_t *__restrict__ prefix, uint32_t nblk, uint32_t total, int mode,
+           uint32_t shell_tiles)
 {
-    constexpr bool PLANE = TY >= 4;
-    constexpr int PC = TX + 4, PR = TY + 4;
-    __shared__ double plane[PLANE ? 5 * PR * PC : 1];
+    __shared__ double plane[VISC_LDS<TX, TY>];
     const uint32_t all = total + (BND ? nblk * shell_tiles : 0u);
-    for (uint32_t wg = blockIdx.x; wg < all; wg += gridDim.x) {
+    auto tile = [&](uint32_t wg) {
         if (BND && wg >= total) {
-            const uint32_t s = wg - total;
-            const BlockDev &B = blks[s / shell_tiles];
-            const uint32_t t = (s % shell_tiles) * (TX * TY) + threadIdx.x;
-            if (!B.viscous || t >= shell_count(B)) continue;
-            int i, j, k;
-            shell_node(B, t, i, j, k);
-            visc_node<S, true, !BND>(B, i, j, k, mode);
-            continue;
+            visc_shell_tile<S>(blks, wg - total, mode, shell_tiles);
+            return;
         }
         const uint32_t t = xcd_tile(wg, total);
         const BlockDev &B = blks[find_block(prefix, nblk, t)];
-        if (!B.viscous) continue;
-        const uint32_t lt = t - B.tile0[0];
-        int i0, j0, k;
-        node_tile(B, lt, TX, TY, i0, j0, k);
-        const int tx = (int)(threadIdx.x % TX), ty = (int)(threadIdx.x / TX);
-        const int i = i0 + tx, j = j0 + ty;
-        if constexpr (PLANE) {
-            // the stage vector of the tile and its in-plane halo (2 nodes on each side, corners
-            // left out) into LDS; points past the last node a tile node reaches are skipped
-            const double *const *Uin = (mode == 0 || mode == 3) ? B.U0 : B.Us;
-            __syncthreads();   // the previous tile's plane fully read
-            for (int p = (int)threadIdx.x; p < PR * PC; p += TX * TY) {
-                const int r = p / PC, q = p % PC;
-                const bool hi = q >= 2 && q < TX + 2, hj = r >= 2 && r < TY + 2;
-                if (!hi && !hj) continue;
-                if (i0 + q - 2 > B.ni + 1 || j0 + r - 2 > B.nj + 1) continue;
-                const uint32_t x = node_index(B, along_shift(B, 0, i0, q - 2, B.ni), along_shift(B, 1, j0, r - 2, B.nj), k);
-#pragma unroll
-                for (int c = 0; c < 5; ++c) plane[(c * PR + r) * PC + q] = ld(Uin[c], x);
-            }
-            __syncthreads();
-        }
-        if (i >= B.ni || j >= B.nj) continue;
-        if (BND && B.code && in_shell(B, i, j, k)) continue;   // a shell tile's node
-        if constexpr (PLANE) visc_node<S, false, !BND, true>(B, i, j, k, mode, plane, tx, ty, PC, PR);
-        else visc_node<S, false, !BND>(B, i, j, k, mode);
-    }
+        if (B.viscous) visc_tile<S, TX, TY, BND>(B, t - B.tile0[0], mode, plane);
+    };
+    each_tile<LOOP>(all, tile);
 }
 
 // ---------------------------------------------------------------------------
@@ -367,123 +420,175 @@ __device__ __forceinline__ uint32_t tile_node(const BlockDev &B, int along, int 
     return node_index(B, across, fixed, along);
 }
 
-// Waves per SIMD the face kernel is compiled for: 4 (at most 128 VGPRs) for the tiles whose FP64
-// form fits them without spilling (every i tile, the (32, 8) tile along j and k), else 3. A
-// kernel that spills needs scratch memory, and its launches ran up to 40 % slower in a sequence of
-// sweeps than at 3 waves without.
-template <int DIR, int TA, int TB>
-constexpr int FACE_WAVES = (DIR == 0 || (TA == 32 && TB == 8)) ? 4 : 3;
+// Mixed form: the Roe state's inputs (rho, u, v, w, h) of the stencil points are staged too, so
+// phase 2 reads the two centre nodes from LDS; FP64 derives them from the conserved states of
+// the two centre nodes, which phase 2 holds in registers anyway (no primitive loads; staging
+// them in FP64 would cost a wave per SIMD).
+template <typename S>
+constexpr bool STAGE_ROE = std::is_same<S, float>::value;
 
+// Values of LDS a face tile stages: Q, the node flux and (mixed form) the Roe inputs of its points.
+template <typename S, int TA, int TB>
+constexpr int FACE_LDS = (STAGE_ROE<S> ? 15 : 10) * (TB + 5) * TA;
+
+// The faces of tile lt of block B along DIR; sq: FACE_LDS<S, TA, TB> values of LDS.
 template <typename S, int DIR, int TA, int TB>
-__global__ void __launch_bounds__(256, (FACE_WAVES<DIR, TA, TB>)) k_face(const BlockDev *__restrict__ blks, const uint32_t *__restrict__ prefix,
-                                              uint32_t nblk, uint32_t total)
+__device__ __forceinline__ void face_tile(const BlockDev &B, uint32_t lt, S *sq)
 {
     static_assert(TA * TB == 256, "face tiles have 256 threads");
     constexpr int NP = TB + 5;
-    // mixed form: the Roe state's inputs (rho, u, v, w, h) of the stencil points are staged too, so
-    // phase 2 reads the two centre nodes from LDS; FP64 derives them from the conserved states of
-    // the two centre nodes, which phase 2 holds in registers anyway (no primitive loads; staging
-    // them in FP64 would cost a wave per SIMD).
-    constexpr bool STAGE_ROE = std::is_same<S, float>::value;
-    __shared__ S sq[5 * NP * TA];
-    __shared__ S sf[5 * NP * TA];
-    __shared__ S sp[STAGE_ROE ? 5 * NP * TA : 1];
+    S *const sf = sq + 5 * NP * TA;
+    S *const sp = sq + 10 * NP * TA;   // STAGE_ROE only
     const int tid = threadIdx.x;
-    for (uint32_t wg = blockIdx.x; wg < total; wg += gridDim.x) {
+            const int n_along = DIR == 0 ? B.ni : DIR == 1 ? B.nj : B.nk;
+            const int n_across = DIR == 0 ? B.nj : B.ni;
+            // face f of a line is the +1/2 face of along-coordinate f - sh (sh = 1 in a bounded
+            // direction: the first face lies between the first owned node and its ghost)
+            const int nfa = faces_along(B, DIR), sh = B.off[DIR] ? 1 : 0;
+            const uint32_t nta = (n_across + TA - 1) / TA, ntb = (nfa + TB - 1) / TB;
+            // tiles run along the lines' direction before the fixed coordinate, so that the next tile of
+            // an XCD re-reads the stencil halo planes of this one from its L2
+            int b0, a0, fixed;
+    if (DIR == 0) { b0 = (lt % ntb) * TB; a0 = ((lt / ntb) % nta) * TA; fixed = lt / (ntb * nta); }
+    else { a0 = (lt % nta) * TA; b0 = ((lt / nta) % ntb) * TB; fixed = lt / (nta * ntb); }
+    const S *P0 = (const S *)B.P[0], *P1 = (const S *)B.P[1], *P2 = (const S *)B.P[2], *P3 = (const S *)B.P[3], *P4 = (const S *)B.P[4];
+
+            __syncthreads();   // the previous tile's LDS fully consumed
+            for (int p = tid; p < NP * TA; p += 256) {
+                const int s = DIR == 0 ? p % NP : p / TA;
+                const int a = DIR == 0 ? p / NP : p % TA;
+                if (a0 + a >= n_across) continue;
+                // the points past the stencil of the tile's last computed face feed no face: skip them
+                // (a bounded line ends 3 ghost nodes past its last owned node; a periodic line shorter
+                // than the tile would wrap more than once)
+                if (s > nfa - b0 + 4) continue;
+                const int along = along_shift(B, DIR, b0 - sh, s - 2, n_along);
+                const uint32_t x = tile_node<DIR>(B, along, a0 + a, fixed);
+                const S rho = ld(P0, x), u = ld(P1, x), v = ld(P2, x), w = ld(P3, x), pr = ld(P4, x);
+                S q[5], f[5];
+                prim_to_q(rho, u, v, w, pr, q);
+                node_flux_e(rho, u, v, w, pr, q[4] + pr, ld(geo<S>(B, 1 + 3 * DIR), x), ld(geo<S>(B, 2 + 3 * DIR), x),
+                            ld(geo<S>(B, 3 + 3 * DIR), x), ld(geo<S>(B, 0), x), f);
+    #pragma unroll
+                for (int c = 0; c < 5; ++c) {
+                    sq[lds_at<DIR, TA, TB>(c, s, a)] = q[c];
+                    sf[lds_at<DIR, TA, TB>(c, s, a)] = f[c];
+                }
+                if constexpr (STAGE_ROE<S>) {
+                    sp[lds_at<DIR, TA, TB>(0, s, a)] = rho; sp[lds_at<DIR, TA, TB>(1, s, a)] = u;
+                    sp[lds_at<DIR, TA, TB>(2, s, a)] = v; sp[lds_at<DIR, TA, TB>(3, s, a)] = w;
+                    sp[lds_at<DIR, TA, TB>(4, s, a)] = enthalpy(rho, u, v, w, pr);
+                }
+            }
+            __syncthreads();
+
+            const int b = DIR == 0 ? tid % TB : tid / TA;
+            const int a = DIR == 0 ? tid / TB : tid % TA;
+            if (b0 + b < nfa && a0 + a < n_across) {
+                auto q = [&](int m, int c) { return sq[lds_at<DIR, TA, TB>(c, b + m, a)]; };
+        const uint32_t gl = tile_node<DIR>(B, b0 + b - sh, a0 + a, fixed);
+        S roe[5], irho;
+        if constexpr (STAGE_ROE<S>) {
+            // the face's two centre nodes are stencil points 2 and 3
+            auto at = [&](int c, int m) { return sp[lds_at<DIR, TA, TB>(c, b + m, a)]; };
+            irho = roe_average(at(0, 2), at(1, 2), at(2, 2), at(3, 2), at(4, 2), at(0, 3), at(1, 3), at(2, 3), at(3, 3), at(4, 3), roe);
+        } else {
+            // from the conserved states of the two centre nodes
+            S qa[5], qb[5], ia, ib, ua, va, wa, ha, ub, vb, wb, hb;
+#pragma unroll
+            for (int c = 0; c < 5; ++c) { qa[c] = q(2, c); qb[c] = q(3, c); }
+            pinv2_(qa[0], qb[0], ia, ib);
+            q_roe_inputs(qa, ia, ua, va, wa, ha);
+            q_roe_inputs(qb, ib, ub, vb, wb, hb);
+            irho = roe_average(qa[0], ua, va, wa, ha, qb[0], ub, vb, wb, hb, roe);
+        }
+        // unit face normal and det_f |k| (the stored face arrays after geometry_finalize);
+                // streaming accesses on periodic blocks (B.code null)
+                S fg[4];
+                if (B.code) {
+    #pragma unroll
+                    for (int c = 0; c < 3; ++c) fg[c] = ld(geo<S>(B, 10 + 3 * DIR + c), gl);
+                    fg[3] = ld(geo<S>(B, 19 + DIR), gl);
+                } else {
+    #pragma unroll
+                    for (int c = 0; c < 3; ++c) fg[c] = ldx<true>(geo<S>(B, 10 + 3 * DIR + c), gl);
+                    fg[3] = ldx<true>(geo<S>(B, 19 + DIR), gl);
+                }
+                S llf[5];
+                face_llf(q, roe, irho, fg[0], fg[1], fg[2], fg[3], S(B.eps), llf);
+                S fh[5];
+    #pragma unroll
+                for (int c = 0; c < 5; ++c)
+                    fh[c] = S(llf[c] + midpoint_correction(sf[lds_at<DIR, TA, TB>(c, b, a)], sf[lds_at<DIR, TA, TB>(c, b + 1, a)],
+                                                           sf[lds_at<DIR, TA, TB>(c, b + 2, a)], sf[lds_at<DIR, TA, TB>(c, b + 3, a)],
+                                                           sf[lds_at<DIR, TA, TB>(c, b + 4, a)], sf[lds_at<DIR, TA, TB>(c, b + 5, a)]));
+                if (B.code) {
+    #pragma unroll
+                    for (int c = 0; c < 5; ++c) st((S *)B.FH[DIR][c], gl, fh[c]);
+                } else {
+    #pragma unroll
+                    for (int c = 0; c < 5; ++c) stx<true>((S *)B.FH[DIR][c], gl, fh[c]);
+                }
+            }
+}
+
+template <typename S, int DIR, int TA, int TB, bool LOOP>
+__global__ void __launch_bounds__(256, 4) k_face(const BlockDev *__restrict__ blks, const uint32_t *__restrict__ prefix,
+                                              uint32_t nblk, uint32_t total)
+{
+    __shared__ S lds[FACE_LDS<S, TA, TB>];
+    auto tile = [&](uint32_t wg) {
         const uint32_t t = xcd_tile(wg, total);
         const BlockDev &B = blks[find_block(prefix, nblk, t)];
-        const uint32_t lt = t - B.tile0[1 + DIR];
-        const int n_along = DIR == 0 ? B.ni : DIR == 1 ? B.nj : B.nk;
-        const int n_across = DIR == 0 ? B.nj : B.ni;
-        // face f of a line is the +1/2 face of along-coordinate f - sh (sh = 1 in a bounded
-        // direction: the first face lies between the first owned node and its ghost)
-        const int nfa = faces_along(B, DIR), sh = B.off[DIR] ? 1 : 0;
-        const uint32_t nta = (n_across + TA - 1) / TA, ntb = (nfa + TB - 1) / TB;
-        // tiles run along the lines' direction before the fixed coordinate, so that the next tile of
-        // an XCD re-reads the stencil halo planes of this one from its L2
-        int b0, a0, fixed;
-        if (DIR == 0) { b0 = (lt % ntb) * TB; a0 = ((lt / ntb) % nta) * TA; fixed = lt / (ntb * nta); }
-        else { a0 = (lt % nta) * TA; b0 = ((lt / nta) % ntb) * TB; fixed = lt / (nta * ntb); }
-        const S *P0 = (const S *)B.P[0], *P1 = (const S *)B.P[1], *P2 = (const S *)B.P[2], *P3 = (const S *)B.P[3], *P4 = (const S *)B.P[4];
+        face_tile<S, DIR, TA, TB>(B, t - B.tile0[1 + DIR], lds);
+    };
+    each_tile<LOOP>(total, tile);
+}
 
-        __syncthreads();   // the previous tile's LDS fully consumed
-        for (int p = tid; p < NP * TA; p += 256) {
-            const int s = DIR == 0 ? p % NP : p / TA;
-            const int a = DIR == 0 ? p / NP : p % TA;
-            if (a0 + a >= n_across) continue;
-            // the points past the stencil of the tile's last computed face feed no face: skip them
-            // (a bounded line ends 3 ghost nodes past its last owned node; a periodic line shorter
-            // than the tile would wrap more than once)
-            if (s > nfa - b0 + 4) continue;
-            const int along = along_shift(B, DIR, b0 - sh, s - 2, n_along);
-            const uint32_t x = tile_node<DIR>(B, along, a0 + a, fixed);
-            const S rho = ld(P0, x), u = ld(P1, x), v = ld(P2, x), w = ld(P3, x), pr = ld(P4, x);
-            S q[5], f[5];
-            prim_to_q(rho, u, v, w, pr, q);
-            node_flux_e(rho, u, v, w, pr, q[4] + pr, ld(geo<S>(B, 1 + 3 * DIR), x), ld(geo<S>(B, 2 + 3 * DIR), x),
-                        ld(geo<S>(B, 3 + 3 * DIR), x), ld(geo<S>(B, 0), x), f);
-#pragma unroll
-            for (int c = 0; c < 5; ++c) {
-                sq[lds_at<DIR, TA, TB>(c, s, a)] = q[c];
-                sf[lds_at<DIR, TA, TB>(c, s, a)] = f[c];
-            }
-            if constexpr (STAGE_ROE) {
-                sp[lds_at<DIR, TA, TB>(0, s, a)] = rho; sp[lds_at<DIR, TA, TB>(1, s, a)] = u;
-                sp[lds_at<DIR, TA, TB>(2, s, a)] = v; sp[lds_at<DIR, TA, TB>(3, s, a)] = w;
-                sp[lds_at<DIR, TA, TB>(4, s, a)] = enthalpy(rho, u, v, w, pr);
-            }
-        }
-        __syncthreads();
+// The viscous node tiles and the three face sweeps of a stage in one launch (tile variants 0). They
+// depend on nothing of each other, and apart each launch ends with a tail and a gap: at 64^3 the
+// five launches of a stage take 87 us (FP64) and 59 us (mixed), the two that are left 71 and 42 us;
+// at 128^3 511 us against 546 apart (FP64) and 294 against 325 (mixed), at 256^3 4.19 ms against 4.26 and
+// 2.40 against 2.43. Each XCD takes its own contiguous share of every kind of tile and runs through them
+// FLUX_CHUNK tiles of a kind at a time: with the kinds alternating tile by tile they fall into step
+// with the CUs (each CU draws tiles of one kind; 256^3 8 % slower in FP64, 23 % mixed), 4 and 16 are
+// best, a kind's whole share at a time 1 % slower at 256^3 FP64 and 3 % at 128^3 mixed.
+constexpr uint32_t FLUX_CHUNK = 16;
+struct FluxTotals {
+    const uint32_t *prefix[4];
+    uint32_t total[4];   // tiles of the node kernel and of the i, j, k sweeps
+    uint32_t chunk;      // tiles of a kind that an XCD takes at a time
+};
 
-        const int b = DIR == 0 ? tid % TB : tid / TA;
-        const int a = DIR == 0 ? tid / TB : tid % TA;
-        if (b0 + b < nfa && a0 + a < n_across) {
-            S q[6][5];
-#pragma unroll
-            for (int m = 0; m < 6; ++m)
-#pragma unroll
-                for (int c = 0; c < 5; ++c) q[m][c] = sq[lds_at<DIR, TA, TB>(c, b + m, a)];
-            const uint32_t gl = tile_node<DIR>(B, b0 + b - sh, a0 + a, fixed);
-            S roe[5];
-            if constexpr (STAGE_ROE) {
-                // the face's two centre nodes are stencil points 2 and 3
-                auto at = [&](int c, int m) { return sp[lds_at<DIR, TA, TB>(c, b + m, a)]; };
-                roe_average(at(0, 2), at(1, 2), at(2, 2), at(3, 2), at(4, 2), at(0, 3), at(1, 3), at(2, 3), at(3, 3), at(4, 3), roe);
-            } else {
-                // from the conserved states of the two centre nodes, already in registers
-                S ra, ua, va, wa, ha, rb, ub, vb, wb, hb;
-                q_roe_inputs(q[2], ra, ua, va, wa, ha);
-                q_roe_inputs(q[3], rb, ub, vb, wb, hb);
-                roe_average(ra, ua, va, wa, ha, rb, ub, vb, wb, hb, roe);
-            }
-            // unit face normal and det_f |k| (the stored face arrays after geometry_finalize);
-            // streaming accesses on periodic blocks (B.code null)
-            S fg[4];
-            if (B.code) {
-#pragma unroll
-                for (int c = 0; c < 3; ++c) fg[c] = ld(geo<S>(B, 10 + 3 * DIR + c), gl);
-                fg[3] = ld(geo<S>(B, 19 + DIR), gl);
-            } else {
-#pragma unroll
-                for (int c = 0; c < 3; ++c) fg[c] = ldx<true>(geo<S>(B, 10 + 3 * DIR + c), gl);
-                fg[3] = ldx<true>(geo<S>(B, 19 + DIR), gl);
-            }
-            S llf[5];
-            face_llf(q, roe, fg[0], fg[1], fg[2], fg[3], S(B.eps), llf);
-            S fh[5];
-#pragma unroll
-            for (int c = 0; c < 5; ++c)
-                fh[c] = S(llf[c] + midpoint_correction(sf[lds_at<DIR, TA, TB>(c, b, a)], sf[lds_at<DIR, TA, TB>(c, b + 1, a)],
-                                                       sf[lds_at<DIR, TA, TB>(c, b + 2, a)], sf[lds_at<DIR, TA, TB>(c, b + 3, a)],
-                                                       sf[lds_at<DIR, TA, TB>(c, b + 4, a)], sf[lds_at<DIR, TA, TB>(c, b + 5, a)]));
-            if (B.code) {
-#pragma unroll
-                for (int c = 0; c < 5; ++c) st((S *)B.FH[DIR][c], gl, fh[c]);
-            } else {
-#pragma unroll
-                for (int c = 0; c < 5; ++c) stx<true>((S *)B.FH[DIR][c], gl, fh[c]);
-            }
-        }
+template <typename S, bool VISC, bool BND>
+__global__ void __launch_bounds__(256, 4) k_flux(const BlockDev *__restrict__ blks, FluxTotals T, uint32_t nblk, uint32_t slots,
+                                                 int mode, uint32_t shell_tiles)
+{
+    constexpr int IA = FACE_I_TILES[0][0], IB = FACE_I_TILES[0][1], JA = FACE_JK_TILES[0][0], JB = FACE_JK_TILES[0][1];
+    constexpr int TX = NODE_TILES[0][0], TY = NODE_TILES[0][1];
+    constexpr int L0 = VISC ? VISC_LDS<TX, TY> * (int)sizeof(double) : 0, L1 = FACE_LDS<S, IA, IB> * (int)sizeof(S),
+                  L2 = FACE_LDS<S, JA, JB> * (int)sizeof(S);
+    __shared__ __align__(16) char lds[L0 > L1 ? (L0 > L2 ? L0 : L2) : (L1 > L2 ? L1 : L2)];
+    constexpr uint32_t K = VISC ? 4 : 3;
+    const uint32_t main = 8 * K * slots, wg = blockIdx.x;
+    if (VISC && BND && wg >= main) {
+        visc_shell_tile<S>(blks, wg - main, mode, shell_tiles);
+        return;
+    }
+    const uint32_t x = wg & 7u, l = wg >> 3, kind = (l % (K * T.chunk)) / T.chunk + (4 - K), r = (l / (K * T.chunk)) * T.chunk + l % T.chunk;
+    const uint32_t total = T.total[kind], q = total >> 3, rem = total & 7u;
+    if (r >= q + (x < rem ? 1u : 0u)) return;
+    const uint32_t t = x * q + (x < rem ? x : rem) + r;
+    const BlockDev &B = blks[find_block(T.prefix[kind], nblk, t)];
+    const uint32_t lt = t - B.tile0[kind];
+    if (kind == 0) {
+        if (B.viscous) visc_tile<S, TX, TY, BND>(B, lt, mode, (double *)lds);
+    } else if (kind == 1) {
+        face_tile<S, 0, IA, IB>(B, lt, (S *)lds);
+    } else if (kind == 2) {
+        face_tile<S, 1, JA, JB>(B, lt, (S *)lds);
+    } else {
+        face_tile<S, 2, JA, JB>(B, lt, (S *)lds);
     }
 }
 
@@ -594,12 +699,12 @@ __device__ __forceinline__ void monitor_wave(const BlockDev &B, uint32_t slot, d
 
 // tiles as in k_visc; the shell tiles' monitor slots follow the block's node tiles' (tiles x
 // waves per tile), one per wave of 64 shell nodes
-template <typename S, int TX, int TY, bool BND>
+template <typename S, int TX, int TY, bool BND, bool LOOP>
 __global__ void __launch_bounds__(TX *TY) k_update(const BlockDev *__restrict__ blks, const uint32_t *__restrict__ prefix,
                                                    uint32_t nblk, uint32_t total, int mode, uint32_t shell_tiles)
 {
     const uint32_t all = total + (BND ? nblk * shell_tiles : 0u);
-    for (uint32_t wg = blockIdx.x; wg < all; wg += gridDim.x) {
+    auto tile = [&](uint32_t wg) {
         // residual monitor of the step (Solver.cpp:546-573): |du|, |dv|, |de| against the RK base
         double mdu = 0.0, mdv = 0.0, mde = 0.0;
         if (BND && wg >= total) {
@@ -607,7 +712,7 @@ __global__ void __launch_bounds__(TX *TY) k_update(const BlockDev *__restrict__ 
             const BlockDev &B = blks[s / shell_tiles];
             const uint32_t t = (s % shell_tiles) * (TX * TY) + threadIdx.x;
             const uint32_t ns = shell_count(B);
-            if ((s % shell_tiles) * (TX * TY) >= ns) continue;   // whole tile past the shell
+            if ((s % shell_tiles) * (TX * TY) >= ns) return;   // whole tile past the shell
             if (t < ns) {
                 int i, j, k;
                 shell_node(B, t, i, j, k);
@@ -617,7 +722,7 @@ __global__ void __launch_bounds__(TX *TY) k_update(const BlockDev *__restrict__ 
                 const uint32_t main_slots = ((B.ni + TX - 1) / TX) * ((B.nj + TY - 1) / TY) * B.nk * (uint32_t)(TX * TY / 64);
                 monitor_wave(B, main_slots + t / 64, mdu, mdv, mde);
             }
-            continue;
+            return;
         }
         const uint32_t t = xcd_tile(wg, total);
         const BlockDev &B = blks[find_block(prefix, nblk, t)];
@@ -628,7 +733,8 @@ __global__ void __launch_bounds__(TX *TY) k_update(const BlockDev *__restrict__ 
         if (i < B.ni && j < B.nj && !(BND && B.code && in_shell(B, i, j, k)))
             update_node<S, false, !BND>(B, i, j, k, mode, mdu, mdv, mde);
         if (mode == 2 && B.mon) monitor_wave(B, lt * (TX * TY / 64) + threadIdx.x / 64, mdu, mdv, mde);
-    }
+    };
+    each_tile<LOOP>(all, tile);
 }
 
 // maxima over the per-wave monitor values: out[0..2] = max |du|, |dv|, |de|
@@ -855,99 +961,131 @@ void launch_bc(const LaunchList &L, int mode, hipStream_t st)
 // ---------------------------------------------------------------------------
 // host launchers
 // ---------------------------------------------------------------------------
-template <typename S, int V>
-void launch_face_i(const LaunchList &L, dim3 g, hipStream_t st)
+template <typename S, int DIR, int TA, int TB>
+void launch_face(const LaunchList &L, hipStream_t st)
 {
-    hipLaunchKernelGGL((k_face<S, 0, FACE_I_TILES[V][0], FACE_I_TILES[V][1]>), g, dim3(256), 0, st, L.blks, L.prefix[1],
-                       L.nblk, L.total[1]);
+    const uint32_t n = L.total[1 + DIR];
+    if (L.grid_cap && L.grid_cap < n)
+        hipLaunchKernelGGL((k_face<S, DIR, TA, TB, true>), dim3(L.grid_cap), dim3(256), 0, st, L.blks, L.prefix[1 + DIR], L.nblk, n);
+    else
+        hipLaunchKernelGGL((k_face<S, DIR, TA, TB, false>), dim3(n), dim3(256), 0, st, L.blks, L.prefix[1 + DIR], L.nblk, n);
 }
-template <typename S, int DIR, int V>
-void launch_face_jk(const LaunchList &L, dim3 g, hipStream_t st)
-{
-    hipLaunchKernelGGL((k_face<S, DIR, FACE_JK_TILES[V][0], FACE_JK_TILES[V][1]>), g, dim3(256), 0, st, L.blks,
-                       L.prefix[1 + DIR], L.nblk, L.total[1 + DIR]);
-}
+// cap: workgroups of the launch (0: one per tile)
 template <typename S, int V, bool BND>
-void launch_node_b(const LaunchList &L, dim3 g, hipStream_t st, bool visc_kernel, int mode)
+void launch_node_b(const LaunchList &L, uint32_t cap, hipStream_t st, bool visc_kernel, int mode)
 {
     constexpr int TX = NODE_TILES[V][0], TY = NODE_TILES[V][1];
     static_assert(TX * TY == 256, "node tiles have 256 threads");
     const uint32_t shell_tiles = BND ? (L.shell_max + TX * TY - 1) / (TX * TY) : 0u;
-    dim3 ga = g;
-    if (BND && !L.grid_cap) ga.x += L.nblk * shell_tiles;   // one workgroup per shell tile too
-    if (visc_kernel)
-        hipLaunchKernelGGL((k_visc<S, TX, TY, BND>), ga, dim3(TX * TY), 0, st, L.blks, L.prefix[0], L.nblk, L.total[0], mode,
+    const uint32_t all = L.total[0] + L.nblk * shell_tiles;   // one workgroup per shell tile too
+    const bool loop = cap && cap < all;
+    auto go = [&](auto kernel) {
+        hipLaunchKernelGGL(kernel, dim3(loop ? cap : all), dim3(TX * TY), 0, st, L.blks, L.prefix[0], L.nblk, L.total[0], mode,
                            shell_tiles);
-    else
-        hipLaunchKernelGGL((k_update<S, TX, TY, BND>), ga, dim3(TX * TY), 0, st, L.blks, L.prefix[0], L.nblk, L.total[0], mode,
-                           shell_tiles);
+    };
+    if (visc_kernel && loop) go(k_visc<S, TX, TY, BND, true>);
+    else if (visc_kernel) go(k_visc<S, TX, TY, BND, false>);
+    else if (loop) go(k_update<S, TX, TY, BND, true>);
+    else go(k_update<S, TX, TY, BND, false>);
 }
 // lists without bounded blocks run the node kernels without the loc-code branches
 template <typename S, int V>
-void launch_node(const LaunchList &L, dim3 g, hipStream_t st, bool visc_kernel, int mode)
+void launch_node(const LaunchList &L, uint32_t cap, hipStream_t st, bool visc_kernel, int mode)
 {
-    if (L.bc_face) launch_node_b<S, V, true>(L, g, st, visc_kernel, mode);
-    else launch_node_b<S, V, false>(L, g, st, visc_kernel, mode);
+    if (L.bc_face) launch_node_b<S, V, true>(L, cap, st, visc_kernel, mode);
+    else launch_node_b<S, V, false>(L, cap, st, visc_kernel, mode);
 }
 
 template <typename S>
-void node_kernel(const LaunchList &L, dim3 g, hipStream_t st, bool visc_kernel, int mode)
+void node_kernel(const LaunchList &L, uint32_t cap, hipStream_t st, bool visc_kernel, int mode)
 {
     switch (L.tiles.node) {
-    case 1: launch_node<S, 1>(L, g, st, visc_kernel, mode); break;
-    case 2: launch_node<S, 2>(L, g, st, visc_kernel, mode); break;
-    case 3: launch_node<S, 3>(L, g, st, visc_kernel, mode); break;
-    default: launch_node<S, 0>(L, g, st, visc_kernel, mode);
+    case 1: launch_node<S, 1>(L, cap, st, visc_kernel, mode); break;
+    case 2: launch_node<S, 2>(L, cap, st, visc_kernel, mode); break;
+    case 3: launch_node<S, 3>(L, cap, st, visc_kernel, mode); break;
+    default: launch_node<S, 0>(L, cap, st, visc_kernel, mode);
+    }
+}
+
+template <typename S>
+void face_i(const LaunchList &L, hipStream_t st)
+{
+    constexpr auto &T = FACE_I_TILES;
+    switch (L.tiles.face[0]) {
+    case 1: launch_face<S, 0, T[1][0], T[1][1]>(L, st); break;
+    case 2: launch_face<S, 0, T[2][0], T[2][1]>(L, st); break;
+    default: launch_face<S, 0, T[0][0], T[0][1]>(L, st);
     }
 }
 
 template <typename S, int DIR>
-void face_jk(const LaunchList &L, dim3 g, hipStream_t st)
+void face_jk(const LaunchList &L, hipStream_t st)
 {
+    constexpr auto &T = FACE_JK_TILES;
     switch (L.tiles.face[DIR]) {
-    case 1: launch_face_jk<S, DIR, 1>(L, g, st); break;
-    case 2: launch_face_jk<S, DIR, 2>(L, g, st); break;
-    case 3: launch_face_jk<S, DIR, 3>(L, g, st); break;
-    default: launch_face_jk<S, DIR, 0>(L, g, st);
+    case 1: launch_face<S, DIR, T[1][0], T[1][1]>(L, st); break;
+    case 2: launch_face<S, DIR, T[2][0], T[2][1]>(L, st); break;
+    case 3: launch_face<S, DIR, T[3][0], T[3][1]>(L, st); break;
+    default: launch_face<S, DIR, T[0][0], T[0][1]>(L, st);
     }
+}
+
+template <typename S>
+void launch_flux(const LaunchList &L, int mode, hipStream_t st, bool any_visc)
+{
+    FluxTotals T;
+    uint32_t most = 0;
+    for (int q = 0; q < 4; ++q) {
+        T.prefix[q] = L.prefix[q];
+        T.total[q] = L.total[q];
+        if (q > 0 || any_visc) most = std::max(most, L.total[q]);
+    }
+    uint32_t slots = (most + 7) / 8;
+    T.chunk = std::min(FLUX_CHUNK, slots);
+    slots = (slots + T.chunk - 1) / T.chunk * T.chunk;
+    const uint32_t shell_tiles = L.bc_face && any_visc ? (L.shell_max + 255) / 256 : 0u;
+    const dim3 g(8 * (any_visc ? 4u : 3u) * slots + L.nblk * shell_tiles);
+    auto go = [&](auto kernel) {
+        hipLaunchKernelGGL(kernel, g, dim3(256), 0, st, L.blks, T, L.nblk, slots, mode, shell_tiles);
+    };
+    if (!any_visc) go(k_flux<S, false, false>);
+    else if (L.bc_face) go(k_flux<S, true, true>);
+    else go(k_flux<S, true, false>);
 }
 
 template <typename S>
 void launch_stage(const LaunchList &L, int mode, hipStream_t st, bool any_visc, hipEvent_t *ev, const Overlap *ov)
 {
     auto rec = [&](int s) { if (ev) (void)hipEventRecord(ev[s], st); };
-    auto grid = [&](uint32_t total) { return dim3(L.grid_cap ? std::min(total, L.grid_cap) : total); };
     rec(0);
     // the viscous node kernel reads the stage vector, primitives and geometry and writes Fv and mu;
-    // the face sweeps read the primitives and geometry and write F-hat: independent until the
-    // update, so the viscous kernel may run beside the sweeps on the second stream (persistent,
-    // one workgroup per CU, leaving the CUs' remaining slots to the sweeps)
-    const bool overlap = ov && !ev && any_visc;
+    // the face sweeps read the primitives and geometry and write F-hat: independent until the update
+    const TileCfg &t = L.tiles;
+    const bool overlap = ov && !ev, together = overlap && !L.grid_cap && !(t.face[0] | t.face[1] | t.face[2] | t.node);
     hipStream_t vs = st;
-    dim3 gv = grid(L.total[0]);
-    if (overlap) {
-        (void)hipEventRecord(ov->fork, st);
-        (void)hipStreamWaitEvent(ov->aux, ov->fork, 0);
-        vs = ov->aux;
-        gv.x = std::min(gv.x, ov->visc_grid);
+    if (together) {
+        launch_flux<S>(L, mode, st, any_visc);
+    } else if (any_visc) {
+        if (overlap) {
+            // other tile shapes or a capped grid: beside the sweeps on the second stream
+            (void)hipEventRecord(ov->fork, st);
+            (void)hipStreamWaitEvent(ov->aux, ov->fork, 0);
+            vs = ov->aux;
+        }
+        node_kernel<S>(L, L.grid_cap, vs, true, mode);
     }
-    if (any_visc) node_kernel<S>(L, gv, vs, true, mode);
     if (any_visc && L.any_cut)
         hipLaunchKernelGGL(k_cut_viscous<S>, dim3((3 * L.bc_face_d[1] + 255) / 256, L.nblk), dim3(256), 0, vs, L.blks);
-    if (overlap) (void)hipEventRecord(ov->join, vs);
+    if (vs != st) (void)hipEventRecord(ov->join, vs);
     rec(1);
-    switch (L.tiles.face[0]) {
-    case 1: launch_face_i<S, 1>(L, grid(L.total[1]), st); break;
-    case 2: launch_face_i<S, 2>(L, grid(L.total[1]), st); break;
-    default: launch_face_i<S, 0>(L, grid(L.total[1]), st);
-    }
+    if (!together) face_i<S>(L, st);
     rec(2);
-    face_jk<S, 1>(L, grid(L.total[2]), st);
+    if (!together) face_jk<S, 1>(L, st);
     rec(3);
-    face_jk<S, 2>(L, grid(L.total[3]), st);
+    if (!together) face_jk<S, 2>(L, st);
     rec(4);
-    if (overlap) (void)hipStreamWaitEvent(st, ov->join, 0);
-    node_kernel<S>(L, grid(L.total[0]), st, false, mode);
+    if (vs != st) (void)hipStreamWaitEvent(st, ov->join, 0);
+    node_kernel<S>(L, L.grid_cap, st, false, mode);
     if (L.bc_face && mode <= 2) launch_bc<S>(L, mode, st);
     rec(5);
 }

@@ -129,7 +129,6 @@ extern "C" int cfdx_ctx_create(int device, void *stream, cfdx_ctx **out)
         hipError_t e = hipStreamCreateWithFlags(&c->aux, hipStreamNonBlocking);
         if (e == hipSuccess) e = hipEventCreateWithFlags(&c->fork, hipEventDisableTiming);
         if (e == hipSuccess) e = hipEventCreateWithFlags(&c->join, hipEventDisableTiming);
-        if (e == hipSuccess) e = hipDeviceGetAttribute(&c->n_cu, hipDeviceAttributeMultiprocessorCount, device);
         if (e != hipSuccess) {
             cfdx::ctx_release(c);
             return cfdx::hip_fail(e, "ctx_create second stream");

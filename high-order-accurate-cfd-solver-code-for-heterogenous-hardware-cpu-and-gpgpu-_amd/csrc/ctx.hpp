@@ -14,11 +14,10 @@ struct cfdx_ctx {
     bool owns_stream = false;
     hipEvent_t ev[8] = {};
     // a second stream of the device for work of a stage that may overlap the main stream's
-    // (forked from and joined back to the main stream by the two events), and the device's CUs
+    // (forked from and joined back to the main stream by the two events)
     hipStream_t aux = nullptr;
     hipEvent_t fork = nullptr, join = nullptr;
-    int n_cu = 0;
-    bool overlap = true;   // mixed stages (and FP64 ones in graphs) overlap the viscous kernel with the face sweeps
+    bool overlap = true;   // a stage's viscous kernel and its face sweeps run together
     // bumped by every change that a captured batch graph depends on (overlap switch, stream): a batch
     // re-captures its step when the generation it captured under is not the current one
     std::atomic<uint64_t> gen{1};

@@ -58,6 +58,12 @@ template <> __device__ Cnt prsq_<Cnt>(Cnt x) { return opc::tally(g_ops.sqrt, 1.0
 template <> __device__ Cnt inv_<Cnt>(Cnt x) { return opc::tally(g_ops.rcp, 1.0 / x.v, x.var); }
 template <> __device__ Cnt pinv_<Cnt>(Cnt x) { return opc::tally(g_ops.rcp, 1.0 / x.v, x.var); }
 template <> __device__ Cnt div_<Cnt>(Cnt a, Cnt b) { return opc::tally(g_ops.div, a.v / b.v, a.var || b.var); }
+template <> __device__ Cnt psqrt_half_<Cnt>(Cnt x, Cnt &h)
+{
+    h = Cnt(0.5 / __builtin_sqrt(x.v), x.var);   // a by-product of the square root's refinement
+    return psqrt_<Cnt>(x);
+}
+template <> __device__ Cnt tiny_<Cnt>() { return Cnt(1e-280); }
 template <> __device__ Cnt prcbrt_<Cnt>(Cnt x) { return opc::tally(g_ops.cbrt, 1.0 / cbrt(x.v), x.var); }
 }  // namespace dev
 
@@ -87,14 +93,15 @@ __global__ void k_opcount(Ops *out, ViscParams vp)
             for (int c = 0; c < 5; ++c) nf[m][c] = in(0.3 * (c + 1) * s);
         }
         // the FP64 sweep takes the Roe inputs of the two centre nodes from their conserved states
-        Cnt ra, ua, va, wa, ha, rb, ub, vb, wb, hb;
-        q_roe_inputs(q[2], ra, ua, va, wa, ha);
-        q_roe_inputs(q[3], rb, ub, vb, wb, hb);
+        Cnt ia, ib, ua, va, wa, ha, ub, vb, wb, hb;
+        pinv2_(q[2][0], q[3][0], ia, ib);
+        q_roe_inputs(q[2], ia, ua, va, wa, ha);
+        q_roe_inputs(q[3], ib, ub, vb, wb, hb);
         Cnt roe[5];
-        roe_average(ra, ua, va, wa, ha, rb, ub, vb, wb, hb, roe);
+        const Cnt irho = roe_average(q[2][0], ua, va, wa, ha, q[3][0], ub, vb, wb, hb, roe);
         Cnt llf[5];
         // the unit face normal and det_f |k| as the sweeps read them
-        face_llf(q, roe, in(0.99), in(0.11), in(0.055), in(1.2), Cnt(1e-7), llf);
+        face_llf([&](int m, int c) { return q[m][c]; }, roe, irho, in(0.99), in(0.11), in(0.055), in(1.2), Cnt(1e-7), llf);
         Cnt fh[5];
         for (int c = 0; c < 5; ++c)
             fh[c] = llf[c] + midpoint_correction(nf[0][c], nf[1][c], nf[2][c], nf[3][c], nf[4][c], nf[5][c]);

@@ -68,6 +68,33 @@ template <> __device__ __forceinline__ double prsq_<double>(double x)
 }
 template <> __device__ __forceinline__ float prsq_<float>(float x) { return __builtin_amdgcn_rsqf(x); }
 
+// Keeps the computation of x where it stands in the instruction stream: the scheduler otherwise moves
+// loads up and uses down until a long kernel holds far more values than it needs (the FP64 face
+// sweep: 168 registers, 128 and no spill with the pins of characteristic_states).
+template <typename T>
+__device__ __forceinline__ void pin_(T &x)
+{
+    if constexpr (std::is_arithmetic<T>::value) asm volatile("" : "+v"(x));
+}
+
+// s = sqrt(x) and r = 1 / sqrt(x) together: in double from one hardware estimate (h of the square
+// root's step is half of r, refined once), in float the hardware square root and reciprocal
+template <typename T> __device__ __forceinline__ T psqrt_half_(T x, T &h);
+template <> __device__ __forceinline__ double psqrt_half_<double>(double x, double &h) { return gold_sqrt(x, h); }
+template <typename T>
+__device__ __forceinline__ void psqrt_rsq_(T x, T &s, T &r)
+{
+    if constexpr (std::is_same<T, float>::value) {
+        s = psqrt_(x);
+        r = pinv_(s);
+    } else {
+        T h;
+        s = psqrt_half_(x, h);
+        r = T(2) * h;
+        r = r + r * (T(1) - s * r);
+    }
+}
+
 // Conserved state Q = (rho, rho u, rho v, rho w, p/0.4 + rho |u|^2 / 2) of primitives (U_Q.cl:118-122).
 // No fused multiply-adds, so every kernel that builds the RK base det * Q from the same primitives
 // (the last RK stage, set_flow) gets the same bits: a state saved and restored continues exactly.
@@ -90,30 +117,45 @@ __device__ __forceinline__ T enthalpy(T rho, T u, T v, T w, T p)
     return (p * T(3.5) + T(0.5) * rho * (u * u + v * v + w * w)) * pinv_(rho);   // (p/0.4 + ke + p) / rho
 }
 
-// Roe-average inputs (rho, u, v, w, H) of a node from its conserved state Q: the face kernels hold
-// the Q of the stencil points already, so the two centre nodes need no primitive loads.
+// The reciprocals of two positive operands: in double by one reciprocal of their product (the
+// hardware estimate issues at a quarter of the rate of a multiplication).
 template <typename T>
-__device__ __forceinline__ void q_roe_inputs(const T (&q)[5], T &rho, T &u, T &v, T &w, T &h)
+__device__ __forceinline__ void pinv2_(T x, T y, T &ix, T &iy)
 {
-    const T r = pinv_(q[0]);
-    rho = q[0];
+    if constexpr (std::is_same<T, float>::value) {
+        ix = pinv_(x);
+        iy = pinv_(y);
+    } else {
+        const T r = pinv_(x * y);
+        ix = r * y;
+        iy = r * x;
+    }
+}
+
+// Roe-average inputs (u, v, w, H) of a node from its conserved state Q and r = 1 / Q0: the face kernels
+// hold the Q of the stencil points already, so the two centre nodes need no primitive loads.
+template <typename T>
+__device__ __forceinline__ void q_roe_inputs(const T (&q)[5], T r, T &u, T &v, T &w, T &h)
+{
     u = q[1] * r;
     v = q[2] * r;
     w = q[3] * r;
     h = (T(1.4) * q[4] - T(0.2) * (q[1] * u + q[2] * v + q[3] * w)) * r;   // (E + p) / rho, p = 0.4 (E - rho |u|^2 / 2)
 }
 
-// Roe average of the face between states a and b (U_Q.cl:60-109): (u, v, w, h, rho).
+// Roe average of the face between states a and b (U_Q.cl:60-109): (u, v, w, h, rho), and 1 / rho.
 template <typename T>
-__device__ __forceinline__ void roe_average(T ra, T ua, T va, T wa, T ha, T rb, T ub, T vb, T wb, T hb, T (&r)[5])
+__device__ __forceinline__ T roe_average(T ra, T ua, T va, T wa, T ha, T rb, T ub, T vb, T wb, T hb, T (&r)[5])
 {
     const T sa = psqrt_(ra), sb = psqrt_(rb);
-    const T is = pinv_(sa + sb);
+    T is, irho;
+    r[4] = sb * sa;
+    pinv2_(sa + sb, r[4], is, irho);
     r[0] = (sb * ub + sa * ua) * is;
     r[1] = (sb * vb + sa * va) * is;
     r[2] = (sb * wb + sa * wa) * is;
     r[3] = (sb * hb + sa * ha) * is;
-    r[4] = sb * sa;
+    return irho;
 }
 
 // Contravariant, det-scaled inviscid node flux along metric row m (Viscous.cl:560-611):
@@ -142,54 +184,50 @@ __device__ __forceinline__ void node_flux(T rho, T u, T v, T w, T p, T mx, T my,
     f[4] = D * (Ep * V);
 }
 
-// WCNS-E5 interpolation of one characteristic field to the face between W[2] and W[3]
-// (W[0..5] at offsets -2..+3 from the left node), Weno.cl:1056-1279:
+// WCNS-E5 interpolation of one characteristic field W[0..5] (offsets -2..+3 from the left node) to the
+// face between W[2] and W[3], Weno.cl:1056-1279, from its first differences d_m = W[m+1] - W[m]:
 //   candidates (15/8, -5/4, 3/8), (3/8, 3/4, -1/8), (-1/8, 3/4, 3/8),
 //   Jiang-Shu indicators, w_k = d_k / (eps + IS_k)^2, value = sum w_k q_k / sum w_k.
-// pos = right-biased (d = 1/16, 5/8, 5/16), neg = left-biased (d = 5/16, 5/8, 1/16).
+// pos = right-biased (d = 1/16, 5/8, 5/16), neg = left-biased (d = 5/16, 5/8, 1/16), both as eight
+// times the value less the mean (W[2] + W[3]) / 2: every candidate less that mean is a combination
+// of two neighbouring second differences s_k = d_{k+1} - d_k,
+//   8 (pos q0 - mean) = 3 s3 - 4 s2   8 (pos q1, neg q0) = -s2   8 (pos q2, neg q1) = -s1
+//   8 (neg q2 - mean) = 3 s0 - 4 s1,
+// so no value of W itself is needed, the middle candidates cost nothing, and nothing large cancels.
 template <typename T>
-__device__ __forceinline__ void wcns_pair(const T (&W)[6], T eps, T &pos, T &neg)
+__device__ __forceinline__ void wcns_pair(const T (&d)[5], T eps4, T &pos, T &neg)
 {
-    // the candidates, the second differences and the indicators' first-derivative terms are the
-    // same linear forms of W, written in the first differences d_m = W[m+1] - W[m]
-    const T d0 = W[1] - W[0], d1 = W[2] - W[1], d2 = W[3] - W[2], d3 = W[4] - W[3], d4 = W[5] - W[4];
-    const T h_r = W[3] + T(3.0 / 8.0) * d4 - T(7.0 / 8.0) * d3;    // pos q0 = (15 W3 - 10 W4 + 3 W5) / 8
-    const T h_c = W[3] - T(3.0 / 8.0) * d2 - T(1.0 / 8.0) * d3;    // pos q1 = neg q0 = (3 W2 + 6 W3 - W4) / 8
-    const T h_l = W[2] + T(1.0 / 8.0) * d1 + T(3.0 / 8.0) * d2;    // pos q2 = neg q1 = (-W1 + 6 W2 + 3 W3) / 8
-    const T h_ll = W[2] + T(7.0 / 8.0) * d1 - T(3.0 / 8.0) * d0;   // neg q2 = (3 W0 - 10 W1 + 15 W2) / 8
     // the indicators are formed four times larger, 4 IS = 13/3 s^2 + t^2, from the second
-    // differences s_k = d_{k+1} - d_k (each 13/3 s_k^2 shared by two indicators) and the
-    // first-derivative terms t; with eps also taken four times larger every (eps + IS)^2 carries the
-    // same factor 16, which cancels in the weights
-    const T c13 = T(13.0 / 3.0), eps4 = T(4) * eps;
-    const T s0 = d1 - d0, s1 = d2 - d1, s2 = d3 - d2, s3 = d4 - d3;
+    // differences (each 13/3 s_k^2 shared by two indicators) and the first-derivative terms t; with
+    // eps also taken four times larger (eps4) every (eps + IS)^2 carries the same factor 16, which
+    // cancels in the weights
+    const T c13 = T(13.0 / 3.0);
+    const T s0 = d[1] - d[0], s1 = d[2] - d[1], s2 = d[3] - d[2], s3 = d[4] - d[3];
     // eps + 13/3 s_k^2, each shared by two indicators
     const T S0 = c13 * s0 * s0 + eps4, S1 = c13 * s1 * s1 + eps4, S2 = c13 * s2 * s2 + eps4, S3 = c13 * s3 * s3 + eps4;
-    const T t0 = d4 - T(3) * d3;   // 3 W3 - 4 W4 + W5
-    const T t1 = d2 + d3;          // W4 - W2
-    const T t2 = T(3) * d2 - d1;   // W1 - 4 W2 + 3 W3
-    const T u0 = d3 - T(3) * d2;   // 3 W2 - 4 W3 + W4
-    const T u1 = d1 + d2;          // W3 - W1
-    const T u2 = T(3) * d1 - d0;   // W0 - 4 W1 + 3 W2
-    const T ISp0 = S3 + t0 * t0, ISp1 = S2 + t1 * t1, ISp2 = S1 + t2 * t2;   // eps + IS, four times larger
-    const T ISm0 = S2 + u0 * u0, ISm1 = S1 + u1 * u1, ISm2 = S0 + u2 * u2;
+    const T t0 = d[4] - T(3) * d[3];   // 3 W3 - 4 W4 + W5
+    const T t1 = d[2] + d[3];          // W4 - W2
+    const T t2 = T(3) * d[2] - d[1];   // W1 - 4 W2 + 3 W3
+    const T u0 = d[3] - T(3) * d[2];   // 3 W2 - 4 W3 + W4
+    const T u1 = d[1] + d[2];          // W3 - W1
+    const T u2 = T(3) * d[1] - d[0];   // W0 - 4 W1 + 3 W2
+    T a0 = S3 + t0 * t0, a1 = S2 + t1 * t1, a2 = S1 + t2 * t2;   // eps + IS, four times larger
+    T b0 = S2 + u0 * u0, b1 = S1 + u1 * u1, b2 = S0 + u2 * u2;
     // w_k proportional to d_k * prod_{m != k} (eps + IS_m)^2, so each side needs one division; the
     // linear weights are taken 16 times larger (pos 1, 10, 5; neg 5, 10, 1): the factor cancels in
     // the quotients
     T np_, dp_, nn_, dn_;
     {
-        T a0 = ISp0, a1 = ISp1, a2 = ISp2;
         a0 *= a0; a1 *= a1; a2 *= a2;
-        const T e = a1 * a2, A2 = T(10) * a2, A1 = T(5) * a1;
-        np_ = e * h_r + a0 * (A2 * h_c + A1 * h_l);
-        dp_ = e + a0 * (A2 + A1);
+        const T e = a1 * a2, w = T(5) * a0, a22 = T(2) * a2;
+        np_ = e * (T(3) * s3 - T(4) * s2) - w * (a22 * s2 + a1 * s1);
+        dp_ = e + w * (a22 + a1);
     }
     {
-        T b0 = ISm0, b1 = ISm1, b2 = ISm2;
         b0 *= b0; b1 *= b1; b2 *= b2;
-        const T e = b0 * b1, B1 = T(5) * b1, B0 = T(10) * b0;
-        nn_ = e * h_ll + b2 * (B1 * h_c + B0 * h_l);
-        dn_ = e + b2 * (B1 + B0);
+        const T e = b0 * b1, w = T(5) * b2, b02 = T(2) * b0;
+        nn_ = e * (T(3) * s0 - T(4) * s1) - w * (b1 * s2 + b02 * s1);
+        dn_ = e + w * (b1 + b02);
     }
     if constexpr (!std::is_same<T, float>::value) {
         // one reciprocal serves both sides
@@ -206,69 +244,93 @@ __device__ __forceinline__ void wcns_pair(const T (&W)[6], T eps, T &pos, T &neg
 
 // Characteristic reconstruction of the two interface states of one face
 // (Weno.cl:336-455 eigenvectors and projection, :1056-2187 WCNS, :2188-2287 back projection).
-//   q[m][c]: conserved Q at offsets -2..+3 from the left node
-//   roe = (u, v, w, h, rho) of the face; (kx, ky, kz) = the face metric row over its length
+//   q(m, c): conserved Q at offsets -2..+3 from the left node (m = 0..5)
+//   roe = (u, v, w, h, rho) of the face, irho = 1 / rho; (kx, ky, kz) = the face metric row over its
+//   length
 //   qp / qn: right-biased / left-biased conserved states (not det-scaled)
-template <typename T>
-__device__ __forceinline__ void characteristic_states(const T (&q)[6][5], const T (&roe)[5], T kx, T ky, T kz, T eps,
+// The five first differences of the stencil states are projected, not the six states: the
+// reconstruction needs nothing else, and the interface states are the mean of the two centre
+// states plus the back projection of the corrections.
+template <typename T, typename GetQ>
+__device__ __forceinline__ void characteristic_states(const GetQ &q, const T (&roe)[5], T irho, T kx, T ky, T kz, T eps,
                                                       T (&qp)[5], T (&qn)[5])
 {
     const T u = roe[0], v = roe[1], w = roe[2], h = roe[3], rho = roe[4];
     const T q2 = u * u + v * v + w * w;
-    const T a = psqrt_(T(0.4) * (h - T(0.5) * q2));
+    T a, ia;
+    psqrt_rsq_(T(0.4) * (h - T(0.5) * q2), a, ia);
     const T theta = kx * u + ky * v + kz * w;
     const T phi = T(0.2) * q2;
-    const T irho = pinv_(rho);
-    const T ia = pinv_(a);
     const T iaa = ia * ia;
-    const T s2 = T(0.70710678118654752440);           // 1/sqrt(2)
-    const T alpha = rho * ia * s2;                      // rho / (sqrt2 a)
+    const T s2 = T(0.70710678118654752440);             // 1/sqrt(2)
     const T beta = irho * ia * s2;                      // 1 / (sqrt2 rho a)
     const T g4aa = T(0.4) * iaa;
     const T one_m = T(1) - phi * iaa;
     const T cv = kz * v - ky * w, cw = kx * w - kz * u, cu = ky * u - kx * v;  // u x k
-    const T phi_g = phi * T(2.5);
-    const T hh = (phi + a * a) * T(2.5);
 
-    // Projection W = L q of the 6 stencil states, written through L's structure: rows 0-2 are
+    // Projection L dq of the 5 stencil differences, written through L's structure: rows 0-2 are
     // k_c E + (1/rho) (q_mom x k - (u x k) q0)_c with E = (1 - phi/a^2) q0 + (0.4/a^2) m and
     // m = u.q_mom - q4; rows 3 and 4 are beta (phi q0 - 0.4 m) -/+ beta a (theta q0 - k.q_mom).
     const T ikx = irho * kx, iky = irho * ky, ikz = irho * kz;
     const T icu = irho * cu, icv = irho * cv, icw = irho * cw;
-    const T bphi = beta * phi, b04 = beta * T(0.4), ba = beta * a;
-    T W[5][6];
+    const T bphi = beta * phi, b04 = beta * T(0.4), ba = irho * s2;
+    T W[5][5];
+    T lo[5];
 #pragma unroll
-    for (int m = 0; m < 6; ++m) {
-        const T q0 = q[m][0], qx = q[m][1], qy = q[m][2], qz = q[m][3], q4 = q[m][4];
-        const T mm = u * qx - q4 + v * qy + w * qz;
-        const T nn = kx * qx + ky * qy + kz * qz;
-        const T E = one_m * q0 + g4aa * mm;
-        W[0][m] = kx * E + (ikz * qy - iky * qz - icv * q0);
-        W[1][m] = ky * E + (ikx * qz - ikz * qx - icw * q0);
-        W[2][m] = kz * E + (iky * qx - ikx * qy - icu * q0);
-        const T bA = bphi * q0 - b04 * mm;
-        const T Bv = theta * q0 - nn;
-        W[3][m] = bA - ba * Bv;
-        W[4][m] = bA + ba * Bv;
+    for (int c = 0; c < 5; ++c) lo[c] = q(0, c);
+#pragma unroll
+    for (int m = 0; m < 5; ++m) {
+        T d[5];
+#pragma unroll
+        for (int c = 0; c < 5; ++c) {
+            const T hi = q(m + 1, c);
+            d[c] = hi - lo[c];
+            lo[c] = hi;
+            pin_(lo[c]);
+        }
+        const T mm = u * d[1] - d[4] + v * d[2] + w * d[3];
+        const T B = theta * d[0] - kx * d[1] - ky * d[2] - kz * d[3];
+        const T E = one_m * d[0] + g4aa * mm;
+        W[0][m] = kx * E + (ikz * d[2] - iky * d[3] - icv * d[0]);
+        W[1][m] = ky * E + (ikx * d[3] - ikz * d[1] - icw * d[0]);
+        W[2][m] = kz * E + (iky * d[1] - ikx * d[2] - icu * d[0]);
+        const T bA = bphi * d[0] - b04 * mm;
+        W[3][m] = bA - ba * B;
+        W[4][m] = bA + ba * B;
+#pragma unroll
+        for (int c = 0; c < 5; ++c) pin_(W[c][m]);
     }
+    const T eps4 = T(4) * eps;
     T xp[5], xn[5];
 #pragma unroll
-    for (int c = 0; c < 5; ++c) wcns_pair(W[c], eps, xp[c], xn[c]);
-    // Back projection Q = R x through R's structure: with x' = (x0, x1, x2), X = k.x',
-    // P = alpha (x3 + x4) and M = alpha a (x3 - x4): Q0 = X + P, Q_mom = u Q0 + k M + rho (k x x'),
+    for (int c = 0; c < 5; ++c) {
+        wcns_pair(W[c], eps4, xp[c], xn[c]);
+        pin_(xp[c]);
+        pin_(xn[c]);
+    }
+    // Back projection R x of the corrections through R's structure (x carries the factor 8 of
+    // wcns_pair): with x' = (x0, x1, x2), X = k.x', P = alpha (x3 + x4) and M = alpha a (x3 - x4),
+    // alpha = rho / (sqrt2 a): Q0 = X + P, Q_mom = u Q0 + k M + rho (k x x'),
     // Q4 = (phi/0.4) X + H P + theta M + rho (u x k).x'
-    const T rkx = rho * kx, rky = rho * ky, rkz = rho * kz;
-    const T rcu = rho * cu, rcv = rho * cv, rcw = rho * cw;
-    const T aa = alpha * a;
+    const T k8x = T(0.125) * kx, k8y = T(0.125) * ky, k8z = T(0.125) * kz, r8 = T(0.125) * rho;
+    const T rkx = r8 * kx, rky = r8 * ky, rkz = r8 * kz;
+    const T rcu = r8 * cu, rcv = r8 * cv, rcw = r8 * cw;
+    const T aa = r8 * s2, alpha = aa * ia;
+    const T phi_g = phi * T(2.5);
+    const T hh = phi_g + a * a * T(2.5);
+    T qm[5];
+#pragma unroll
+    for (int c = 0; c < 5; ++c) qm[c] = T(0.5) * (q(2, c) + q(3, c));
     auto back = [&](const T (&x)[5], T (&Q)[5]) {
-        const T X = kx * x[0] + ky * x[1] + kz * x[2];
+        const T X = k8x * x[0] + k8y * x[1] + k8z * x[2];
         const T P = alpha * (x[3] + x[4]);
         const T M = aa * (x[3] - x[4]);
-        Q[0] = X + P;
-        Q[1] = u * Q[0] + kx * M + rky * x[2] - rkz * x[1];
-        Q[2] = v * Q[0] + ky * M + rkz * x[0] - rkx * x[2];
-        Q[3] = w * Q[0] + kz * M + rkx * x[1] - rky * x[0];
-        Q[4] = phi_g * X + hh * P + theta * M + rcv * x[0] + rcw * x[1] + rcu * x[2];
+        const T d0 = X + P;
+        Q[0] = qm[0] + d0;
+        Q[1] = qm[1] + u * d0 + kx * M + rky * x[2] - rkz * x[1];
+        Q[2] = qm[2] + v * d0 + ky * M + rkz * x[0] - rkx * x[2];
+        Q[3] = qm[3] + w * d0 + kz * M + rkx * x[1] - rky * x[0];
+        Q[4] = qm[4] + phi_g * X + hh * P + theta * M + rcv * x[0] + rcw * x[1] + rcu * x[2];
     };
     back(xp, qp);
     back(xn, qn);
@@ -277,10 +339,10 @@ __device__ __forceinline__ void characteristic_states(const T (&q)[6][5], const 
 // n . (F, E, G)(Q) and lambda_5 = n.u + c of one interface state along the unit face normal n
 // (Weno.cl:2291-2507 fluxes, :2511-2581 eigenvalues, :2585-2655 contravariant form: the face's
 // |k| det_f scales the LLF sum once).
+// r = 1 / Q0.
 template <typename T>
-__device__ __forceinline__ void face_state_flux(const T (&Q)[5], T kx, T ky, T kz, T (&c)[5], T &lam)
+__device__ __forceinline__ void face_state_flux(const T (&Q)[5], T r, T kx, T ky, T kz, T (&c)[5], T &lam)
 {
-    const T r = pinv_(Q[0]);
     const T ke = (Q[1] * Q[1] + Q[2] * Q[2] + Q[3] * Q[3]) * r;
     const T P = T(0.4) * (Q[4] - T(0.5) * ke);
     const T Un = (kx * Q[1] + ky * Q[2] + kz * Q[3]) * r;
@@ -294,15 +356,16 @@ __device__ __forceinline__ void face_state_flux(const T (&Q)[5], T kx, T ky, T k
 
 // LLF face flux with alpha = max(|lambda_5|) of the two interface states (Weno.cl:2859-2947):
 // (kx, ky, kz) the unit face normal, dk = det_f |k| of the face metric row k.
-template <typename T>
-__device__ __forceinline__ void face_llf(const T (&q)[6][5], const T (&roe)[5], T kx, T ky, T kz, T dk, T eps,
+template <typename T, typename GetQ>
+__device__ __forceinline__ void face_llf(const GetQ &q, const T (&roe)[5], T irho, T kx, T ky, T kz, T dk, T eps,
                                          T (&llf)[5])
 {
     T qp[5], qn[5];
-    characteristic_states(q, roe, kx, ky, kz, eps, qp, qn);
-    T cp[5], cn[5], lp, ln;
-    face_state_flux(qp, kx, ky, kz, cp, lp);
-    face_state_flux(qn, kx, ky, kz, cn, ln);
+    characteristic_states(q, roe, irho, kx, ky, kz, eps, qp, qn);
+    T cp[5], cn[5], lp, ln, rp, rn;
+    pinv2_(qp[0], qn[0], rp, rn);
+    face_state_flux(qp, rp, kx, ky, kz, cp, lp);
+    face_state_flux(qn, rn, kx, ky, kz, cn, ln);
     const T al = fabs_(lp) >= fabs_(ln) ? fabs_(lp) : fabs_(ln);
     const T hd = T(0.5) * dk;
 #pragma unroll
@@ -328,7 +391,7 @@ __device__ __forceinline__ void face_flux(const T (&q)[6][5], const T (&roe)[5],
 {
     const T kn = sqrt_(k0 * k0 + k1 * k1 + k2 * k2), ik = inv_(kn);
     T llf[5];
-    face_llf(q, roe, k0 * ik, k1 * ik, k2 * ik, detf * kn, eps, llf);
+    face_llf([&](int m, int c) { return q[m][c]; }, roe, pinv_(roe[4]), k0 * ik, k1 * ik, k2 * ik, detf * kn, eps, llf);
 #pragma unroll
     for (int c = 0; c < 5; ++c)
         out[c] = TO(llf[c] + midpoint_correction(nf[0][c], nf[1][c], nf[2][c], nf[3][c], nf[4][c], nf[5][c]));
@@ -388,106 +451,146 @@ template <> __device__ __forceinline__ double prcbrt_<double>(double x)
     return __builtin_fma(y * (1.0 / 3.0), __builtin_fma(-x * y, y * y, 1.0), y);
 }
 
+// The smallest denominator the positive-operand reciprocal and the square root are given in the
+// eddy viscosity: below it |S| or the scale-similarity magnitude is taken as zero.
+template <typename T> __device__ __forceinline__ T tiny_();
+template <> __device__ __forceinline__ double tiny_<double>() { return 1e-280; }
+template <> __device__ __forceinline__ float tiny_<float>() { return 1e-35f; }
+
+// U_c / U_0 of a node: velocity (0..2) and E / rho (3), with 1 / U_0.
 template <typename T>
-__device__ __forceinline__ T viscous_node(const T (&dU)[5][3], const T (&U)[5], T u, T v, T w, const T (&m)[9], T D,
-                                          const T (&KS)[3], const ViscParams &vp, T (&fvis)[3][5])
+struct NodeRatios {
+    T iU0, r[4];
+};
+template <typename T>
+__device__ __forceinline__ NodeRatios<T> node_ratios(const T (&U)[5])
 {
-    const T C_MTS = T(vp.c_mts);
-    const T iU0 = pinv_(U[0]);
-    const T iU02 = iU0 * iU0;
-    T ug[3], vg[3], wg[3], tg[3];
+    NodeRatios<T> n;
+    n.iU0 = pinv_(U[0]);
 #pragma unroll
-    for (int d = 0; d < 3; ++d) {
-        ug[d] = iU0 * dU[1][d] - (U[1] * iU02) * dU[0][d];
-        vg[d] = iU0 * dU[2][d] - (U[2] * iU02) * dU[0][d];
-        wg[d] = iU0 * dU[3][d] - (U[3] * iU02) * dU[0][d];
+    for (int c = 0; c < 4; ++c) n.r[c] = U[1 + c] * n.iU0;
+    return n;
+}
+
+// Adds the part of direction d to the Cartesian gradients G[0..3][x, y, z] of u, v, w and the internal
+// energy: X_x = X_zeta zeta_x + X_eta eta_x + X_xi xi_x, one direction at a time (dU = dU_c / d(zeta,
+// eta, xi)_d, (mx, my, mz) the metric row of d), so that a kernel holds twelve gradients instead of
+// fifteen differences and nine metrics (k_visc in FP64: 167 VGPRs with all directions held).
+template <typename T>
+__device__ __forceinline__ void add_gradient(const T (&dU)[5], const NodeRatios<T> &n, T mx, T my, T mz, T (&G)[4][3])
+{
+    T g[4];
+#pragma unroll
+    for (int c = 0; c < 4; ++c) g[c] = n.iU0 * (dU[1 + c] - n.r[c] * dU[0]);
+    g[3] = g[3] - n.r[0] * g[0] - n.r[1] * g[1] - n.r[2] * g[2];
+#pragma unroll
+    for (int c = 0; c < 4; ++c) {
+        G[c][0] += g[c] * mx;
+        G[c][1] += g[c] * my;
+        G[c][2] += g[c] * mz;
     }
-#pragma unroll
-    for (int d = 0; d < 3; ++d)
-        tg[d] = iU0 * dU[4][d] - (U[4] * iU02) * dU[0][d] - (U[1] * iU0) * ug[d] - (U[2] * iU0) * vg[d] - (U[3] * iU0) * wg[d];
-    // Cartesian gradients: X_x = X_zeta zeta_x + X_eta eta_x + X_xi xi_x, etc.
-    const T ux = ug[0] * m[0] + ug[1] * m[3] + ug[2] * m[6];
-    const T uy = ug[0] * m[1] + ug[1] * m[4] + ug[2] * m[7];
-    const T uz = ug[0] * m[2] + ug[1] * m[5] + ug[2] * m[8];
-    const T vx = vg[0] * m[0] + vg[1] * m[3] + vg[2] * m[6];
-    const T vy = vg[0] * m[1] + vg[1] * m[4] + vg[2] * m[7];
-    const T vz = vg[0] * m[2] + vg[1] * m[5] + vg[2] * m[8];
-    const T wx = wg[0] * m[0] + wg[1] * m[3] + wg[2] * m[6];
-    const T wy = wg[0] * m[1] + wg[1] * m[4] + wg[2] * m[7];
-    const T wz = wg[0] * m[2] + wg[1] * m[5] + wg[2] * m[8];
-    const T ex = tg[0] * m[0] + tg[1] * m[3] + tg[2] * m[6];
-    const T ey = tg[0] * m[1] + tg[1] * m[4] + tg[2] * m[7];
-    const T ez = tg[0] * m[2] + tg[1] * m[5] + tg[2] * m[8];
+}
+
+// Viscous and SGS node fluxes from the Cartesian gradients. (u, v, w): the velocity in the work
+// terms; sk: the magnitudes of the scale-similarity terms (square roots of KS_x, KS_y, KS_z).
+template <typename T>
+__device__ __forceinline__ T viscous_fluxes(const T (&G)[4][3], const T (&U)[5], const NodeRatios<T> &n, T u, T v, T w,
+                                            const T (&m)[9], T D, const T (&sk)[3], const ViscParams &vp, T (&fvis)[3][5])
+{
+    const T ux = G[0][0], uy = G[0][1], uz = G[0][2];
+    const T vx = G[1][0], vy = G[1][1], vz = G[1][2];
+    const T wx = G[2][0], wy = G[2][1], wz = G[2][2];
+    const T ex = G[3][0], ey = G[3][1], ez = G[3][2];
+    const T C_MTS = T(vp.c_mts);
 
     // Viscous.cl:455-458: T = gamma M^2 (gamma-1) e, Sutherland mu with S = 110.4
-    const T d_temp = T(vp.tfac) * (U[4] * iU0 - T(0.5) * ((U[1] * U[1] + U[2] * U[2] + U[3] * U[3]) * iU02));
+    const T d_temp = T(vp.tfac) * (n.r[3] - T(0.5) * (n.r[0] * n.r[0] + n.r[1] * n.r[1] + n.r[2] * n.r[2]));
     const T st = psqrt_(d_temp);
-    const T mu = (st * st * st) * (T(vp.suth1) * pinv_(d_temp + T(vp.suth)));
+    const T mu = (st * d_temp) * (T(vp.suth1) * pinv_(d_temp + T(vp.suth)));
     // Viscous.cl:461-476 heat flux and Stokes stresses
     const T kq = -(mu * T(vp.kheat));
     const T qx = kq * ex, qy = kq * ey, qz = kq * ez;
     const T mr = mu * T(vp.inv_reyl);
-    const T txx = mr * (T(4.0 / 3.0) * ux - T(2.0 / 3.0) * vy - T(2.0 / 3.0) * wz);
-    const T tyy = mr * (T(4.0 / 3.0) * vy - T(2.0 / 3.0) * ux - T(2.0 / 3.0) * wz);
-    const T tzz = mr * (T(4.0 / 3.0) * wz - T(2.0 / 3.0) * ux - T(2.0 / 3.0) * vy);
-    const T txy = mr * (uy + vx);
-    const T txz = mr * (uz + wx);
-    const T tyz = mr * (vz + wy);
-    // Viscous.cl:490-558 mixed-time-scale eddy viscosity, one per direction
-    const T sxy = T(0.5) * (uy + vx), syz = T(0.5) * (vz + wy), sxz = T(0.5) * (wx + uz);
-    const T sxx = ux, syy = vy, szz = wz;
-    const T mod = sqrt_(T(2) * ((sxy * sxy + syz * syz + sxz * sxz) + T(2.0 / 3.0) * (sxx * sxx + syy * syy + szz * szz)));
+    const T sxy2 = uy + vx, syz2 = vz + wy, sxz2 = wx + uz;
+    const T dv = T(2.0 / 3.0) * (ux + vy + wz);
+    const T txx = mr * (T(2) * ux - dv);
+    const T tyy = mr * (T(2) * vy - dv);
+    const T tzz = mr * (T(2) * wz - dv);
+    const T txy = mr * sxy2, txz = mr * sxz2, tyz = mr * syz2;
+    // Viscous.cl:490-558 mixed-time-scale eddy viscosity, one per direction: with S_xy = sxy2 / 2,
+    // |S|^2 = 2 (S_xy^2 + S_yz^2 + S_xz^2 + 2/3 (S_xx^2 + S_yy^2 + S_zz^2))
+    const T off = sxy2 * sxy2 + syz2 * syz2 + sxz2 * sxz2, diag = ux * ux + vy * vy + wz * wz;
     const T DEL = prcbrt_(D);
     T eddy[3];
     if (vp.sgs == 1) {
         // Smagorinsky (no reference counterpart): nu_t = (C_s Delta)^2 |S| with Delta = det^(1/3) and
         // |S| = sqrt(2 S_ij S_ij), the same in every direction. The SGS stress below is
         // -2 U0 eddy S_ij with U0 = det rho, so eddy = nu_t / det = C_s^2 |S| det^(-1/3) = C_s^2 |S| DEL.
-        const T s2 = T(2) * (sxx * sxx + syy * syy + szz * szz) + T(4) * (sxy * sxy + syz * syz + sxz * sxz);
-        const T e = T(vp.cs2) * DEL * sqrt_(s2);
+        const T s2 = T(2) * diag + off;
+        const T e = T(vp.cs2) * DEL * (s2 > tiny_<T>() ? psqrt_(s2) : T(0));
         eddy[0] = e; eddy[1] = e; eddy[2] = e;
     } else {
+        const T s2 = T(0.5) * off + T(4.0 / 3.0) * diag;
+        const T dm = DEL * (s2 > tiny_<T>() ? psqrt_(s2) : T(0)) * T(vp.inv_ct);
+        const T cd = C_MTS * DEL;
 #pragma unroll
         for (int d = 0; d < 3; ++d) {
-            const T sk = sqrt_(KS[d]);
-            if (mod != T(0)) {
-                // C_MTS / (1 + R / C_T) * DEL * sk with R = DEL |S| / sk, written with one division
-                // (sk = 0 gives R = inf and a zero eddy viscosity either way)
-                eddy[d] = (C_MTS * DEL * sk * sk) * pinv_(sk + DEL * mod * T(vp.inv_ct));
-            } else {
-                eddy[d] = C_MTS * DEL * sk;
-            }
+            // C_MTS / (1 + R / C_T) * DEL * sk with R = DEL |S| / sk, written with one division (sk = 0
+            // gives R = inf and a zero eddy viscosity either way; |S| = 0 gives C_MTS DEL sk)
+            const T den = sk[d] + dm;
+            eddy[d] = den > tiny_<T>() ? (cd * sk[d] * sk[d]) * pinv_(den) : cd * sk[d];
         }
     }
     // SGS stresses scale with U0 = det * rho (Viscous.cl:529-535)
-    const T m2U = T(-2) * U[0];
-    const T Sxy = m2U * eddy[0] * sxy, Syz = m2U * eddy[1] * syz, Sxz = m2U * eddy[2] * sxz;
-    const T Sxx = m2U * eddy[0] * sxx, Syy = m2U * eddy[1] * syy, Szz = m2U * eddy[2] * szz;
+    const T mU = -U[0];
+    const T e0 = mU * eddy[0], e1 = mU * eddy[1], e2 = mU * eddy[2];   // -2 U0 eddy S_ij = e (2 S_ij)
+    const T Sxy = e0 * sxy2, Syz = e1 * syz2, Sxz = e2 * sxz2;
+    const T Sxx = e0 * (T(2) * ux), Syy = e1 * (T(2) * vy), Szz = e2 * (T(2) * wz);
     T Hx, Hy, Hz;
     if (vp.sgs == 1) {
         // Smagorinsky: the molecular forms with rho nu_t (= U0 eddy) for mu / Re: heat flux
         // -1.4 rho nu_t / Pr grad e, and the work of the SGS stresses
-        const T kS = -(T(vp.kheat_t) * (U[0] * eddy[0]));
+        const T kS = T(vp.kheat_t) * e0;
         Hx = kS * ex + (u * Sxx + v * Sxy + w * Sxz);
         Hy = kS * ey + (u * Sxy + v * Syy + w * Syz);
         Hz = kS * ez + (u * Sxz + v * Syz + w * Szz);
     } else {
-        const T kQ = T(vp.kQ);
-        const T Qx = kQ * eddy[0] * ex, Qy = kQ * eddy[1] * ey, Qz = kQ * eddy[2] * ez;
-        const T DX = (Sxx + Sxy + Sxz) * u, DY = (Sxy + Syy + Syz) * v, DZ = (Sxz + Syz + Szz) * w;
-        // H = Q + DEL and D = 0.4 Q (Viscous.cl:549-557)
-        Hx = Qx + DX + T(0.4) * Qx; Hy = Qy + DY + T(0.4) * Qy; Hz = Qz + DZ + T(0.4) * Qz;
+        // H = Q + DEL and D = 0.4 Q (Viscous.cl:549-557): 1.4 Q + (row sum) times the velocity component
+        const T kQ = T(1.4) * T(vp.kQ);
+        Hx = kQ * eddy[0] * ex + (Sxx + Sxy + Sxz) * u;
+        Hy = kQ * eddy[1] * ey + (Sxy + Syy + Syz) * v;
+        Hz = kQ * eddy[2] * ez + (Sxz + Syz + Szz) * w;
     }
     // Viscous.cl:576-595 Cartesian viscous fluxes
-    const T tF[5] = {T(0), -txx + Sxx, -txy + Sxy, -txz + Sxz, (-u * txx - v * txy - w * txz) + qx + Hx};
-    const T tE[5] = {T(0), -txy + Sxy, -tyy + Syy, -tyz + Syz, (-u * txy - v * tyy - w * tyz) + qy + Hy};
-    const T tG[5] = {T(0), -txz + Sxz, -tyz + Syz, -tzz + Szz, (-u * txz - v * tyz - w * tzz) + qz + Hz};
+    const T tF[5] = {T(0), Sxx - txx, Sxy - txy, Sxz - txz, (-u * txx - v * txy - w * txz) + qx + Hx};
+    const T tE[5] = {T(0), Sxy - txy, Syy - tyy, Syz - tyz, (-u * txy - v * tyy - w * tyz) + qy + Hy};
+    const T tG[5] = {T(0), Sxz - txz, Syz - tyz, Szz - tzz, (-u * txz - v * tyz - w * tzz) + qz + Hz};
     // Viscous.cl:615-631 contravariant and det-scaled
 #pragma unroll
-    for (int d = 0; d < 3; ++d)
+    for (int d = 0; d < 3; ++d) {
+        const T a = D * m[3 * d], b = D * m[3 * d + 1], c3 = D * m[3 * d + 2];
+        fvis[d][0] = T(0);
 #pragma unroll
-        for (int c = 0; c < 5; ++c) fvis[d][c] = D * (m[3 * d] * tF[c] + m[3 * d + 1] * tE[c] + m[3 * d + 2] * tG[c]);
+        for (int c = 1; c < 5; ++c) fvis[d][c] = a * tF[c] + b * tE[c] + c3 * tG[c];
+    }
     return mu;
+}
+
+// The same from all differences at once. KS[3]: the scale-similarity terms, squared.
+template <typename T>
+__device__ __forceinline__ T viscous_node(const T (&dU)[5][3], const T (&U)[5], T u, T v, T w, const T (&m)[9], T D,
+                                          const T (&KS)[3], const ViscParams &vp, T (&fvis)[3][5])
+{
+    const NodeRatios<T> n = node_ratios(U);
+    T G[4][3] = {};
+    T sk[3];
+#pragma unroll
+    for (int d = 0; d < 3; ++d) {
+        const T dUd[5] = {dU[0][d], dU[1][d], dU[2][d], dU[3][d], dU[4][d]};
+        add_gradient(dUd, n, m[3 * d], m[3 * d + 1], m[3 * d + 2], G);
+        sk[d] = sqrt_(KS[d]);
+    }
+    return viscous_fluxes(G, U, n, u, v, w, m, D, sk, vp, fvis);
 }
 
 // One-direction derivative of Viscous.cl:285-435 (weno_form = false) or Weno.cl:2732-2856

@@ -102,10 +102,10 @@ int cfdx_ctx_create(int device, void *stream, cfdx_ctx **out);
 int cfdx_ctx_destroy(cfdx_ctx *ctx);
 int cfdx_ctx_set_stream(cfdx_ctx *ctx, void *stream);
 void *cfdx_ctx_stream(cfdx_ctx *ctx);
-/* Overlap (no reference counterpart): mixed-precision block and batch stages, and the FP64 stages
- * of a captured batch graph, run the viscous node kernel on a second stream of the context, beside
- * the face sweeps of the same stage (forked from and joined back to the context's stream by events;
- * a captured batch graph holds both). On by
+/* Overlap (no reference counterpart): the viscous node kernel and the face sweeps of a stage run
+ * together: in one launch with the default tile shapes and grid, otherwise with the viscous kernel on
+ * a second stream of the context (forked from and joined back to the context's stream by events; a
+ * captured batch graph holds both). Off: one kernel after the other on the context's stream. On by
  * default (environment CFDX_OVERLAP=0 turns the default off); timed passes (cfdx_block_set_timing)
  * always run in order. Changing it (or the stream, cfdx_ctx_set_stream) makes the batches of the
  * context capture their step again at their next cfdx_batch_step. */

@@ -1,0 +1,87 @@
+"""The launch that takes a stage's viscous node tiles and face sweeps together (GPU): bitwise the results
+of the kernels run one after the other, over the shapes where its tile bookkeeping can go wrong: the
+smallest blocks, partial tiles in every direction, fewer tiles than XCDs, kinds with very different
+tile counts, bounded blocks with their shells, inviscid blocks, lists of both."""
+import math
+
+import numpy as np
+import pytest
+
+import cfdx
+from test_gpu_bounded import CASES, perturbed
+
+pytestmark = pytest.mark.gpu
+FIELDS = ("rho", "u", "v", "w", "p", "mu")
+
+
+@pytest.fixture(scope="module")
+def ctx():
+    if cfdx.device_count() < 1:
+        pytest.skip("no HIP device")
+    c = cfdx.Ctx(0)
+    yield c
+    c.set_overlap(True)
+
+
+def periodic(ctx, shape, precision, prm):
+    b = cfdx.Block(*shape, precision=precision, ctx=ctx)
+    b.init_case(grid="sinusoid", length=(2 * math.pi,) * 3, amp=0.05 * 2 * math.pi / max(shape), phases=(0.3, 1.1, 2.0),
+                init="tgv", mach=0.3)
+    b.configure(0.3, 0.02 * 2 * math.pi / max(shape), prm)
+    return b
+
+
+def bounded(ctx, name, precision):
+    d, xyz, geo, mach, aoa, pk = CASES[name]()
+    prm = cfdx.default_params(**pk)
+    b = cfdx.Block(d.ni, d.nj, d.nk, precision=precision, ctx=ctx, desc=cfdx.BlockDesc.from_buffer_copy(d))
+    b.set_geometry_soa(geo)
+    b.configure(mach, 0.0, prm)
+    b.set_flow(perturbed(xyz[cfdx.owned_index(d)], mach, aoa))
+    b.configure(mach, 0.5 * b.cfl_dt(0.5), prm)
+    return b
+
+
+def both(ctx, make, steps):
+    """The flows of make()'s blocks after `steps` batch steps, together and apart."""
+    out = []
+    for on in (True, False):
+        ctx.set_overlap(on)
+        blocks = make()
+        q = cfdx.Batch(blocks[0].precision, ctx)
+        for b in blocks:
+            q.add(b)
+        q.step(steps, False)
+        out.append([b.get_flow() for b in blocks])
+        q.close()
+        for b in blocks:
+            b.close()
+    ctx.set_overlap(True)
+    return out
+
+
+def same(pair):
+    for a, r in zip(*pair):
+        for f in FIELDS:
+            assert np.array_equal(a[f], r[f]), f
+            assert np.isfinite(a[f]).all(), f
+
+
+@pytest.mark.parametrize("precision", [cfdx.FP64, cfdx.MIXED], ids=["fp64", "mixed"])
+@pytest.mark.parametrize("viscous", [True, False], ids=["viscous", "inviscid"])
+@pytest.mark.parametrize("shape", [(3, 3, 3), (4, 3, 90), (130, 3, 5), (3, 75, 4), (64, 16, 16), (65, 17, 19), (128, 4, 33)],
+                         ids=lambda s: "x".join(map(str, s)))
+def test_one_launch_gives_the_bits_of_the_kernels_apart(ctx, shape, viscous, precision):
+    prm = cfdx.default_params(mach=0.3, reyl=900.0) if viscous else cfdx.euler_params()
+    same(both(ctx, lambda: [periodic(ctx, shape, precision, prm)], 2))
+
+
+@pytest.mark.parametrize("precision", [cfdx.FP64, cfdx.MIXED], ids=["fp64", "mixed"])
+def test_one_launch_over_a_mixed_list(ctx, precision):
+    """Bounded and periodic, viscous and inviscid blocks of uneven sizes in one list."""
+    visc, inv = cfdx.default_params(mach=0.3, reyl=900.0), cfdx.euler_params()
+
+    def make():
+        return ([periodic(ctx, s, precision, p) for s, p in (((5, 4, 3), visc), ((40, 21, 9), inv), ((66, 10, 7), visc))]
+                + [bounded(ctx, n, precision) for n in CASES])
+    same(both(ctx, make, 2))
