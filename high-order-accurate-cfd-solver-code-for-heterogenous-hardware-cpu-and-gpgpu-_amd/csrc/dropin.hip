@@ -79,7 +79,7 @@ __global__ void __launch_bounds__(256) k_uq(double *__restrict__ U_C, double *__
 // ---------------------------------------------------------------------------
 // Viscous.cl:23-643
 // ---------------------------------------------------------------------------
-__global__ void __launch_bounds__(128) k_viscous(const double *__restrict__ U_C, double *__restrict__ Fo, double *__restrict__ Eo,
+__global__ void __launch_bounds__(128, 4) k_viscous(const double *__restrict__ U_C, double *__restrict__ Fo, double *__restrict__ Eo,
                                                  double *__restrict__ Go, double *__restrict__ Fvo, double *__restrict__ Evo,
                                                  double *__restrict__ Gvo, const int32_t *__restrict__ G,
                                                  const double *__restrict__ metric, const double *__restrict__ det,
@@ -87,38 +87,44 @@ __global__ void __launch_bounds__(128) k_viscous(const double *__restrict__ U_C,
 {
     const int g = blockIdx.x * blockDim.x + threadIdx.x;
     if (g >= n) return;
-    double dU[5][3];
-    double KS[3];
     double U[5];
 #pragma unroll
     for (int c = 0; c < 5; ++c) U[c] = U_C[(size_t)5 * g + c];
+    const NodeRatios<double> nr = node_ratios(U);
+    double Gr[4][3] = {}, sk[3], m[9];
 #pragma unroll
     for (int d = 0; d < 3; ++d) {
         int idx[7];
         walk(G, g, d, idx);
         int loc[7];
 #pragma unroll
-        for (int s = 0; s < 7; ++s) loc[s] = G[GRID_N * idx[s] + G_LOC];
+        for (int s = 1; s < 6; ++s) loc[s] = G[GRID_N * idx[s] + G_LOC];
+        double dU[5];
 #pragma unroll
         for (int c = 0; c < 5; ++c) {
             double f[7];
 #pragma unroll
             for (int s = 0; s < 7; ++s) f[s] = U_C[(size_t)5 * idx[s] + c];
-            dU[c][d] = loc_derivative(f, loc[3], loc[1], loc[2], loc[4], loc[5], false);
+            dU[c] = loc_derivative(f, loc[3], loc[1], loc[2], loc[4], loc[5], false);
+            pin_(dU[c]);
         }
-        // MTS scale-similarity term of momentum component d+1 along d (Viscous.cl:493-495)
+        // magnitude of the MTS scale-similarity term of momentum component d+1 along d (Viscous.cl:493-495)
         const double *um = U_C + (size_t)5 * idx[2], *up = U_C + (size_t)5 * idx[4];
-        const double a = (U[1 + d] / U[0]) - ((0.25 * um[1 + d] + 0.5 * U[1 + d] + 0.25 * up[1 + d]) / (0.25 * um[0] + 0.5 * U[0] + 0.25 * up[0]));
-        KS[d] = a * a;
-    }
-    double m[9];
+        sk[d] = fabs_(nr.r[d] - ((0.25 * um[1 + d] + 0.5 * U[1 + d] + 0.25 * up[1 + d]) * pinv_(0.25 * um[0] + 0.5 * U[0] + 0.25 * up[0])));
+        pin_(sk[d]);
 #pragma unroll
-    for (int c = 0; c < 9; ++c) m[c] = metric[(size_t)MET_N * g + c];
+        for (int c = 3 * d; c < 3 * d + 3; ++c) m[c] = metric[(size_t)MET_N * g + c];
+        add_gradient(dU, nr, m[3 * d], m[3 * d + 1], m[3 * d + 2], Gr);
+#pragma unroll
+        for (int c = 0; c < 4; ++c)
+#pragma unroll
+            for (int x = 0; x < 3; ++x) pin_(Gr[c][x]);
+    }
     const double D = det[g];
     double *f = FLOW + (size_t)FLOW_N * g;
     const double rho = f[F_RHO], u = f[F_U], v = f[F_V], w = f[F_W], p = f[F_P];
     double fv[3][5];
-    const double mu = viscous_node(dU, U, u, v, w, m, D, KS, vp, fv);
+    const double mu = viscous_fluxes(Gr, U, nr, u, v, w, m, D, sk, vp, fv);
     double *outv[3] = {Fvo, Evo, Gvo};
     double *outi[3] = {Fo, Eo, Go};
 #pragma unroll
@@ -137,7 +143,7 @@ __global__ void __launch_bounds__(128) k_viscous(const double *__restrict__ U_C,
 // ---------------------------------------------------------------------------
 // Weno.cl:36-3137
 // ---------------------------------------------------------------------------
-__global__ void __launch_bounds__(128) k_weno(int j, double Mach, double del_t, const double *__restrict__ deter,
+__global__ void __launch_bounds__(64 * 6, 3) k_weno(int j, double Mach, double del_t, const double *__restrict__ deter,
                                               const double *__restrict__ det, double *__restrict__ U0, double *__restrict__ U1,
                                               double *__restrict__ U2, const int32_t *__restrict__ G,
                                               const double *__restrict__ Q_C, const double *__restrict__ metric,
@@ -146,51 +152,55 @@ __global__ void __launch_bounds__(128) k_weno(int j, double Mach, double del_t, 
                                               const double *__restrict__ F, const double *__restrict__ E,
                                               const double *__restrict__ Gf, double *__restrict__ FLOW, int n, double eps)
 {
-    const int g = blockIdx.x * blockDim.x + threadIdx.x;
-    if (g >= n) return;
-    const double *nodeF[3] = {F, E, Gf};
-    const double *nodeV[3] = {Fv, Ev, Gv};
-    double L[5] = {0, 0, 0, 0, 0};
-    double dvis[3][5];
-#pragma unroll 1
-    for (int d = 0; d < 3; ++d) {
+    // one wave per (direction, side) of 64 nodes' faces: a face at a time keeps the kernel under 168 registers
+    // (3 waves per SIMD) and gives a small mesh six times the waves. Both faces of a node on one thread, one
+    // direction after the other, took 406 (one wave per SIMD).
+    __shared__ double face[6][5][64], vis[3][5][64];
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), d = wave >> 1, side = wave & 1;
+    const int g = blockIdx.x * 64 + lane;
+    if (g < n) {
         int idx[7];
         walk(G, g, d, idx);
-        double hp[5], hm[5];
+        // plus face: stencil offsets -2..+3 from g; minus face: -3..+2 (left node g-1)
+        size_t at[6];
 #pragma unroll
-        for (int side = 0; side < 2; ++side) {
-            // plus face: stencil offsets -2..+3 from g; minus face: -3..+2 (left node g-1)
-            const int o = side == 0 ? 1 : 0;
-            double q[6][5], nf[6][5];
-#pragma unroll
-            for (int s = 0; s < 6; ++s)
-#pragma unroll
-                for (int c = 0; c < 5; ++c) {
-                    q[s][c] = Q_C[(size_t)5 * idx[s + o] + c];
-                    nf[s][c] = nodeF[d][(size_t)5 * idx[s + o] + c];
-                }
-            // ROE slots ip, jp, kp, im, jm, km; metric faces ip, im, jp, jm, kp, km; deter ip, im, jp, jm, kp, km
-            const double *ro = ROE + (size_t)ROE_N * g + 6 * (side == 0 ? d : 3 + d);
-            const double roe[5] = {ro[0], ro[1], ro[2], ro[4], ro[5]};
-            const double *k = metric + (size_t)MET_N * g + 9 + 9 * (2 * d + side) + 3 * d;
-            const double detf = deter[(size_t)DET_N * g + 2 * d + side];
-            if (side == 0) face_flux(q, roe, k[0], k[1], k[2], detf, eps, nf, hp);
-            else face_flux(q, roe, k[0], k[1], k[2], detf, eps, nf, hm);
+        for (int s = 0; s < 6; ++s) {
+            const int p = idx[s + 1], m = idx[s];
+            at[s] = (size_t)5 * (side == 0 ? p : m);
         }
-        int loc[7];
+        // ROE slots ip, jp, kp, im, jm, km; metric faces ip, im, jp, jm, kp, km; deter ip, im, jp, jm, kp, km
+        const double *ro = ROE + (size_t)ROE_N * g + 6 * (side == 0 ? d : 3 + d);
+        const double roe[5] = {ro[0], ro[1], ro[2], ro[4], ro[5]};
+        const double *k = metric + (size_t)MET_N * g + 9 + 9 * (2 * d + side) + 3 * d;
+        const double detf = deter[(size_t)DET_N * g + 2 * d + side];
+        const double *nf = d == 0 ? F : d == 1 ? E : Gf;
+        double h[5];
+        face_flux([&](int m, int c) { return Q_C[at[m] + c]; }, roe, k[0], k[1], k[2], detf, eps,
+                  [&](int m, int c) { return nf[at[m] + c]; }, h);
 #pragma unroll
-        for (int s = 0; s < 7; ++s) loc[s] = G[GRID_N * idx[s] + G_LOC];
+        for (int c = 0; c < 5; ++c) face[wave][c][lane] = h[c];
+        if (side == 0) {
+            const double *nv = d == 0 ? Fv : d == 1 ? Ev : Gv;
+            int loc[7];
 #pragma unroll
-        for (int c = 0; c < 5; ++c) {
-            double fv[7];
+            for (int s = 1; s < 6; ++s) loc[s] = G[GRID_N * idx[s] + G_LOC];
 #pragma unroll
-            for (int s = 0; s < 7; ++s) fv[s] = nodeV[d][(size_t)5 * idx[s] + c];
-            dvis[d][c] = loc_derivative(fv, loc[3], loc[1], loc[2], loc[4], loc[5], true);
-            L[c] += hp[c] - hm[c];
+            for (int c = 0; c < 5; ++c) {
+                double fv[7];
+#pragma unroll
+                for (int s = 0; s < 7; ++s) fv[s] = nv[(size_t)5 * idx[s] + c];
+                vis[d][c][lane] = loc_derivative(fv, loc[3], loc[1], loc[2], loc[4], loc[5], true);
+            }
         }
     }
+    __syncthreads();
+    if (wave != 0 || g >= n) return;
+    double L[5];
 #pragma unroll
-    for (int c = 0; c < 5; ++c) L[c] = -(L[c] + dvis[0][c] + dvis[1][c] + dvis[2][c]);   // Weno.cl:3078-3082
+    for (int c = 0; c < 5; ++c) {
+        const double f = (face[0][c][lane] - face[1][c][lane]) + (face[2][c][lane] - face[3][c][lane]) + (face[4][c][lane] - face[5][c][lane]);
+        L[c] = -(f + vis[0][c][lane] + vis[1][c][lane] + vis[2][c][lane]);   // Weno.cl:3078-3082
+    }
 
     // Weno.cl:3084-3126 SSP-RK3 stage j
     double fu[5];
@@ -270,7 +280,7 @@ extern "C" int cfdx_weno(cfdx_ctx *ctx, int j, double Mach, double del_t, const 
     if (n_launch == 0) return CFDX_OK;
     cfdx_params d;
     if (!params) { cfdx_params_default(&d); params = &d; }
-    hipLaunchKernelGGL(k_weno, dim3(cfdx::blocks_for(n_launch, 128)), dim3(128), 0, ctx->stream, j, Mach, del_t,
+    hipLaunchKernelGGL(k_weno, dim3(cfdx::blocks_for(n_launch, 64)), dim3(64 * 6), 0, ctx->stream, j, Mach, del_t,
                        (const double *)deter, det, (double *)U0, (double *)U1, (double *)U2, (const int32_t *)Grid_P,
                        (const double *)Q_C, (const double *)metric, (const double *)ROE_AVER, (const double *)Fv,
                        (const double *)Ev, (const double *)Gv, (const double *)F, (const double *)E, (const double *)G,
