@@ -59,7 +59,6 @@ struct BlockDev {
     void *Fv[3][4];             // viscous fluxes, components 1..4 (the mass component is identically 0)
     double *mu;
     void *FH[3][5];             // face fluxes F-hat at the +1/2 faces
-    double *Lout;               // RHS output (mode 3)
     double *mon;                // residual monitor: per-wave max |du|, |dv|, |de| of the last step (null: off)
     double del_t, mach, eps;
     int viscous;
@@ -98,6 +97,7 @@ struct LaunchList {
     uint32_t bc_face_d[3] = {};       // the same per direction (0: no block bounded in that direction)
     bool any_cut = false;             // some block has a wake cut
     uint32_t shell_max = 0;           // largest shell of the bounded blocks
+    double *Lout = nullptr;           // mode 3 (a single block): the right-hand side, 5 x owned nodes
 };
 
 // kernels (block_kernels.hip)

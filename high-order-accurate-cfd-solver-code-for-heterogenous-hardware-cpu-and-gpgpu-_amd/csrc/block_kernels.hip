@@ -594,13 +594,13 @@ __global__ void __launch_bounds__(256, 4) k_flux(const BlockDev *__restrict__ bl
 
 // ---------------------------------------------------------------------------
 // update kernel: L and the SSP-RK3 stage (Weno.cl:3060-3135), in double.
-//   mode 0..2: RK stage j; mode 3: write L to the block's Lout only
+//   mode 0..2: RK stage j; mode 3: write L only, to Lout (owned order, component-major)
 // ---------------------------------------------------------------------------
 // L and the SSP-RK3 stage of one node; mdu / mdv / mde: the node's monitor values (mode 2 with
 // the monitor on). LOC as in visc_node.
 template <typename S, bool LOC, bool NT>
-__device__ __forceinline__ void update_node(const BlockDev &B, int i, int j, int k, int mode, double &mdu, double &mdv,
-                                            double &mde)
+__device__ __forceinline__ void update_node(const BlockDev &B, int i, int j, int k, int mode, double *Lout, double &mdu,
+                                            double &mdv, double &mde)
 {
     const uint32_t g = node_index(B, i, j, k);
     double L[5] = {0, 0, 0, 0, 0};
@@ -642,8 +642,9 @@ __device__ __forceinline__ void update_node(const BlockDev &B, int i, int j, int
 #pragma unroll
     for (int c = 0; c < 5; ++c) L[c] = -L[c];
     if (mode == 3) {
+        const size_t no = (size_t)B.ni * B.nj * B.nk, o = (size_t)i + (size_t)B.ni * ((size_t)j + (size_t)B.nj * k);
 #pragma unroll
-        for (int c = 0; c < 5; ++c) B.Lout[(size_t)c * B.n + g] = L[c];
+        for (int c = 0; c < 5; ++c) Lout[c * no + o] = L[c];
     } else {
         const double del_t = B.del_t;
         double un[5], u0[5];
@@ -701,7 +702,8 @@ __device__ __forceinline__ void monitor_wave(const BlockDev &B, uint32_t slot, d
 // waves per tile), one per wave of 64 shell nodes
 template <typename S, int TX, int TY, bool BND, bool LOOP>
 __global__ void __launch_bounds__(TX *TY) k_update(const BlockDev *__restrict__ blks, const uint32_t *__restrict__ prefix,
-                                                   uint32_t nblk, uint32_t total, int mode, uint32_t shell_tiles)
+                                                   uint32_t nblk, uint32_t total, int mode, uint32_t shell_tiles,
+                                                   double *Lout)
 {
     const uint32_t all = total + (BND ? nblk * shell_tiles : 0u);
     auto tile = [&](uint32_t wg) {
@@ -716,7 +718,7 @@ __global__ void __launch_bounds__(TX *TY) k_update(const BlockDev *__restrict__ 
             if (t < ns) {
                 int i, j, k;
                 shell_node(B, t, i, j, k);
-                update_node<S, true, !BND>(B, i, j, k, mode, mdu, mdv, mde);
+                update_node<S, true, !BND>(B, i, j, k, mode, Lout, mdu, mdv, mde);
             }
             if (mode == 2 && B.mon && (t & ~63u) < ns) {
                 const uint32_t main_slots = ((B.ni + TX - 1) / TX) * ((B.nj + TY - 1) / TY) * B.nk * (uint32_t)(TX * TY / 64);
@@ -731,7 +733,7 @@ __global__ void __launch_bounds__(TX *TY) k_update(const BlockDev *__restrict__ 
         node_tile(B, lt, TX, TY, i0, j0, k);
         const int i = i0 + (int)(threadIdx.x % TX), j = j0 + (int)(threadIdx.x / TX);
         if (i < B.ni && j < B.nj && !(BND && B.code && in_shell(B, i, j, k)))
-            update_node<S, false, !BND>(B, i, j, k, mode, mdu, mdv, mde);
+            update_node<S, false, !BND>(B, i, j, k, mode, Lout, mdu, mdv, mde);
         if (mode == 2 && B.mon) monitor_wave(B, lt * (TX * TY / 64) + threadIdx.x / 64, mdu, mdv, mde);
     };
     each_tile<LOOP>(all, tile);
@@ -979,14 +981,14 @@ void launch_node_b(const LaunchList &L, uint32_t cap, hipStream_t st, bool visc_
     const uint32_t shell_tiles = BND ? (L.shell_max + TX * TY - 1) / (TX * TY) : 0u;
     const uint32_t all = L.total[0] + L.nblk * shell_tiles;   // one workgroup per shell tile too
     const bool loop = cap && cap < all;
-    auto go = [&](auto kernel) {
+    auto go = [&](auto kernel, auto... out) {
         hipLaunchKernelGGL(kernel, dim3(loop ? cap : all), dim3(TX * TY), 0, st, L.blks, L.prefix[0], L.nblk, L.total[0], mode,
-                           shell_tiles);
+                           shell_tiles, out...);
     };
     if (visc_kernel && loop) go(k_visc<S, TX, TY, BND, true>);
     else if (visc_kernel) go(k_visc<S, TX, TY, BND, false>);
-    else if (loop) go(k_update<S, TX, TY, BND, true>);
-    else go(k_update<S, TX, TY, BND, false>);
+    else if (loop) go(k_update<S, TX, TY, BND, true>, L.Lout);
+    else go(k_update<S, TX, TY, BND, false>, L.Lout);
 }
 // lists without bounded blocks run the node kernels without the loc-code branches
 template <typename S, int V>
