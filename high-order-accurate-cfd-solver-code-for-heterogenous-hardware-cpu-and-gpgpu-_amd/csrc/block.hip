@@ -215,7 +215,7 @@ void bc_extent(const BlockDev &B, LaunchList &L)
             L.bc_face_d[d] = std::max(L.bc_face_d[d], f[d]);
             L.bc_face = std::max(L.bc_face, f[d]);
         }
-    if (B.off[1] && B.bc[2] == CFDX_BC_WALL_CUT) L.any_cut = true;
+    if (B.off[0]) L.bc_planes = std::max(L.bc_planes, (uint32_t)B.nk);
     L.shell_max = std::max(L.shell_max, cfdx::blk::shell_count(B));
 }
 
@@ -345,7 +345,7 @@ int upload_batch(cfdx_batch *q)
     q->L.tiles = q->tiles;
     q->L.bc_face = 0;
     for (int d = 0; d < 3; ++d) q->L.bc_face_d[d] = 0;
-    q->L.any_cut = false;
+    q->L.bc_planes = 0;
     q->L.shell_max = 0;
     for (size_t i = 0; i < nb; ++i) bc_extent(h[i], q->L);
     q->seen.resize(nb);

@@ -95,7 +95,7 @@ struct LaunchList {
     TileCfg tiles;
     uint32_t bc_face = 0;             // largest side face (owned nodes) of the bounded blocks; 0 if none
     uint32_t bc_face_d[3] = {};       // the same per direction (0: no block bounded in that direction)
-    bool any_cut = false;             // some block has a wake cut
+    uint32_t bc_planes = 0;           // largest nk of the blocks bounded along i
     uint32_t shell_max = 0;           // largest shell of the bounded blocks
     double *Lout = nullptr;           // mode 3 (a single block): the right-hand side, 5 x owned nodes
 };

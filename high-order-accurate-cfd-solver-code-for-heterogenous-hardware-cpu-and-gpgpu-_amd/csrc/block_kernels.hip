@@ -570,10 +570,14 @@ __global__ void __launch_bounds__(256, 4) k_flux(const BlockDev *__restrict__ bl
                   L2 = FACE_LDS<S, JA, JB> * (int)sizeof(S);
     __shared__ __align__(16) char lds[L0 > L1 ? (L0 > L2 ? L0 : L2) : (L1 > L2 ? L1 : L2)];
     constexpr uint32_t K = VISC ? 4 : 3;
-    const uint32_t main = 8 * K * slots, wg = blockIdx.x;
-    if (VISC && BND && wg >= main) {
-        visc_shell_tile<S>(blks, wg - main, mode, shell_tiles);
-        return;
+    uint32_t wg = blockIdx.x;
+    if (VISC && BND) {
+        // the shell tiles first (a multiple of 8 workgroups, so that the others keep their XCDs): their long
+        // chains would otherwise be the tail of the launch
+        const uint32_t shell = nblk * shell_tiles, first = (shell + 7) & ~7u;
+        if (wg < shell) visc_shell_tile<S>(blks, wg, mode, shell_tiles);
+        if (wg < first) return;
+        wg -= first;
     }
     const uint32_t x = wg & 7u, l = wg >> 3, kind = (l % (K * T.chunk)) / T.chunk + (4 - K), r = (l / (K * T.chunk)) * T.chunk + l % T.chunk;
     const uint32_t total = T.total[kind], q = total >> 3, rem = total & 7u;
@@ -623,10 +627,18 @@ __device__ __forceinline__ void update_node(const BlockDev &B, int i, int j, int
                 const uint32_t m3 = shifted(B, i, j, k, d, -3), p3 = shifted(B, i, j, k, d, 3);
                 const int LI = ld(B.code, g), LM2 = ld(B.code, m2), LM1 = ld(B.code, m1), LP1 = ld(B.code, p1),
                           LP2 = ld(B.code, p2);
+                // across a wake cut the row -m of column i is the row m of column ni - 1 - i, where eta runs the
+                // other way: its flux along j, negated
+                const bool cut = d == 1 && B.bc[2] == CFDX_BC_WALL_CUT && !(i >= B.cut_i0 && i <= B.cut_i1);
+                const auto below = [&](int o, uint32_t own) {
+                    return cut && j < o ? node_index(B, B.ni - 1 - i, o - j, k) : own;
+                };
+                const uint32_t x3 = below(3, m3), x2 = below(2, m2), x1 = below(1, m1);
+                const double s3 = cut && j < 3 ? -1.0 : 1.0, s2 = cut && j < 2 ? -1.0 : 1.0, s1 = cut && j < 1 ? -1.0 : 1.0;
 #pragma unroll
                 for (int c = 1; c < 5; ++c) {
                     const S *fv = (const S *)B.Fv[d][c - 1];
-                    const double f[7] = {(double)ld(fv, m3), (double)ld(fv, m2), (double)ld(fv, m1), (double)ld(fv, g),
+                    const double f[7] = {s3 * (double)ld(fv, x3), s2 * (double)ld(fv, x2), s1 * (double)ld(fv, x1), (double)ld(fv, g),
                                          (double)ld(fv, p1), (double)ld(fv, p2), (double)ld(fv, p3)};
                     L[c] += loc_derivative(f, LI, LM2, LM1, LP1, LP2, true);
                 }
@@ -705,12 +717,13 @@ __global__ void __launch_bounds__(TX *TY) k_update(const BlockDev *__restrict__ 
                                                    uint32_t nblk, uint32_t total, int mode, uint32_t shell_tiles,
                                                    double *Lout)
 {
-    const uint32_t all = total + (BND ? nblk * shell_tiles : 0u);
+    const uint32_t shell = BND ? nblk * shell_tiles : 0u, first = (shell + 7) & ~7u, all = first + total;
     auto tile = [&](uint32_t wg) {
         // residual monitor of the step (Solver.cpp:546-573): |du|, |dv|, |de| against the RK base
         double mdu = 0.0, mdv = 0.0, mde = 0.0;
-        if (BND && wg >= total) {
-            const uint32_t s = wg - total;
+        if (BND && wg < first) {   // the shell tiles first, as in k_flux
+            const uint32_t s = wg;
+            if (s >= shell) return;
             const BlockDev &B = blks[s / shell_tiles];
             const uint32_t t = (s % shell_tiles) * (TX * TY) + threadIdx.x;
             const uint32_t ns = shell_count(B);
@@ -726,7 +739,7 @@ __global__ void __launch_bounds__(TX *TY) k_update(const BlockDev *__restrict__ 
             }
             return;
         }
-        const uint32_t t = xcd_tile(wg, total);
+        const uint32_t t = xcd_tile(wg - first, total);
         const BlockDev &B = blks[find_block(prefix, nblk, t)];
         const uint32_t lt = t - B.tile0[0];
         int i0, j0, k;
@@ -861,27 +874,16 @@ __device__ __forceinline__ void copy_node(const BlockDev &B, uint32_t dst, uint3
     }
 }
 
-// The two sides of direction d (blockIdx.z = 0: low side, 1: high side), one thread per node of
-// a side's face and layer m (0: the boundary node, 1..3: the ghost layers). The nodes a side
+// One node of side hi (0: low, 1: high) of direction d: face node (a, bq) and layer m (0: the boundary
+// node, 1..3: the ghost layers). The nodes a side
 // writes are its boundary nodes and ghost layers; it reads the first owned layers in from its
 // side (a bounded direction has >= 7 nodes), so the two sides of a direction are independent and
 // the directions run one after the other (i, then j, then k: a node on two sides ends with the
 // later direction's value).
 template <typename S>
-__global__ void __launch_bounds__(256) k_bc(const BlockDev *__restrict__ blks, int d, int mode)
+__device__ __forceinline__ void bc_node(const BlockDev &B, int d, int hi, int a, int bq, int m, int mode)
 {
-    const BlockDev &B = blks[blockIdx.y];
-    if (!B.off[d]) return;
-    const int hi = (int)blockIdx.z, side = 2 * d + hi;
-    const int na = d == 0 ? B.nj : B.ni, nb = d == 2 ? B.nj : B.nk;
-    const uint32_t nf = (uint32_t)na * (uint32_t)nb;
-    const uint32_t t = blockIdx.x * blockDim.x + threadIdx.x;
-    if (t >= 4 * nf) return;
-    // i sides: the four layers of a face node are adjacent in memory, so they go to four adjacent
-    // threads; j and k sides: adjacent threads take adjacent i of one layer
-    const int m = d == 0 ? (int)(t & 3u) : (int)(t / nf);
-    const uint32_t r = d == 0 ? t >> 2 : t - (uint32_t)m * nf;
-    const int a = (int)(r % (uint32_t)na), bq = (int)(r / (uint32_t)na);
+    const int side = 2 * d + hi;
     const int n = d == 0 ? B.ni : d == 1 ? B.nj : B.nk;
     auto at = [&](int c) -> uint32_t {
         if (d == 0) return node_index(B, c, a, bq);
@@ -925,37 +927,65 @@ __global__ void __launch_bounds__(256) k_bc(const BlockDev *__restrict__ blks, i
     put_node<S>(B, at(c0 - in * m), w, mode, m > 0);
 }
 
-// viscous node fluxes of the ghost rows across a wake cut: the mirror node's, with the signs of
-// the i and j directions reversed (zeta and eta run the other way on the other side of the cut);
-// one thread per (i, layer m, k)
+// One direction's two sides (blockIdx.z), one thread per node of a side's face and layer.
 template <typename S>
-__global__ void __launch_bounds__(256) k_cut_viscous(const BlockDev *__restrict__ blks)
+__global__ void __launch_bounds__(256) k_bc(const BlockDev *__restrict__ blks, int d, int mode)
 {
     const BlockDev &B = blks[blockIdx.y];
-    if (!B.off[1] || B.bc[2] != CFDX_BC_WALL_CUT || !B.viscous) return;
-    const uint32_t nf = (uint32_t)B.ni * (uint32_t)B.nk;
+    if (!B.off[d]) return;
+    const int na = d == 0 ? B.nj : B.ni, nb = d == 2 ? B.nj : B.nk;
+    const uint32_t nf = (uint32_t)na * (uint32_t)nb;
     const uint32_t t = blockIdx.x * blockDim.x + threadIdx.x;
-    if (t >= 3 * nf) return;
-    const int m = 1 + (int)(t / nf);
-    const uint32_t r = t % nf;
-    const int i = (int)(r % (uint32_t)B.ni), k = (int)(r / (uint32_t)B.ni);
-    if (i >= B.cut_i0 && i <= B.cut_i1) return;
-    const uint32_t dst = node_index(B, i, -m, k), src = node_index(B, B.ni - 1 - i, m, k);
-    S v[3][4];
-#pragma unroll
-    for (int dd = 0; dd < 3; ++dd)
-#pragma unroll
-        for (int c = 0; c < 4; ++c) v[dd][c] = ld((const S *)B.Fv[dd][c], src);
-#pragma unroll
-    for (int dd = 0; dd < 3; ++dd)
-#pragma unroll
-        for (int c = 0; c < 4; ++c) st((S *)B.Fv[dd][c], dst, dd == 2 ? v[dd][c] : -v[dd][c]);
+    if (t >= 4 * nf) return;
+    // i sides: the four layers of a face node are adjacent in memory, so they go to four adjacent
+    // threads; j and k sides: adjacent threads take adjacent i of one layer
+    const int m = d == 0 ? (int)(t & 3u) : (int)(t / nf);
+    const uint32_t r = d == 0 ? t >> 2 : t - (uint32_t)m * nf;
+    bc_node<S>(B, d, (int)blockIdx.z, (int)(r % (uint32_t)na), (int)(r / (uint32_t)na), m, mode);
+}
+
+// The side conditions of the i and j directions of blocks bounded in either, in one launch: i first, then
+// j, as k_bc one after the other. Workgroups 0 .. planes - 1 take the two i sides of a k plane each and,
+// after them, the j sides of the four columns at either end, the only ones that read what the i sides
+// wrote or write what they read; the other workgroups take the j sides of the columns between. (Two
+// launches of 6-7 us each on a C-grid of any size of the served ladder.)
+constexpr int BC_IJ = 512, BC_END = 4;
+template <typename S>
+__global__ void __launch_bounds__(BC_IJ) k_bc_ij(const BlockDev *__restrict__ blks, uint32_t planes, int mode)
+{
+    const BlockDev &B = blks[blockIdx.y];
+    const int ni = B.ni, nj = B.nj, nk = B.nk;
+    if (blockIdx.x < planes) {
+        const int k = (int)blockIdx.x;
+        if (!B.off[0] || k >= nk) return;
+        // the four layers of a face node are adjacent in memory, so they go to four adjacent threads
+        for (int t = (int)threadIdx.x; t < 8 * nj; t += BC_IJ) bc_node<S>(B, 0, (t >> 2) >= nj, (t >> 2) % nj, k, t & 3, mode);
+        if (!B.off[1]) return;
+        __syncthreads();
+        const int cols = min(2 * BC_END, ni);
+        for (int t = (int)threadIdx.x; t < 8 * cols; t += BC_IJ) {
+            const int c = t % cols, r = t / cols;
+            bc_node<S>(B, 1, r >> 2, c < BC_END ? c : ni - cols + c, k, r & 3, mode);
+        }
+        return;
+    }
+    if (!B.off[1]) return;
+    const uint32_t first = B.off[0] ? BC_END : 0, cols = B.off[0] ? (uint32_t)max(ni - 2 * BC_END, 0) : (uint32_t)ni;
+    const uint32_t t = (blockIdx.x - planes) * BC_IJ + threadIdx.x;
+    if (t >= 8 * cols * (uint32_t)nk) return;
+    const uint32_t c = t % cols, r = t / cols;
+    bc_node<S>(B, 1, (int)((r / (uint32_t)nk) >> 2), (int)(first + c), (int)(r % (uint32_t)nk), (int)((r / (uint32_t)nk) & 3u), mode);
 }
 
 template <typename S>
 void launch_bc(const LaunchList &L, int mode, hipStream_t st)
 {
-    for (int d = 0; d < 3; ++d)
+    const bool ij = L.bc_face_d[0] && L.bc_face_d[1];
+    if (ij) {
+        const uint32_t js = (8 * L.bc_face_d[1] + BC_IJ - 1) / BC_IJ;
+        hipLaunchKernelGGL(k_bc_ij<S>, dim3(L.bc_planes + js, L.nblk), dim3(BC_IJ), 0, st, L.blks, L.bc_planes, mode);
+    }
+    for (int d = ij ? 2 : 0; d < 3; ++d)
         if (L.bc_face_d[d])
             hipLaunchKernelGGL(k_bc<S>, dim3((4 * L.bc_face_d[d] + 255) / 256, L.nblk, 2), dim3(256), 0, st, L.blks, d, mode);
 }
@@ -979,7 +1009,8 @@ void launch_node_b(const LaunchList &L, uint32_t cap, hipStream_t st, bool visc_
     constexpr int TX = NODE_TILES[V][0], TY = NODE_TILES[V][1];
     static_assert(TX * TY == 256, "node tiles have 256 threads");
     const uint32_t shell_tiles = BND ? (L.shell_max + TX * TY - 1) / (TX * TY) : 0u;
-    const uint32_t all = L.total[0] + L.nblk * shell_tiles;   // one workgroup per shell tile too
+    // one workgroup per shell tile too
+    const uint32_t shell = L.nblk * shell_tiles, all = L.total[0] + (visc_kernel ? shell : (shell + 7) & ~7u);
     const bool loop = cap && cap < all;
     auto go = [&](auto kernel, auto... out) {
         hipLaunchKernelGGL(kernel, dim3(loop ? cap : all), dim3(TX * TY), 0, st, L.blks, L.prefix[0], L.nblk, L.total[0], mode,
@@ -1046,7 +1077,7 @@ void launch_flux(const LaunchList &L, int mode, hipStream_t st, bool any_visc)
     T.chunk = std::min(FLUX_CHUNK, slots);
     slots = (slots + T.chunk - 1) / T.chunk * T.chunk;
     const uint32_t shell_tiles = L.bc_face && any_visc ? (L.shell_max + 255) / 256 : 0u;
-    const dim3 g(8 * (any_visc ? 4u : 3u) * slots + L.nblk * shell_tiles);
+    const dim3 g(8 * (any_visc ? 4u : 3u) * slots + ((L.nblk * shell_tiles + 7) & ~7u));
     auto go = [&](auto kernel) {
         hipLaunchKernelGGL(kernel, g, dim3(256), 0, st, L.blks, T, L.nblk, slots, mode, shell_tiles);
     };
@@ -1076,8 +1107,6 @@ void launch_stage(const LaunchList &L, int mode, hipStream_t st, bool any_visc, 
         }
         node_kernel<S>(L, L.grid_cap, vs, true, mode);
     }
-    if (any_visc && L.any_cut)
-        hipLaunchKernelGGL(k_cut_viscous<S>, dim3((3 * L.bc_face_d[1] + 255) / 256, L.nblk), dim3(256), 0, vs, L.blks);
     if (vs != st) (void)hipEventRecord(ov->join, vs);
     rec(1);
     if (!together) face_i<S>(L, st);
