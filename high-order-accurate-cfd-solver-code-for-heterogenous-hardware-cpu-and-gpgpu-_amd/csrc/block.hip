@@ -225,6 +225,7 @@ int upload_single(cfdx_block *b)
     if (b->uploaded == b->version) return CFDX_OK;
     BlockDev B = b->B;
     B.strip = (uint32_t)b->tiles.strip;
+    B.stream = cfdx::blk::streams_past_cache(cfdx::blk::stage_bytes(B), cfdx::blk::rows_stream(B));
     uint32_t pre[8];
     for (int kind = 0; kind < 4; ++kind) {
         B.tile0[kind] = 0;
@@ -244,6 +245,7 @@ LaunchList single_list(cfdx_block *b)
     L.blks = b->dB;
     L.nblk = 1;
     L.tiles = b->tiles;
+    L.stream = cfdx::blk::streams_past_cache(cfdx::blk::stage_bytes(b->B), cfdx::blk::rows_stream(b->B));
     bc_extent(b->B, L);
     for (int kind = 0; kind < 4; ++kind) {
         L.prefix[kind] = b->dprefix + 2 * kind;
@@ -321,8 +323,16 @@ int upload_batch(cfdx_batch *q)
     std::vector<uint32_t> pre(4 * (q->cap + 1), 0);
     uint32_t tot[4] = {0, 0, 0, 0};
     q->any_visc = false;
+    uint64_t bytes = 0;
+    bool rows = true;
+    for (const cfdx_block *b : q->blocks) {
+        bytes += cfdx::blk::stage_bytes(b->B);
+        rows = rows && cfdx::blk::rows_stream(b->B);
+    }
+    q->L.stream = cfdx::blk::streams_past_cache(bytes, rows);
     for (size_t i = 0; i < nb; ++i) {
         h[i] = q->blocks[i]->B;
+        h[i].stream = q->L.stream;
         h[i].strip = (uint32_t)q->tiles.strip;
         for (int kind = 0; kind < 4; ++kind) {
             h[i].tile0[kind] = tot[kind];
@@ -437,6 +447,7 @@ extern "C" int cfdx_block_create(cfdx_ctx *ctx, const cfdx_block_desc *desc, cfd
         p += (size_t)22 * n * sizeof(float);
     }
     B.strip = 0;
+    B.stream = 0;
     B.code = nullptr;
     if (desc->periodic != 7) {
         const std::vector<uint8_t> codes = loc_codes(desc);

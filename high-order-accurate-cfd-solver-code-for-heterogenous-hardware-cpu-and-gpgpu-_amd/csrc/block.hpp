@@ -46,6 +46,7 @@ struct BlockDev {
     int cut_i0, cut_i1;         // wall range of a CFDX_BC_WALL_CUT side
     double cos_aoa, sin_aoa;    // far-field flow direction
     uint32_t tile0[4];          // first global tile of this block: node tiles, face tiles x, y, z
+    uint32_t stream;            // the list's non-temporal switch, for the face sweeps
     uint32_t strip;             // node tiles: rows of tiles per strip walked plane by plane (0: whole planes)
     const double *det;          // det at the node
     const double *m[9];         // node metrics zeta_x .. xi_z
@@ -85,6 +86,29 @@ __host__ __device__ inline uint32_t shell_count(const BlockDev &B)
     return n;
 }
 
+// How the node kernels of a list access memory.
+enum : int {
+    LIST_PLAIN,     // periodic blocks
+    LIST_STREAM,    // periodic blocks, non-temporal accesses to what a kernel touches once
+    LIST_BOUNDED    // some block has a bounded direction: shell tiles beside the node tiles
+};
+
+// Bytes of a stored node that a stage reads and writes (FP64: 22 geometry arrays, U0, Us, P, Fv, FH; mixed:
+// the float geometry, det, U0, Us and the 32 float arrays).
+inline uint64_t stage_bytes(const BlockDev &B) { return (uint64_t)B.n * (B.geo32 ? 304 : 512); }
+
+// Whether a block's rows take non-temporal accesses well: whole 64-byte pieces. With others the hint
+// drops lines that the neighbouring rows still need (FP64 161x131x127 1.5 % slower, 255x200x160 2.5 %, mixed 4 and
+// 5 %; the C-grids, rows of ni + 6 nodes, 14 % at 128x64x16 to 1 % at 384x128x32).
+inline bool rows_stream(const BlockDev &B) { return !B.code && (uint64_t)B.pi * (B.geo32 ? 4 : 8) % 64 == 0; }
+
+// The size past which a list of blocks streams: below it a stage's arrays stay in the 256 MB last-level
+// cache (and the L2s) from one stage to the next, and the hint gives that up. FP64: 64^3 197 us a step
+// with the hint, 177 without; 80^3 (262 MB) 449 and 391; 96^3 (453 MB) 708 and 731; 256^3 12.88 and 13.09 ms.
+// Mixed: 64^3 125 and 112 us, 96^3 (269 MB) 400 and 369, 112^3 (427 MB) 622 and 643, 128^3 889 and 937.
+constexpr uint64_t STREAM_BYTES = (uint64_t)320 << 20;
+inline bool streams_past_cache(uint64_t bytes, bool rows) { return rows && bytes > STREAM_BYTES; }
+
 // One launch over a list of blocks.
 struct LaunchList {
     const BlockDev *blks = nullptr;   // device array
@@ -97,6 +121,7 @@ struct LaunchList {
     uint32_t bc_face_d[3] = {};       // the same per direction (0: no block bounded in that direction)
     uint32_t bc_planes = 0;           // largest nk of the blocks bounded along i
     uint32_t shell_max = 0;           // largest shell of the bounded blocks
+    bool stream = false;              // periodic blocks past the cache: non-temporal accesses
     double *Lout = nullptr;           // mode 3 (a single block): the right-hand side, 5 x owned nodes
 };
 

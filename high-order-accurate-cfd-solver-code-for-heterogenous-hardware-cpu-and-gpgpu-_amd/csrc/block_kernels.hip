@@ -41,9 +41,7 @@ __device__ __forceinline__ void st(T *base, uint32_t i, T v)
 
 // Streaming forms for data a kernel touches once (geometry read at its own node, outputs): the
 // non-temporal hint lets the L2 evict these lines first, keeping the stencil neighbours that
-// adjacent tiles read again. Used for periodic blocks only (measured at 128^3: the whole step
-// 5 % faster in FP64 and mixed, 64 cubes 4 %); on the bounded C-grid (384x128x32) the hint
-// costs 1 % in FP64 and 4 % mixed, so lists with bounded blocks keep plain accesses.
+// adjacent tiles read again. For the lists of blocks that streams_past_cache chooses.
 template <bool NT, typename T>
 __device__ __forceinline__ T ldx(const T *base, uint32_t i)
 {
@@ -335,9 +333,10 @@ template <int TX, int TY>
 constexpr int VISC_LDS = TY >= 4 ? 5 * (TY + 4) * (TX + 4) : 1;
 
 // Viscous node fluxes of the nodes of tile lt of block B; plane: VISC_LDS<TX, TY> doubles of LDS.
-template <typename S, int TX, int TY, bool BND>
+template <typename S, int TX, int TY, int K>
 __device__ __forceinline__ void visc_tile(const BlockDev &B, uint32_t lt, int mode, double *plane)
 {
+    constexpr bool BND = K == LIST_BOUNDED, NT = K == LIST_STREAM;
     constexpr int PC = TX + 4, PR = TY + 4;
     int i0, j0, k;
     node_tile(B, lt, TX, TY, i0, j0, k);
@@ -361,8 +360,8 @@ __device__ __forceinline__ void visc_tile(const BlockDev &B, uint32_t lt, int mo
     }
     if (i >= B.ni || j >= B.nj) return;
     if (BND && B.code && in_shell(B, i, j, k)) return;   // a shell tile's node
-    if constexpr (TY >= 4) visc_node<S, false, !BND, true>(B, i, j, k, mode, plane, tx, ty, PC, PR);
-    else visc_node<S, false, !BND>(B, i, j, k, mode);
+    if constexpr (TY >= 4) visc_node<S, false, NT, true>(B, i, j, k, mode, plane, tx, ty, PC, PR);
+    else visc_node<S, false, NT>(B, i, j, k, mode);
 }
 
 // Viscous node fluxes of 256 shell nodes: shell tile s of the list (block = s / shell_tiles).
@@ -380,11 +379,12 @@ __device__ __forceinline__ void visc_shell_tile(const BlockDev *__restrict__ blk
 // Node tiles of the list first (tile ids through the XCD remap), then, for lists with bounded
 // blocks, nblk x shell_tiles shell tiles of TX * TY shell nodes each (block = id / shell_tiles),
 // dispatched last in plain order so that they spread over the XCDs at the end of the launch.
-template <typename S, int TX, int TY, bool BND, bool LOOP>
-__global__ void __launch_bounds__(TX *TY, ((TY >= 4 && !(LOOP && BND)) || sizeof(S) == 4 ? 4 : 3))
+template <typename S, int TX, int TY, int K, bool LOOP>
+__global__ void __launch_bounds__(TX *TY, ((TY >= 4 && !(LOOP && K == LIST_BOUNDED)) || sizeof(S) == 4 ? 4 : 3))
     k_visc(const BlockDev *__restrict__ blks, const uint32_t *__restrict__ prefix, uint32_t nblk, uint32_t total, int mode,
            uint32_t shell_tiles)
 {
+    constexpr bool BND = K == LIST_BOUNDED;
     __shared__ double plane[VISC_LDS<TX, TY>];
     const uint32_t all = total + (BND ? nblk * shell_tiles : 0u);
     auto tile = [&](uint32_t wg) {
@@ -394,7 +394,7 @@ __global__ void __launch_bounds__(TX *TY, ((TY >= 4 && !(LOOP && BND)) || sizeof
         }
         const uint32_t t = xcd_tile(wg, total);
         const BlockDev &B = blks[find_block(prefix, nblk, t)];
-        if (B.viscous) visc_tile<S, TX, TY, BND>(B, t - B.tile0[0], mode, plane);
+        if (B.viscous) visc_tile<S, TX, TY, K>(B, t - B.tile0[0], mode, plane);
     };
     each_tile<LOOP>(all, tile);
 }
@@ -440,52 +440,52 @@ __device__ __forceinline__ void face_tile(const BlockDev &B, uint32_t lt, S *sq)
     S *const sf = sq + 5 * NP * TA;
     S *const sp = sq + 10 * NP * TA;   // STAGE_ROE only
     const int tid = threadIdx.x;
-            const int n_along = DIR == 0 ? B.ni : DIR == 1 ? B.nj : B.nk;
-            const int n_across = DIR == 0 ? B.nj : B.ni;
-            // face f of a line is the +1/2 face of along-coordinate f - sh (sh = 1 in a bounded
-            // direction: the first face lies between the first owned node and its ghost)
-            const int nfa = faces_along(B, DIR), sh = B.off[DIR] ? 1 : 0;
-            const uint32_t nta = (n_across + TA - 1) / TA, ntb = (nfa + TB - 1) / TB;
-            // tiles run along the lines' direction before the fixed coordinate, so that the next tile of
-            // an XCD re-reads the stencil halo planes of this one from its L2
-            int b0, a0, fixed;
+    const int n_along = DIR == 0 ? B.ni : DIR == 1 ? B.nj : B.nk;
+    const int n_across = DIR == 0 ? B.nj : B.ni;
+    // face f of a line is the +1/2 face of along-coordinate f - sh (sh = 1 in a bounded
+    // direction: the first face lies between the first owned node and its ghost)
+    const int nfa = faces_along(B, DIR), sh = B.off[DIR] ? 1 : 0;
+    const uint32_t nta = (n_across + TA - 1) / TA, ntb = (nfa + TB - 1) / TB;
+    // tiles run along the lines' direction before the fixed coordinate, so that the next tile of
+    // an XCD re-reads the stencil halo planes of this one from its L2
+    int b0, a0, fixed;
     if (DIR == 0) { b0 = (lt % ntb) * TB; a0 = ((lt / ntb) % nta) * TA; fixed = lt / (ntb * nta); }
     else { a0 = (lt % nta) * TA; b0 = ((lt / nta) % ntb) * TB; fixed = lt / (nta * ntb); }
     const S *P0 = (const S *)B.P[0], *P1 = (const S *)B.P[1], *P2 = (const S *)B.P[2], *P3 = (const S *)B.P[3], *P4 = (const S *)B.P[4];
 
-            __syncthreads();   // the previous tile's LDS fully consumed
-            for (int p = tid; p < NP * TA; p += 256) {
-                const int s = DIR == 0 ? p % NP : p / TA;
-                const int a = DIR == 0 ? p / NP : p % TA;
-                if (a0 + a >= n_across) continue;
-                // the points past the stencil of the tile's last computed face feed no face: skip them
-                // (a bounded line ends 3 ghost nodes past its last owned node; a periodic line shorter
-                // than the tile would wrap more than once)
-                if (s > nfa - b0 + 4) continue;
-                const int along = along_shift(B, DIR, b0 - sh, s - 2, n_along);
-                const uint32_t x = tile_node<DIR>(B, along, a0 + a, fixed);
-                const S rho = ld(P0, x), u = ld(P1, x), v = ld(P2, x), w = ld(P3, x), pr = ld(P4, x);
-                S q[5], f[5];
-                prim_to_q(rho, u, v, w, pr, q);
-                node_flux_e(rho, u, v, w, pr, q[4] + pr, ld(geo<S>(B, 1 + 3 * DIR), x), ld(geo<S>(B, 2 + 3 * DIR), x),
-                            ld(geo<S>(B, 3 + 3 * DIR), x), ld(geo<S>(B, 0), x), f);
-    #pragma unroll
-                for (int c = 0; c < 5; ++c) {
-                    sq[lds_at<DIR, TA, TB>(c, s, a)] = q[c];
-                    sf[lds_at<DIR, TA, TB>(c, s, a)] = f[c];
-                }
-                if constexpr (STAGE_ROE<S>) {
-                    sp[lds_at<DIR, TA, TB>(0, s, a)] = rho; sp[lds_at<DIR, TA, TB>(1, s, a)] = u;
-                    sp[lds_at<DIR, TA, TB>(2, s, a)] = v; sp[lds_at<DIR, TA, TB>(3, s, a)] = w;
-                    sp[lds_at<DIR, TA, TB>(4, s, a)] = enthalpy(rho, u, v, w, pr);
-                }
-            }
-            __syncthreads();
+    __syncthreads();   // the previous tile's LDS fully consumed
+    for (int p = tid; p < NP * TA; p += 256) {
+        const int s = DIR == 0 ? p % NP : p / TA;
+        const int a = DIR == 0 ? p / NP : p % TA;
+        if (a0 + a >= n_across) continue;
+        // the points past the stencil of the tile's last computed face feed no face: skip them
+        // (a bounded line ends 3 ghost nodes past its last owned node; a periodic line shorter
+        // than the tile would wrap more than once)
+        if (s > nfa - b0 + 4) continue;
+        const int along = along_shift(B, DIR, b0 - sh, s - 2, n_along);
+        const uint32_t x = tile_node<DIR>(B, along, a0 + a, fixed);
+        const S rho = ld(P0, x), u = ld(P1, x), v = ld(P2, x), w = ld(P3, x), pr = ld(P4, x);
+        S q[5], f[5];
+        prim_to_q(rho, u, v, w, pr, q);
+        node_flux_e(rho, u, v, w, pr, q[4] + pr, ld(geo<S>(B, 1 + 3 * DIR), x), ld(geo<S>(B, 2 + 3 * DIR), x),
+                    ld(geo<S>(B, 3 + 3 * DIR), x), ld(geo<S>(B, 0), x), f);
+#pragma unroll
+        for (int c = 0; c < 5; ++c) {
+            sq[lds_at<DIR, TA, TB>(c, s, a)] = q[c];
+            sf[lds_at<DIR, TA, TB>(c, s, a)] = f[c];
+        }
+        if constexpr (STAGE_ROE<S>) {
+            sp[lds_at<DIR, TA, TB>(0, s, a)] = rho; sp[lds_at<DIR, TA, TB>(1, s, a)] = u;
+            sp[lds_at<DIR, TA, TB>(2, s, a)] = v; sp[lds_at<DIR, TA, TB>(3, s, a)] = w;
+            sp[lds_at<DIR, TA, TB>(4, s, a)] = enthalpy(rho, u, v, w, pr);
+        }
+    }
+    __syncthreads();
 
-            const int b = DIR == 0 ? tid % TB : tid / TA;
-            const int a = DIR == 0 ? tid / TB : tid % TA;
-            if (b0 + b < nfa && a0 + a < n_across) {
-                auto q = [&](int m, int c) { return sq[lds_at<DIR, TA, TB>(c, b + m, a)]; };
+    const int b = DIR == 0 ? tid % TB : tid / TA;
+    const int a = DIR == 0 ? tid / TB : tid % TA;
+    if (b0 + b < nfa && a0 + a < n_across) {
+        auto q = [&](int m, int c) { return sq[lds_at<DIR, TA, TB>(c, b + m, a)]; };
         const uint32_t gl = tile_node<DIR>(B, b0 + b - sh, a0 + a, fixed);
         S roe[5], irho;
         if constexpr (STAGE_ROE<S>) {
@@ -502,38 +502,37 @@ __device__ __forceinline__ void face_tile(const BlockDev &B, uint32_t lt, S *sq)
             q_roe_inputs(qb, ib, ub, vb, wb, hb);
             irho = roe_average(qa[0], ua, va, wa, ha, qb[0], ub, vb, wb, hb, roe);
         }
-        // unit face normal and det_f |k| (the stored face arrays after geometry_finalize);
-                // streaming accesses on periodic blocks (B.code null)
-                S fg[4];
-                if (B.code) {
-    #pragma unroll
-                    for (int c = 0; c < 3; ++c) fg[c] = ld(geo<S>(B, 10 + 3 * DIR + c), gl);
-                    fg[3] = ld(geo<S>(B, 19 + DIR), gl);
-                } else {
-    #pragma unroll
-                    for (int c = 0; c < 3; ++c) fg[c] = ldx<true>(geo<S>(B, 10 + 3 * DIR + c), gl);
-                    fg[3] = ldx<true>(geo<S>(B, 19 + DIR), gl);
-                }
-                S llf[5];
-                face_llf(q, roe, irho, fg[0], fg[1], fg[2], fg[3], S(B.eps), llf);
-                S fh[5];
-    #pragma unroll
-                for (int c = 0; c < 5; ++c)
-                    fh[c] = S(llf[c] + midpoint_correction(sf[lds_at<DIR, TA, TB>(c, b, a)], sf[lds_at<DIR, TA, TB>(c, b + 1, a)],
-                                                           sf[lds_at<DIR, TA, TB>(c, b + 2, a)], sf[lds_at<DIR, TA, TB>(c, b + 3, a)],
-                                                           sf[lds_at<DIR, TA, TB>(c, b + 4, a)], sf[lds_at<DIR, TA, TB>(c, b + 5, a)]));
-                if (B.code) {
-    #pragma unroll
-                    for (int c = 0; c < 5; ++c) st((S *)B.FH[DIR][c], gl, fh[c]);
-                } else {
-    #pragma unroll
-                    for (int c = 0; c < 5; ++c) stx<true>((S *)B.FH[DIR][c], gl, fh[c]);
-                }
-            }
+        // unit face normal and det_f |k| (the stored face arrays after geometry_finalize)
+        S fg[4];
+        if (!B.stream) {
+#pragma unroll
+            for (int c = 0; c < 3; ++c) fg[c] = ld(geo<S>(B, 10 + 3 * DIR + c), gl);
+            fg[3] = ld(geo<S>(B, 19 + DIR), gl);
+        } else {
+#pragma unroll
+            for (int c = 0; c < 3; ++c) fg[c] = ldx<true>(geo<S>(B, 10 + 3 * DIR + c), gl);
+            fg[3] = ldx<true>(geo<S>(B, 19 + DIR), gl);
+        }
+        S llf[5];
+        face_llf(q, roe, irho, fg[0], fg[1], fg[2], fg[3], S(B.eps), llf);
+        S fh[5];
+#pragma unroll
+        for (int c = 0; c < 5; ++c)
+            fh[c] = S(llf[c] + midpoint_correction(sf[lds_at<DIR, TA, TB>(c, b, a)], sf[lds_at<DIR, TA, TB>(c, b + 1, a)],
+                                                   sf[lds_at<DIR, TA, TB>(c, b + 2, a)], sf[lds_at<DIR, TA, TB>(c, b + 3, a)],
+                                                   sf[lds_at<DIR, TA, TB>(c, b + 4, a)], sf[lds_at<DIR, TA, TB>(c, b + 5, a)]));
+        if (!B.stream) {
+#pragma unroll
+            for (int c = 0; c < 5; ++c) st((S *)B.FH[DIR][c], gl, fh[c]);
+        } else {
+#pragma unroll
+            for (int c = 0; c < 5; ++c) stx<true>((S *)B.FH[DIR][c], gl, fh[c]);
+        }
+    }
 }
 
 template <typename S, int DIR, int TA, int TB, bool LOOP>
-__global__ void __launch_bounds__(256, 4) k_face(const BlockDev *__restrict__ blks, const uint32_t *__restrict__ prefix,
+__global__ void __launch_bounds__(256, (TA == 64 ? 3 : 4)) k_face(const BlockDev *__restrict__ blks, const uint32_t *__restrict__ prefix,
                                               uint32_t nblk, uint32_t total)
 {
     __shared__ S lds[FACE_LDS<S, TA, TB>];
@@ -560,7 +559,7 @@ struct FluxTotals {
     uint32_t chunk;      // tiles of a kind that an XCD takes at a time
 };
 
-template <typename S, bool VISC, bool BND>
+template <typename S, bool VISC, int K>
 __global__ void __launch_bounds__(256, 4) k_flux(const BlockDev *__restrict__ blks, FluxTotals T, uint32_t nblk, uint32_t slots,
                                                  int mode, uint32_t shell_tiles)
 {
@@ -569,7 +568,8 @@ __global__ void __launch_bounds__(256, 4) k_flux(const BlockDev *__restrict__ bl
     constexpr int L0 = VISC ? VISC_LDS<TX, TY> * (int)sizeof(double) : 0, L1 = FACE_LDS<S, IA, IB> * (int)sizeof(S),
                   L2 = FACE_LDS<S, JA, JB> * (int)sizeof(S);
     __shared__ __align__(16) char lds[L0 > L1 ? (L0 > L2 ? L0 : L2) : (L1 > L2 ? L1 : L2)];
-    constexpr uint32_t K = VISC ? 4 : 3;
+    constexpr bool BND = K == LIST_BOUNDED;
+    constexpr uint32_t KINDS = VISC ? 4 : 3;
     uint32_t wg = blockIdx.x;
     if (VISC && BND) {
         // the shell tiles first (a multiple of 8 workgroups, so that the others keep their XCDs): their long
@@ -579,14 +579,15 @@ __global__ void __launch_bounds__(256, 4) k_flux(const BlockDev *__restrict__ bl
         if (wg < first) return;
         wg -= first;
     }
-    const uint32_t x = wg & 7u, l = wg >> 3, kind = (l % (K * T.chunk)) / T.chunk + (4 - K), r = (l / (K * T.chunk)) * T.chunk + l % T.chunk;
+    const uint32_t x = wg & 7u, l = wg >> 3, kind = (l % (KINDS * T.chunk)) / T.chunk + (4 - KINDS),
+                   r = (l / (KINDS * T.chunk)) * T.chunk + l % T.chunk;
     const uint32_t total = T.total[kind], q = total >> 3, rem = total & 7u;
     if (r >= q + (x < rem ? 1u : 0u)) return;
     const uint32_t t = x * q + (x < rem ? x : rem) + r;
     const BlockDev &B = blks[find_block(T.prefix[kind], nblk, t)];
     const uint32_t lt = t - B.tile0[kind];
     if (kind == 0) {
-        if (B.viscous) visc_tile<S, TX, TY, BND>(B, lt, mode, (double *)lds);
+        if (B.viscous) visc_tile<S, TX, TY, K>(B, lt, mode, (double *)lds);
     } else if (kind == 1) {
         face_tile<S, 0, IA, IB>(B, lt, (S *)lds);
     } else if (kind == 2) {
@@ -712,11 +713,12 @@ __device__ __forceinline__ void monitor_wave(const BlockDev &B, uint32_t slot, d
 
 // tiles as in k_visc; the shell tiles' monitor slots follow the block's node tiles' (tiles x
 // waves per tile), one per wave of 64 shell nodes
-template <typename S, int TX, int TY, bool BND, bool LOOP>
+template <typename S, int TX, int TY, int K, bool LOOP>
 __global__ void __launch_bounds__(TX *TY) k_update(const BlockDev *__restrict__ blks, const uint32_t *__restrict__ prefix,
                                                    uint32_t nblk, uint32_t total, int mode, uint32_t shell_tiles,
                                                    double *Lout)
 {
+    constexpr bool BND = K == LIST_BOUNDED, NT = K == LIST_STREAM;
     const uint32_t shell = BND ? nblk * shell_tiles : 0u, first = (shell + 7) & ~7u, all = first + total;
     auto tile = [&](uint32_t wg) {
         // residual monitor of the step (Solver.cpp:546-573): |du|, |dv|, |de| against the RK base
@@ -731,7 +733,7 @@ __global__ void __launch_bounds__(TX *TY) k_update(const BlockDev *__restrict__ 
             if (t < ns) {
                 int i, j, k;
                 shell_node(B, t, i, j, k);
-                update_node<S, true, !BND>(B, i, j, k, mode, Lout, mdu, mdv, mde);
+                update_node<S, true, false>(B, i, j, k, mode, Lout, mdu, mdv, mde);
             }
             if (mode == 2 && B.mon && (t & ~63u) < ns) {
                 const uint32_t main_slots = ((B.ni + TX - 1) / TX) * ((B.nj + TY - 1) / TY) * B.nk * (uint32_t)(TX * TY / 64);
@@ -746,7 +748,7 @@ __global__ void __launch_bounds__(TX *TY) k_update(const BlockDev *__restrict__ 
         node_tile(B, lt, TX, TY, i0, j0, k);
         const int i = i0 + (int)(threadIdx.x % TX), j = j0 + (int)(threadIdx.x / TX);
         if (i < B.ni && j < B.nj && !(BND && B.code && in_shell(B, i, j, k)))
-            update_node<S, false, !BND>(B, i, j, k, mode, Lout, mdu, mdv, mde);
+            update_node<S, false, NT>(B, i, j, k, mode, Lout, mdu, mdv, mde);
         if (mode == 2 && B.mon) monitor_wave(B, lt * (TX * TY / 64) + threadIdx.x / 64, mdu, mdv, mde);
     };
     each_tile<LOOP>(all, tile);
@@ -1003,12 +1005,12 @@ void launch_face(const LaunchList &L, hipStream_t st)
         hipLaunchKernelGGL((k_face<S, DIR, TA, TB, false>), dim3(n), dim3(256), 0, st, L.blks, L.prefix[1 + DIR], L.nblk, n);
 }
 // cap: workgroups of the launch (0: one per tile)
-template <typename S, int V, bool BND>
-void launch_node_b(const LaunchList &L, uint32_t cap, hipStream_t st, bool visc_kernel, int mode)
+template <typename S, int V, int K>
+void launch_node_k(const LaunchList &L, uint32_t cap, hipStream_t st, bool visc_kernel, int mode)
 {
     constexpr int TX = NODE_TILES[V][0], TY = NODE_TILES[V][1];
     static_assert(TX * TY == 256, "node tiles have 256 threads");
-    const uint32_t shell_tiles = BND ? (L.shell_max + TX * TY - 1) / (TX * TY) : 0u;
+    const uint32_t shell_tiles = K == LIST_BOUNDED ? (L.shell_max + TX * TY - 1) / (TX * TY) : 0u;
     // one workgroup per shell tile too
     const uint32_t shell = L.nblk * shell_tiles, all = L.total[0] + (visc_kernel ? shell : (shell + 7) & ~7u);
     const bool loop = cap && cap < all;
@@ -1016,17 +1018,18 @@ void launch_node_b(const LaunchList &L, uint32_t cap, hipStream_t st, bool visc_
         hipLaunchKernelGGL(kernel, dim3(loop ? cap : all), dim3(TX * TY), 0, st, L.blks, L.prefix[0], L.nblk, L.total[0], mode,
                            shell_tiles, out...);
     };
-    if (visc_kernel && loop) go(k_visc<S, TX, TY, BND, true>);
-    else if (visc_kernel) go(k_visc<S, TX, TY, BND, false>);
-    else if (loop) go(k_update<S, TX, TY, BND, true>, L.Lout);
-    else go(k_update<S, TX, TY, BND, false>, L.Lout);
+    if (visc_kernel && loop) go(k_visc<S, TX, TY, K, true>);
+    else if (visc_kernel) go(k_visc<S, TX, TY, K, false>);
+    else if (loop) go(k_update<S, TX, TY, K, true>, L.Lout);
+    else go(k_update<S, TX, TY, K, false>, L.Lout);
 }
 // lists without bounded blocks run the node kernels without the loc-code branches
 template <typename S, int V>
 void launch_node(const LaunchList &L, uint32_t cap, hipStream_t st, bool visc_kernel, int mode)
 {
-    if (L.bc_face) launch_node_b<S, V, true>(L, cap, st, visc_kernel, mode);
-    else launch_node_b<S, V, false>(L, cap, st, visc_kernel, mode);
+    if (L.bc_face) launch_node_k<S, V, LIST_BOUNDED>(L, cap, st, visc_kernel, mode);
+    else if (L.stream) launch_node_k<S, V, LIST_STREAM>(L, cap, st, visc_kernel, mode);
+    else launch_node_k<S, V, LIST_PLAIN>(L, cap, st, visc_kernel, mode);
 }
 
 template <typename S>
@@ -1081,9 +1084,10 @@ void launch_flux(const LaunchList &L, int mode, hipStream_t st, bool any_visc)
     auto go = [&](auto kernel) {
         hipLaunchKernelGGL(kernel, g, dim3(256), 0, st, L.blks, T, L.nblk, slots, mode, shell_tiles);
     };
-    if (!any_visc) go(k_flux<S, false, false>);
-    else if (L.bc_face) go(k_flux<S, true, true>);
-    else go(k_flux<S, true, false>);
+    if (!any_visc) go(k_flux<S, false, LIST_PLAIN>);   // the sweeps alone take the blocks' own switch
+    else if (L.bc_face) go(k_flux<S, true, LIST_BOUNDED>);
+    else if (L.stream) go(k_flux<S, true, LIST_STREAM>);
+    else go(k_flux<S, true, LIST_PLAIN>);
 }
 
 template <typename S>

@@ -85,3 +85,26 @@ def test_one_launch_over_a_mixed_list(ctx, precision):
         return ([periodic(ctx, s, precision, p) for s, p in (((5, 4, 3), visc), ((40, 21, 9), inv), ((66, 10, 7), visc))]
                 + [bounded(ctx, n, precision) for n in CASES])
     same(both(ctx, make, 2))
+
+
+@pytest.mark.parametrize("precision", [cfdx.FP64, cfdx.MIXED], ids=["fp64", "mixed"])
+def test_streaming_accesses_give_the_same_bits(ctx, precision):
+    """A block past the last-level cache with rows of whole 64-byte pieces steps with non-temporal
+    accesses; in a list with a block whose rows are not, with plain ones: a hint, so the same bits."""
+    prm = cfdx.default_params(mach=0.3, reyl=900.0)
+    shape = (112, 112, 112)
+    alone = periodic(ctx, shape, precision, prm)
+    alone.step(2, 0.3, 0.02 * 2 * math.pi / 112, prm)
+    want = alone.get_flow()
+    alone.close()
+    b, odd = periodic(ctx, shape, precision, prm), periodic(ctx, (7, 5, 9), precision, prm)
+    q = cfdx.Batch(precision, ctx)
+    q.add(b)
+    q.add(odd)
+    q.step(2, False)
+    got = b.get_flow()
+    q.close()
+    for x in (b, odd):
+        x.close()
+    for f in FIELDS:
+        assert np.array_equal(got[f], want[f]), f
