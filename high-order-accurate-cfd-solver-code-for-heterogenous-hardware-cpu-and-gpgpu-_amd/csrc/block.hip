@@ -590,11 +590,8 @@ extern "C" int cfdx_block_get_flow(cfdx_block *b, cfdx_flow *flow)
     // from a 16-byte aligned start
     cfdx_flow *tmp = (cfdx_flow *)(((uintptr_t)b->B.Fv[0][0] + 15) & ~(uintptr_t)15);
     cfdx::blk::flow_out(b->B, b->desc.precision, b->ctx->stream, tmp, b->last_mach);
-    hipError_t e = hipGetLastError();
-    if (e == hipSuccess) e = hipMemcpyAsync(flow, tmp, (size_t)n * sizeof(cfdx_flow), hipMemcpyDeviceToHost, b->ctx->stream);
-    if (e == hipSuccess) e = hipStreamSynchronize(b->ctx->stream);
-    if (e != hipSuccess) return cfdx::hip_fail(e, "get_flow");
-    return CFDX_OK;
+    CFDX_TRY(cfdx::check_launch("get_flow"));
+    return cfdx::copy_to_host(b->ctx, flow, tmp, (size_t)n * sizeof(cfdx_flow), "get_flow");
 }
 
 extern "C" int cfdx_block_init_case(cfdx_block *b, const cfdx_case_desc *c)
@@ -705,11 +702,7 @@ extern "C" int cfdx_block_rhs(cfdx_block *b, const cfdx_params *params, double *
     configure(b, b->last_mach, b->B.del_t, params);
     int rc = upload_single(b);
     if (rc == CFDX_OK) rc = run_stage(b, 3, Ld);
-    if (rc == CFDX_OK) {
-        hipError_t e = hipMemcpyAsync(L_host, Ld, bytes, hipMemcpyDeviceToHost, b->ctx->stream);
-        if (e == hipSuccess) e = hipStreamSynchronize(b->ctx->stream);
-        if (e != hipSuccess) rc = cfdx::hip_fail(e, "block_rhs copy");
-    }
+    if (rc == CFDX_OK) rc = cfdx::copy_to_host(b->ctx, L_host, Ld, bytes, "block_rhs copy");
     (void)hipFree(Ld);
     return rc;
 }

@@ -92,6 +92,7 @@ extern "C" int cfdx_pool_trim(cfdx_ctx *ctx)
 {
     CFDX_TRY(cfdx::enter(ctx));
     cfdx::pool_trim(ctx->device);
+    cfdx::staging_trim();
     return CFDX_OK;
 }
 
@@ -260,9 +261,7 @@ extern "C" int cfdx_copy_to_host(cfdx_ctx *ctx, void *dst, const void *src, size
     CFDX_TRY(cfdx::enter(ctx));
     if ((!dst || !src) && bytes) return cfdx::fail(CFDX_E_INVALID, "copy_to_host: null pointer");
     if (!bytes) return CFDX_OK;
-    CFDX_HIP(hipMemcpyAsync(dst, src, bytes, hipMemcpyDeviceToHost, ctx->stream), "hipMemcpyAsync D2H");
-    CFDX_HIP(hipStreamSynchronize(ctx->stream), "hipStreamSynchronize");
-    return CFDX_OK;
+    return cfdx::copy_to_host(ctx, dst, src, bytes, "copy_to_host");
 }
 
 extern "C" int cfdx_event_record(cfdx_ctx *ctx, int slot)

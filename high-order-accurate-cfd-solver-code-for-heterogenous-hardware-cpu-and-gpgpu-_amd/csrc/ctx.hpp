@@ -35,6 +35,11 @@ void *pool_take(int device, size_t bytes, size_t *got);
 void pool_give(int device, void *ptr, size_t bytes);
 void pool_trim(int device);
 size_t pool_cached(int device);
+
+// bytes of device memory to the host, after the work queued on the context's stream; returns when
+// they are there. Large copies go through pinned memory (host_copy.cpp).
+int copy_to_host(cfdx_ctx *ctx, void *dst, const void *src, size_t bytes, const char *what);
+void staging_trim();
 }  // namespace cfdx
 
 namespace cfdx {
