@@ -72,18 +72,40 @@ struct BlockDev {
 // boundary node and the interior, which select the central form.
 constexpr uint32_t SHELL = 2;
 
-// Nodes of the shell of a bounded block (within SHELL nodes of a side along a bounded direction;
-// the node kernels leave them to the shell kernels); 0 for a periodic block.
-__host__ __device__ inline uint32_t shell_count(const BlockDev &B)
+// The shell of a bounded block (the nodes within SHELL of a side along a bounded direction; the tiled node
+// kernels leave them to shell tiles) in two parts: the k planes and j rows, along which i runs, and the i
+// columns left; 0 for a periodic block.
+__host__ __device__ inline uint32_t shell_rows(const BlockDev &B)
 {
     if (!B.code) return 0;
-    const uint32_t ni = B.ni, nj = B.nj, nk = B.nk;
-    const uint32_t kb = B.off[2] ? SHELL : 0u, jb = B.off[1] ? SHELL : 0u;
-    uint32_t n = 0;
-    if (B.off[2]) n += 2 * SHELL * ni * nj;
-    if (B.off[1]) n += 2 * SHELL * ni * (nk - 2 * kb);
-    if (B.off[0]) n += 2 * SHELL * (nj - 2 * jb) * (nk - 2 * kb);
-    return n;
+    const uint32_t ni = B.ni, nj = B.nj, nk = B.nk, kb = B.off[2] ? SHELL : 0u;
+    return (B.off[2] ? 2 * SHELL * ni * nj : 0u) + (B.off[1] ? 2 * SHELL * ni * (nk - 2 * kb) : 0u);
+}
+__host__ __device__ inline uint32_t shell_columns(const BlockDev &B)
+{
+    if (!B.code || !B.off[0]) return 0;
+    return 2 * SHELL * ((uint32_t)B.nj - (B.off[1] ? 2 * SHELL : 0u)) * ((uint32_t)B.nk - (B.off[2] ? 2 * SHELL : 0u));
+}
+
+// Shell tiles: 256 nodes of the rows, 64 or 256 of the columns. A column node's neighbours share no cache line
+// with the next node's, so a wave's loads take 32 lines each and few columns are bound by the address rate of
+// the few CUs they are on: up to COLUMNS_SPREAD nodes they go over four times the CUs. C-grids, FP64 and mixed, us
+// a step with 256 and with 64: 128x64x16 (3840 column nodes) 176 and 136, 153 and 113; 192x96x24 (8832) 371 and 269,
+// 369 and 263; 256x128x32 (15872) 915 and 572, 921 and 579.
+constexpr uint32_t SHELL_TILE = 256, COLUMNS_SPREAD = 12288;
+__host__ __device__ inline uint32_t shell_column_tile(const BlockDev &B) { return shell_columns(B) <= COLUMNS_SPREAD ? 64u : 256u; }
+__host__ __device__ inline uint32_t shell_row_tiles(const BlockDev &B) { return (shell_rows(B) + SHELL_TILE - 1) / SHELL_TILE; }
+__host__ __device__ inline uint32_t shell_tile_count(const BlockDev &B)
+{
+    const uint32_t c = shell_column_tile(B);
+    return shell_row_tiles(B) + (shell_columns(B) + c - 1) / c;
+}
+// The wave of the residual monitor's slots that wave w of shell tile s has: four a row tile, then those of the
+// column tiles.
+__host__ __device__ inline uint32_t shell_wave(const BlockDev &B, uint32_t s, uint32_t w)
+{
+    const uint32_t rows = shell_row_tiles(B);
+    return s < rows ? 4 * s + w : 4 * rows + (s - rows) * (shell_column_tile(B) / 64) + w;
 }
 
 // How the node kernels of a list access memory.
@@ -120,7 +142,7 @@ struct LaunchList {
     uint32_t bc_face = 0;             // largest side face (owned nodes) of the bounded blocks; 0 if none
     uint32_t bc_face_d[3] = {};       // the same per direction (0: no block bounded in that direction)
     uint32_t bc_planes = 0;           // largest nk of the blocks bounded along i
-    uint32_t shell_max = 0;           // largest shell of the bounded blocks
+    uint32_t shell_tiles = 0;         // most shell tiles of a bounded block
     bool stream = false;              // periodic blocks past the cache: non-temporal accesses
     double *Lout = nullptr;           // mode 3 (a single block): the right-hand side, 5 x owned nodes
 };
@@ -137,6 +159,9 @@ struct Overlap {
 };
 void stage(const LaunchList &L, int precision, int mode, hipStream_t st, bool any_visc, hipEvent_t *ev,
            const Overlap *ov = nullptr);
+// whether stage() puts the viscous kernel on the second stream: other tile shapes than the defaults or a
+// capped grid, with the overlap on
+bool stage_forks(const LaunchList &L, const Overlap *ov);
 // the float copies of the geometry of a mixed block (after every write of its double geometry)
 // after every geometry write: face arrays to unit normal and det_f |k|, then the float copy
 void geometry_finalize(const BlockDev &B, hipStream_t st);

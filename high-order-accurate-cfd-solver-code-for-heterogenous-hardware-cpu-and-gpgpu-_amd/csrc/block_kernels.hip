@@ -101,16 +101,46 @@ __device__ __host__ __forceinline__ int faces_along(const BlockDev &B, int d)
     return B.off[d] ? n + 1 : n;
 }
 
-// The loc-selected forms of a bounded block reduce to the central ones unless the node is a side
-// node (code 1) or a side node or ghost (code 100) lies within 2 nodes of it along d; elsewhere
-// the kernels take the central forms directly, so a wave away from the sides keeps the short path.
-__device__ __forceinline__ bool near_side(const BlockDev &B, int i, int j, int k, int d)
+// The form that the loc codes select for a derivative along d at a node (loc_derivative, Viscous.cl:285-435 and
+// with weno_form Weno.cl:2732-2856): four points at offsets o and their weights, found without a branch, so that
+// a shell node reads its codes in one memory round trip and its points in another (a branch per form, with
+// seven points each, made the shell tiles the longest of a small launch: C-grid 128x64x16 update 26 us a
+// stage). No match: zero weights on the node itself.
+struct LocForm {
+    int o[4];
+    double w[4];
+};
+__device__ __forceinline__ LocForm loc_form(int LI, int LM2, int LM1, int LP1, int LP2, bool weno_form)
 {
-    const int c[3] = {i, j, k}, n[3] = {B.ni, B.nj, B.nk};
-    bool s = false;
+    const bool side = LI > 0 && LI <= 52, in = LI == 0;
+    const bool hi = side && LP1 == 100, lo = side && LM1 == 100;
+    const bool by_hi = in && LP1 > 0 && LP1 <= 52 && LP2 == 100;
+    const bool by_lo = in && LM1 > 0 && (!weno_form || LM1 <= 52) && LM2 == 100;
+    const bool mid = LM2 != 100 && LM1 != 100 && LP2 != 100 && LP1 != 100 && (in || (!weno_form && LI > 0));
+    LocForm f = {{0, 0, 0, 0}, {0.0, 0.0, 0.0, 0.0}};
+    auto take = [&](bool c, int o0, int o1, int o2, int o3, double w0, double w1, double w2, double w3) {
+        f.o[0] = c ? o0 : f.o[0]; f.o[1] = c ? o1 : f.o[1]; f.o[2] = c ? o2 : f.o[2]; f.o[3] = c ? o3 : f.o[3];
+        f.w[0] = c ? w0 : f.w[0]; f.w[1] = c ? w1 : f.w[1]; f.w[2] = c ? w2 : f.w[2]; f.w[3] = c ? w3 : f.w[3];
+    };
+    // in the reference's order, a later match over an earlier one
+    take(hi, 0, -1, -2, -3, 11.0 / 6.0, -3.0, 1.5, -1.0 / 3.0);
+    take(lo, 0, 1, 2, 3, -11.0 / 6.0, 3.0, -1.5, 1.0 / 3.0);
+    take(by_hi, 1, 0, -1, -2, 1.0 / 3.0, 0.5, -1.0, 1.0 / 6.0);
+    take(by_lo, -1, 0, 1, 2, -1.0 / 3.0, -0.5, 1.0, -1.0 / 6.0);
+    take(mid, 1, -1, 2, -2, 2.0 / 3.0, -2.0 / 3.0, -1.0 / 12.0, 1.0 / 12.0);
+    return f;
+}
+// the forms of a node along the three directions
+__device__ __forceinline__ void loc_forms(const BlockDev &B, int i, int j, int k, bool weno_form, LocForm (&f)[3])
+{
+    const int LI = ld(B.code, node_index(B, i, j, k));
+    int c[3][4];
 #pragma unroll
-    for (int q = 0; q < 3; ++q) s |= B.off[q] && (c[q] == 0 || c[q] == n[q] - 1);
-    return s || (B.off[d] && (c[d] < (int)SHELL || c[d] > n[d] - 1 - (int)SHELL));
+    for (int d = 0; d < 3; ++d)
+#pragma unroll
+        for (int q = 0; q < 4; ++q) c[d][q] = ld(B.code, shifted(B, i, j, k, d, q < 2 ? q - 2 : q - 1));
+#pragma unroll
+    for (int d = 0; d < 3; ++d) f[d] = loc_form(LI, c[d][0], c[d][1], c[d][2], c[d][3], weno_form);
 }
 
 // The shell of a bounded block: the nodes within SHELL of a side along a bounded direction (the
@@ -127,34 +157,33 @@ __device__ __forceinline__ bool in_shell(const BlockDev &B, int i, int j, int k)
     return s;
 }
 
-__device__ __forceinline__ void shell_node(const BlockDev &B, uint32_t t, int &i, int &j, int &k)
+// Thread's node of shell tile s of the block, if it has one.
+__device__ __forceinline__ bool shell_node(const BlockDev &B, uint32_t s, int &i, int &j, int &k)
 {
-    const uint32_t ni = B.ni, nj = B.nj, nk = B.nk;
+    const uint32_t ni = B.ni, nj = B.nj, nk = B.nk, rows = shell_row_tiles(B), tid = threadIdx.x;
     const uint32_t kb = B.off[2] ? SHELL : 0u, jb = B.off[1] ? SHELL : 0u, w = 2 * SHELL;
     auto layer = [](uint32_t m, uint32_t n) { return (int)(m < SHELL ? m : n - 2 * SHELL + m); };
-    if (B.off[2]) {
-        const uint32_t part = w * ni * nj;
-        if (t < part) {
-            i = (int)(t % ni);
+    if (s < rows) {
+        uint32_t t = s * SHELL_TILE + tid;
+        if (t >= shell_rows(B)) return false;
+        const uint32_t planes = B.off[2] ? w * ni * nj : 0u;
+        i = (int)(t % ni);
+        if (t < planes) {
             j = (int)((t / ni) % nj);
             k = layer(t / (ni * nj), nk);
-            return;
-        }
-        t -= part;
-    }
-    if (B.off[1]) {
-        const uint32_t part = w * ni * (nk - 2 * kb);
-        if (t < part) {
-            i = (int)(t % ni);
+        } else {
+            t -= planes;   // a multiple of ni
             j = layer((t / ni) % w, nj);
             k = (int)(kb + t / (w * ni));
-            return;
         }
-        t -= part;
+        return true;
     }
+    const uint32_t c = shell_column_tile(B), t = (s - rows) * c + tid;
+    if (tid >= c || t >= shell_columns(B)) return false;
     i = layer(t % w, ni);
     j = (int)(jb + (t / w) % (nj - 2 * jb));
     k = (int)(kb + t / (w * (nj - 2 * jb)));
+    return true;
 }
 
 // Workgroups are dispatched round-robin over the 8 XCDs (workgroup b runs on XCD b % 8), each
@@ -256,30 +285,24 @@ __device__ __forceinline__ void visc_node(const BlockDev &B, int i, int j, int k
         return r;
     };
     if constexpr (LOC) {
+        LocForm form[3];
+        loc_forms(B, i, j, k, false, form);
 #pragma unroll
         for (int d = 0; d < 3; ++d) {
-            const uint32_t m2 = shifted(B, i, j, k, d, -2), m1 = shifted(B, i, j, k, d, -1);
-            const uint32_t p1 = shifted(B, i, j, k, d, 1), p2 = shifted(B, i, j, k, d, 2);
-            const bool near = near_side(B, i, j, k, d);
-            // bounded block: the loc-selected one-sided forms of Viscous.cl:285-435 near the sides
-            const uint32_t m3 = near ? shifted(B, i, j, k, d, -3) : g, p3 = near ? shifted(B, i, j, k, d, 3) : g;
-            const int LI = ld(B.code, g), LM2 = ld(B.code, m2), LM1 = ld(B.code, m1), LP1 = ld(B.code, p1),
-                      LP2 = ld(B.code, p2);
+            uint32_t x[4];
+#pragma unroll
+            for (int q = 0; q < 4; ++q) x[q] = shifted(B, i, j, k, d, form[d].o[q]);
+            const uint32_t m1 = shifted(B, i, j, k, d, -1), p1 = shifted(B, i, j, k, d, 1);
+            const double a0 = ld(Uin[0], m1), b0 = ld(Uin[0], p1), ad = ld(Uin[1 + d], m1), bd = ld(Uin[1 + d], p1);
+            const S mx = ld(geo<S>(B, 1 + 3 * d), g), my = ld(geo<S>(B, 2 + 3 * d), g), mz = ld(geo<S>(B, 3 + 3 * d), g);
             S dU[5];
 #pragma unroll
             for (int c = 0; c < 5; ++c) {
                 const double *u = Uin[c];
-                const double a = ld(u, m1), b = ld(u, p1), a2 = ld(u, m2), b2 = ld(u, p2);
-                if (near) {
-                    const double f[7] = {ld(u, m3), a2, a, U[c], b, b2, ld(u, p3)};
-                    dU[c] = S(loc_derivative(f, LI, LM2, LM1, LP1, LP2, false));
-                } else {
-                    dU[c] = S((1.0 / 12.0) * (8.0 * (b - a) - (b2 - a2)));
-                }
-                pin_(dU[c]);
+                dU[c] = S(form[d].w[0] * ld(u, x[0]) + form[d].w[1] * ld(u, x[1]) + form[d].w[2] * ld(u, x[2])
+                          + form[d].w[3] * ld(u, x[3]));
             }
-            sk[d] = add(d, U[1 + d], dU, ld(Uin[0], m1), ld(Uin[0], p1), ld(Uin[1 + d], m1), ld(Uin[1 + d], p1),
-                        ld(geo<S>(B, 1 + 3 * d), g), ld(geo<S>(B, 2 + 3 * d), g), ld(geo<S>(B, 3 + 3 * d), g));
+            sk[d] = add(d, U[1 + d], dU, a0, b0, ad, bd, mx, my, mz);
         }
         uint32_t g2 = g;
         pin_(g2);   // the metrics again, not held through the gradients
@@ -364,16 +387,13 @@ __device__ __forceinline__ void visc_tile(const BlockDev &B, uint32_t lt, int mo
     else visc_node<S, false, NT>(B, i, j, k, mode);
 }
 
-// Viscous node fluxes of 256 shell nodes: shell tile s of the list (block = s / shell_tiles).
+// Viscous node fluxes of shell tile s of the list (block = s / shell_tiles).
 template <typename S>
 __device__ __forceinline__ void visc_shell_tile(const BlockDev *__restrict__ blks, uint32_t s, int mode, uint32_t shell_tiles)
 {
     const BlockDev &B = blks[s / shell_tiles];
-    const uint32_t t = (s % shell_tiles) * 256 + threadIdx.x;
-    if (!B.viscous || t >= shell_count(B)) return;
     int i, j, k;
-    shell_node(B, t, i, j, k);
-    visc_node<S, true, false>(B, i, j, k, mode);
+    if (B.viscous && B.code && shell_node(B, s % shell_tiles, i, j, k)) visc_node<S, true, false>(B, i, j, k, mode);
 }
 
 // Node tiles of the list first (tile ids through the XCD remap), then, for lists with bounded
@@ -619,31 +639,36 @@ __device__ __forceinline__ void update_node(const BlockDev &B, int i, int j, int
         }
     }
     if (B.viscous) {
+        if constexpr (LOC) {
+            // bounded block: the loc-selected forms of Weno.cl:2732-2856
+            LocForm form[3];
+            loc_forms(B, i, j, k, true, form);
+            // across a wake cut the row -m of column i is the row m of column ni - 1 - i, where eta runs the
+            // other way: its flux along j, negated
+            const bool cut = B.bc[2] == CFDX_BC_WALL_CUT && !(i >= B.cut_i0 && i <= B.cut_i1);
 #pragma unroll
-        for (int d = 0; d < 3; ++d) {
-            const uint32_t m2 = shifted(B, i, j, k, d, -2), m1 = shifted(B, i, j, k, d, -1);
-            const uint32_t p1 = shifted(B, i, j, k, d, 1), p2 = shifted(B, i, j, k, d, 2);
-            if (LOC && near_side(B, i, j, k, d)) {
-                // bounded block: the loc-selected forms of Weno.cl:2732-2856
-                const uint32_t m3 = shifted(B, i, j, k, d, -3), p3 = shifted(B, i, j, k, d, 3);
-                const int LI = ld(B.code, g), LM2 = ld(B.code, m2), LM1 = ld(B.code, m1), LP1 = ld(B.code, p1),
-                          LP2 = ld(B.code, p2);
-                // across a wake cut the row -m of column i is the row m of column ni - 1 - i, where eta runs the
-                // other way: its flux along j, negated
-                const bool cut = d == 1 && B.bc[2] == CFDX_BC_WALL_CUT && !(i >= B.cut_i0 && i <= B.cut_i1);
-                const auto below = [&](int o, uint32_t own) {
-                    return cut && j < o ? node_index(B, B.ni - 1 - i, o - j, k) : own;
-                };
-                const uint32_t x3 = below(3, m3), x2 = below(2, m2), x1 = below(1, m1);
-                const double s3 = cut && j < 3 ? -1.0 : 1.0, s2 = cut && j < 2 ? -1.0 : 1.0, s1 = cut && j < 1 ? -1.0 : 1.0;
+            for (int d = 0; d < 3; ++d) {
+                uint32_t x[4];
+                double w[4];
+#pragma unroll
+                for (int q = 0; q < 4; ++q) {
+                    const int o = form[d].o[q];
+                    const bool across = d == 1 && cut && j + o < 0;
+                    x[q] = across ? node_index(B, B.ni - 1 - i, -(j + o), k) : shifted(B, i, j, k, d, o);
+                    w[q] = across ? -form[d].w[q] : form[d].w[q];
+                }
 #pragma unroll
                 for (int c = 1; c < 5; ++c) {
-                    const S *fv = (const S *)B.Fv[d][c - 1];
-                    const double f[7] = {s3 * (double)ld(fv, x3), s2 * (double)ld(fv, x2), s1 * (double)ld(fv, x1), (double)ld(fv, g),
-                                         (double)ld(fv, p1), (double)ld(fv, p2), (double)ld(fv, p3)};
-                    L[c] += loc_derivative(f, LI, LM2, LM1, LP1, LP2, true);
+                    const S *f = (const S *)B.Fv[d][c - 1];
+                    L[c] += w[0] * (double)ld(f, x[0]) + w[1] * (double)ld(f, x[1]) + w[2] * (double)ld(f, x[2])
+                            + w[3] * (double)ld(f, x[3]);
                 }
-            } else {
+            }
+        } else {
+#pragma unroll
+            for (int d = 0; d < 3; ++d) {
+                const uint32_t m2 = shifted(B, i, j, k, d, -2), m1 = shifted(B, i, j, k, d, -1);
+                const uint32_t p1 = shifted(B, i, j, k, d, 1), p2 = shifted(B, i, j, k, d, 2);
 #pragma unroll
                 for (int c = 1; c < 5; ++c) {
                     const S *f = (const S *)B.Fv[d][c - 1];
@@ -712,7 +737,7 @@ __device__ __forceinline__ void monitor_wave(const BlockDev &B, uint32_t slot, d
 }
 
 // tiles as in k_visc; the shell tiles' monitor slots follow the block's node tiles' (tiles x
-// waves per tile), one per wave of 64 shell nodes
+// waves per tile)
 template <typename S, int TX, int TY, int K, bool LOOP>
 __global__ void __launch_bounds__(TX *TY) k_update(const BlockDev *__restrict__ blks, const uint32_t *__restrict__ prefix,
                                                    uint32_t nblk, uint32_t total, int mode, uint32_t shell_tiles,
@@ -724,20 +749,15 @@ __global__ void __launch_bounds__(TX *TY) k_update(const BlockDev *__restrict__ 
         // residual monitor of the step (Solver.cpp:546-573): |du|, |dv|, |de| against the RK base
         double mdu = 0.0, mdv = 0.0, mde = 0.0;
         if (BND && wg < first) {   // the shell tiles first, as in k_flux
-            const uint32_t s = wg;
-            if (s >= shell) return;
-            const BlockDev &B = blks[s / shell_tiles];
-            const uint32_t t = (s % shell_tiles) * (TX * TY) + threadIdx.x;
-            const uint32_t ns = shell_count(B);
-            if ((s % shell_tiles) * (TX * TY) >= ns) return;   // whole tile past the shell
-            if (t < ns) {
-                int i, j, k;
-                shell_node(B, t, i, j, k);
-                update_node<S, true, false>(B, i, j, k, mode, Lout, mdu, mdv, mde);
-            }
-            if (mode == 2 && B.mon && (t & ~63u) < ns) {
+            if (wg >= shell) return;
+            const BlockDev &B = blks[wg / shell_tiles];
+            const uint32_t s = wg % shell_tiles;
+            if (!B.code || s >= shell_tile_count(B)) return;
+            int i, j, k;
+            if (shell_node(B, s, i, j, k)) update_node<S, true, false>(B, i, j, k, mode, Lout, mdu, mdv, mde);
+            if (mode == 2 && B.mon && threadIdx.x < (s < shell_row_tiles(B) ? SHELL_TILE : shell_column_tile(B))) {
                 const uint32_t main_slots = ((B.ni + TX - 1) / TX) * ((B.nj + TY - 1) / TY) * B.nk * (uint32_t)(TX * TY / 64);
-                monitor_wave(B, main_slots + t / 64, mdu, mdv, mde);
+                monitor_wave(B, main_slots + shell_wave(B, s, threadIdx.x / 64), mdu, mdv, mde);
             }
             return;
         }
@@ -1010,7 +1030,7 @@ void launch_node_k(const LaunchList &L, uint32_t cap, hipStream_t st, bool visc_
 {
     constexpr int TX = NODE_TILES[V][0], TY = NODE_TILES[V][1];
     static_assert(TX * TY == 256, "node tiles have 256 threads");
-    const uint32_t shell_tiles = K == LIST_BOUNDED ? (L.shell_max + TX * TY - 1) / (TX * TY) : 0u;
+    const uint32_t shell_tiles = K == LIST_BOUNDED ? L.shell_tiles : 0u;
     // one workgroup per shell tile too
     const uint32_t shell = L.nblk * shell_tiles, all = L.total[0] + (visc_kernel ? shell : (shell + 7) & ~7u);
     const bool loop = cap && cap < all;
@@ -1079,7 +1099,7 @@ void launch_flux(const LaunchList &L, int mode, hipStream_t st, bool any_visc)
     uint32_t slots = (most + 7) / 8;
     T.chunk = std::min(FLUX_CHUNK, slots);
     slots = (slots + T.chunk - 1) / T.chunk * T.chunk;
-    const uint32_t shell_tiles = L.bc_face && any_visc ? (L.shell_max + 255) / 256 : 0u;
+    const uint32_t shell_tiles = L.bc_face && any_visc ? L.shell_tiles : 0u;
     const dim3 g(8 * (any_visc ? 4u : 3u) * slots + ((L.nblk * shell_tiles + 7) & ~7u));
     auto go = [&](auto kernel) {
         hipLaunchKernelGGL(kernel, g, dim3(256), 0, st, L.blks, T, L.nblk, slots, mode, shell_tiles);
@@ -1090,6 +1110,12 @@ void launch_flux(const LaunchList &L, int mode, hipStream_t st, bool any_visc)
     else go(k_flux<S, true, LIST_PLAIN>);
 }
 
+bool stage_forks(const LaunchList &L, const Overlap *ov)
+{
+    const TileCfg &t = L.tiles;
+    return ov && (L.grid_cap || t.face[0] || t.face[1] || t.face[2] || t.node);
+}
+
 template <typename S>
 void launch_stage(const LaunchList &L, int mode, hipStream_t st, bool any_visc, hipEvent_t *ev, const Overlap *ov)
 {
@@ -1097,8 +1123,7 @@ void launch_stage(const LaunchList &L, int mode, hipStream_t st, bool any_visc, 
     rec(0);
     // the viscous node kernel reads the stage vector, primitives and geometry and writes Fv and mu;
     // the face sweeps read the primitives and geometry and write F-hat: independent until the update
-    const TileCfg &t = L.tiles;
-    const bool overlap = ov && !ev, together = overlap && !L.grid_cap && !(t.face[0] | t.face[1] | t.face[2] | t.node);
+    const bool overlap = ov && !ev, together = overlap && !stage_forks(L, ov);
     hipStream_t vs = st;
     if (together) {
         launch_flux<S>(L, mode, st, any_visc);
