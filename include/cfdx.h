@@ -328,8 +328,10 @@ int cfdx_batch_size(cfdx_batch *q);
 /* grid_cap = 0: one workgroup per tile; > 0: persistent launches of at most grid_cap workgroups
  * that loop over the tiles. */
 int cfdx_batch_set_grid(cfdx_batch *q, uint32_t grid_cap);
-/* nsteps RK3 steps of every block; use_graph = 1 captures one step in a hipGraph on first use
- * (re-captured after the batch changes) and replays it. Asynchronous on the context stream. No
+/* nsteps RK3 steps of every block. use_graph = 1: where a stage forks onto the context's second
+ * stream (other tile shapes than the defaults or a capped grid, cfdx_ctx_set_overlap), one step is
+ * captured in a hipGraph on first use (re-captured after the batch changes) and replayed; a stage
+ * on one stream is launched directly, which is faster. Asynchronous on the context stream. No
  * other thread may call the library during a call that captures: the HIP runtime invalidates the
  * capture when another thread allocates device memory or creates streams meanwhile. */
 int cfdx_batch_step(cfdx_batch *q, int nsteps, int use_graph);
