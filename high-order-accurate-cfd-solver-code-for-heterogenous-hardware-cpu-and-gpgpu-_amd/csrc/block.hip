@@ -53,8 +53,12 @@ struct cfdx_batch {
     uint32_t *dprefix = nullptr;
     size_t cap = 0;
     bool dirty = true;
-    LaunchList L;
-    bool any_visc = false;
+    // the blocks' launches: groups that the last-level cache holds, each a list of its own
+    struct Group {
+        LaunchList L;
+        bool any_visc = false;
+    };
+    std::vector<Group> groups;
     uint32_t grid_cap = 0;
     cfdx::blk::TileCfg tiles;
     hipGraph_t graph = nullptr;
@@ -302,6 +306,47 @@ void drop_graph(cfdx_batch *q)
     q->graph = nullptr;
 }
 
+// The blocks of a batch in groups that are stepped one after the other: what a stage of a group touches
+// stays in the 256 MB last-level cache for the next stage and step, and a group still fills the chip. Larger
+// blocks are groups of their own; the others are packed, largest first, each into the first group
+// with room. us a step of all blocks in one list and in groups, mixed and FP64: eight cubes of 32^3 .. 128^3
+// 2205 -> 1910 and 3730 -> 3560; the four C-grids of the served ladder 1949 -> 1758 and 2959 -> 2776; twelve 64^3
+// 1305 -> 1183 (three a group, 239 MB) and 2272 -> 2025 (two, 268 MB; three, 402 MB: 2240; one: 2135); three 128^3 2837 ->
+// 2614 and 4800 -> 4652; twenty-four 32^3 mixed in one list of 239 MB 376, eight a group 430.
+constexpr uint64_t GROUP_BYTES = (uint64_t)256 << 20;
+std::vector<std::vector<size_t>> group_blocks(const std::vector<cfdx_block *> &blocks)
+{
+    std::vector<size_t> order(blocks.size());
+    for (size_t i = 0; i < order.size(); ++i) order[i] = i;
+    auto bytes = [&](size_t i) { return cfdx::blk::stage_bytes(blocks[i]->B); };
+    std::stable_sort(order.begin(), order.end(), [&](size_t a, size_t b) { return bytes(a) > bytes(b); });
+    std::vector<std::vector<size_t>> groups;
+    std::vector<uint64_t> used;
+    auto put = [&](size_t g, size_t i) {
+        groups[g].push_back(i);
+        used[g] += bytes(i);
+    };
+    for (size_t i : order) {
+        size_t g = 0;
+        while (g < groups.size() && used[g] + bytes(i) > GROUP_BYTES) ++g;
+        if (g == groups.size()) {
+            groups.emplace_back();
+            used.push_back(0);
+        }
+        put(g, i);
+    }
+    // the same number of groups, evenly filled where that keeps within the size (a last group of one small
+    // block would cost its launches' latency for little work)
+    std::vector<std::vector<size_t>> first(groups.size());
+    std::vector<uint64_t> first_used(groups.size(), 0);
+    std::swap(groups, first);
+    std::swap(used, first_used);
+    for (size_t i : order) put((size_t)(std::min_element(used.begin(), used.end()) - used.begin()), i);
+    for (size_t g = 0; g < groups.size(); ++g)
+        if (used[g] > GROUP_BYTES && groups[g].size() > 1) return first;
+    return groups;
+}
+
 int upload_batch(cfdx_batch *q)
 {
     bool changed = q->dirty || q->seen.size() != q->blocks.size();
@@ -315,49 +360,55 @@ int upload_batch(cfdx_batch *q)
         q->dprefix = nullptr;
         const size_t cap = std::max<size_t>(nb, 2 * q->cap);
         hipError_t e = hipMalloc((void **)&q->dB, cap * sizeof(BlockDev));
-        if (e == hipSuccess) e = hipMalloc((void **)&q->dprefix, 4 * (cap + 1) * sizeof(uint32_t));
+        if (e == hipSuccess) e = hipMalloc((void **)&q->dprefix, 4 * 2 * cap * sizeof(uint32_t));
         if (e != hipSuccess) { q->cap = 0; return cfdx::fail(CFDX_E_NOMEM, "batch: descriptor allocation failed"); }
         q->cap = cap;
     }
-    std::vector<BlockDev> h(nb);
-    std::vector<uint32_t> pre(4 * (q->cap + 1), 0);
-    uint32_t tot[4] = {0, 0, 0, 0};
-    q->any_visc = false;
-    uint64_t bytes = 0;
-    bool rows = true;
-    for (const cfdx_block *b : q->blocks) {
-        bytes += cfdx::blk::stage_bytes(b->B);
-        rows = rows && cfdx::blk::rows_stream(b->B);
-    }
-    q->L.stream = cfdx::blk::streams_past_cache(bytes, rows);
-    for (size_t i = 0; i < nb; ++i) {
-        h[i] = q->blocks[i]->B;
-        h[i].stream = q->L.stream;
-        h[i].strip = (uint32_t)q->tiles.strip;
-        for (int kind = 0; kind < 4; ++kind) {
-            h[i].tile0[kind] = tot[kind];
-            pre[kind * (q->cap + 1) + i] = tot[kind];
-            tot[kind] += cfdx::blk::tiles_of(q->blocks[i]->B, kind, q->tiles);
+    // descriptors group by group; a group of n blocks has n + 1 prefix entries of each kind, so 2 x cap
+    // entries a kind hold any grouping
+    const std::vector<std::vector<size_t>> packed = group_blocks(q->blocks);
+    std::vector<BlockDev> h;
+    h.reserve(nb);
+    std::vector<uint32_t> pre(4 * 2 * q->cap, 0);
+    q->groups.assign(packed.size(), {});
+    size_t at = 0;   // first prefix entry of the group
+    for (size_t g = 0; g < packed.size(); ++g) {
+        LaunchList &L = q->groups[g].L;
+        L.blks = q->dB + h.size();
+        L.nblk = (uint32_t)packed[g].size();
+        L.grid_cap = q->grid_cap;
+        L.tiles = q->tiles;
+        uint64_t bytes = 0;
+        bool rows = true;
+        for (size_t i : packed[g]) {
+            bytes += cfdx::blk::stage_bytes(q->blocks[i]->B);
+            rows = rows && cfdx::blk::rows_stream(q->blocks[i]->B);
         }
-        q->any_visc |= h[i].viscous != 0;
+        L.stream = cfdx::blk::streams_past_cache(bytes, rows);
+        uint32_t tot[4] = {0, 0, 0, 0};
+        for (size_t n = 0; n < packed[g].size(); ++n) {
+            BlockDev B = q->blocks[packed[g][n]]->B;
+            B.strip = (uint32_t)q->tiles.strip;
+            B.stream = L.stream;
+            for (int kind = 0; kind < 4; ++kind) {
+                B.tile0[kind] = tot[kind];
+                pre[kind * 2 * q->cap + at + n] = tot[kind];
+                tot[kind] += cfdx::blk::tiles_of(B, kind, q->tiles);
+            }
+            q->groups[g].any_visc |= B.viscous != 0;
+            bc_extent(B, L);
+            h.push_back(B);
+        }
+        for (int kind = 0; kind < 4; ++kind) {
+            L.prefix[kind] = q->dprefix + kind * 2 * q->cap + at;
+            L.total[kind] = tot[kind];
+            pre[kind * 2 * q->cap + at + L.nblk] = tot[kind];
+        }
+        at += L.nblk + 1;
     }
-    for (int kind = 0; kind < 4; ++kind) pre[kind * (q->cap + 1) + nb] = tot[kind];
     if (nb) CFDX_HIP(hipMemcpyAsync(q->dB, h.data(), nb * sizeof(BlockDev), hipMemcpyHostToDevice, q->ctx->stream), "batch descriptors");
-    CFDX_HIP(hipMemcpyAsync(q->dprefix, pre.data(), pre.size() * sizeof(uint32_t), hipMemcpyHostToDevice, q->ctx->stream), "batch prefix");
+    if (nb) CFDX_HIP(hipMemcpyAsync(q->dprefix, pre.data(), pre.size() * sizeof(uint32_t), hipMemcpyHostToDevice, q->ctx->stream), "batch prefix");
     CFDX_HIP(hipStreamSynchronize(q->ctx->stream), "batch upload sync");
-    q->L.blks = q->dB;
-    q->L.nblk = (uint32_t)nb;
-    for (int kind = 0; kind < 4; ++kind) {
-        q->L.prefix[kind] = q->dprefix + kind * (q->cap + 1);
-        q->L.total[kind] = tot[kind];
-    }
-    q->L.grid_cap = q->grid_cap;
-    q->L.tiles = q->tiles;
-    q->L.bc_face = 0;
-    for (int d = 0; d < 3; ++d) q->L.bc_face_d[d] = 0;
-    q->L.bc_planes = 0;
-    q->L.shell_tiles = 0;
-    for (size_t i = 0; i < nb; ++i) bc_extent(h[i], q->L);
     q->seen.resize(nb);
     for (size_t i = 0; i < nb; ++i) q->seen[i] = q->blocks[i]->version;
     q->dirty = false;
@@ -939,10 +990,10 @@ extern "C" int cfdx_batch_step(cfdx_batch *q, int nsteps, int use_graph)
     // a captured graph pays for the fork and join of the second stream; the launches of a stage on one
     // stream follow each other faster without (32^3 52 us a step against 57, mixed 40 against 44; 5 us a step at
     // every size, 64^3 178 against 183, 256^3 12.87 ms both)
-    if (!use_graph || !cfdx::blk::stage_forks(q->L, overlap_of(q->ctx, ov))) {
-        for (int s = 0; s < nsteps; ++s)
-            for (int j = 0; j < 3; ++j)
-                cfdx::blk::stage(q->L, q->precision, j, st, q->any_visc, nullptr, overlap_of(q->ctx, ov));
+    if (!use_graph || !cfdx::blk::stage_forks(q->groups[0].L, overlap_of(q->ctx, ov))) {
+        for (const auto &g : q->groups)
+            for (int s = 0; s < nsteps; ++s)
+                for (int j = 0; j < 3; ++j) cfdx::blk::stage(g.L, q->precision, j, st, g.any_visc, nullptr, overlap_of(q->ctx, ov));
         return cfdx::check_launch("batch stage");
     }
     if (q->exec && q->graph_gen != q->ctx->gen.load()) drop_graph(q);   // overlap switch or stream changed
@@ -951,8 +1002,8 @@ extern "C" int cfdx_batch_step(cfdx_batch *q, int nsteps, int use_graph)
         CFDX_HIP(hipStreamBeginCapture(st, hipStreamCaptureModeThreadLocal), "hipStreamBeginCapture");
         // the second stream joins the capture through the fork event and is joined back before
         // each update, so the graph holds the overlap too
-        for (int j = 0; j < 3; ++j)
-            cfdx::blk::stage(q->L, q->precision, j, st, q->any_visc, nullptr, overlap_of(q->ctx, ov));
+        for (const auto &g : q->groups)
+            for (int j = 0; j < 3; ++j) cfdx::blk::stage(g.L, q->precision, j, st, g.any_visc, nullptr, overlap_of(q->ctx, ov));
         hipError_t e = hipStreamEndCapture(st, &q->graph);
         if (e != hipSuccess) { q->graph = nullptr; return cfdx::hip_fail(e, "hipStreamEndCapture"); }
         e = hipGraphInstantiate(&q->exec, q->graph, nullptr, nullptr, 0);

@@ -2,8 +2,10 @@
 // memory.
 #include "ctx.hpp"
 
+#include <chrono>
 #include <map>
 #include <mutex>
+#include <thread>
 #include <vector>
 
 namespace cfdx {
@@ -91,8 +93,17 @@ size_t pool_cached(int device)
 extern "C" int cfdx_pool_trim(cfdx_ctx *ctx)
 {
     CFDX_TRY(cfdx::enter(ctx));
+    // the driver may give freed memory back a little later: wait for it (bounded), so that a
+    // cfdx_mem_info that follows counts it
+    size_t before = 0, now = 0, total = 0;
+    const size_t kept = cfdx::pool_cached(ctx->device);
+    const bool known = hipMemGetInfo(&before, &total) == hipSuccess;
     cfdx::pool_trim(ctx->device);
     cfdx::staging_trim();
+    for (int q = 0; known && kept && q < 400; ++q) {
+        if (hipMemGetInfo(&now, &total) != hipSuccess || now >= before + kept / 2) break;
+        std::this_thread::sleep_for(std::chrono::microseconds(500));
+    }
     return CFDX_OK;
 }
 

@@ -108,3 +108,39 @@ def test_streaming_accesses_give_the_same_bits(ctx, precision):
         x.close()
     for f in FIELDS:
         assert np.array_equal(got[f], want[f]), f
+
+
+@pytest.mark.parametrize("tiles", [(0, 0, 0, 0, 4), (1, 1, 2, 1, 4)], ids=["default", "forked"])
+@pytest.mark.parametrize("graph", [True, False], ids=["graph", "eager"])
+def test_groups_of_a_batch_give_the_bits_of_each_block_alone(ctx, graph, tiles):
+    """More blocks than one cache-sized group holds (134 MB each of three, and small ones, bounded and
+    inviscid among them), also after a block has left: every block as if stepped alone."""
+    visc, inv = cfdx.default_params(mach=0.3, reyl=900.0), cfdx.euler_params()
+
+    def make():
+        return ([periodic(ctx, s, cfdx.FP64, p) for s, p in (((12, 10, 8), visc), ((64, 64, 64), visc), ((64, 64, 64), inv),
+                                                             ((33, 20, 9), inv), ((64, 64, 64), visc))]
+                + [bounded(ctx, "cgrid", cfdx.FP64)])
+    want = []
+    for b, n in zip(make(), (3, 3, 3, 2, 3, 3)):
+        q = cfdx.Batch(cfdx.FP64, ctx)
+        q.add(b)
+        q.step(n, False)
+        want.append(b.get_flow())
+        q.close()
+        b.close()
+    blocks = make()
+    q = cfdx.Batch(cfdx.FP64, ctx)
+    q.set_tiles(tiles)
+    for b in blocks:
+        q.add(b)
+    q.step(2, graph)
+    q.remove(blocks[3])
+    q.step(1, graph)
+    for b, w in zip(blocks, want):
+        got = b.get_flow()
+        for f in FIELDS:
+            assert np.array_equal(got[f], w[f]), f
+    q.close()
+    for b in blocks:
+        b.close()
