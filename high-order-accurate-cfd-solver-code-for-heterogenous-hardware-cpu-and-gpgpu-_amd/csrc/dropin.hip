@@ -42,6 +42,16 @@ __device__ __forceinline__ void walk(const int32_t *G, int g, int d, int (&idx)[
     }
 }
 
+// A record of five doubles (40 bytes, 8-byte aligned): two 16-byte loads and one of 8. Lanes are a record
+// apart, so a load takes as many cache lines whatever its width: the kernels are bound by the address
+// rate, and five 8-byte loads a record cost five times the lines instead of three.
+__device__ __forceinline__ void load5(const double *p, double (&v)[5])
+{
+    typedef double pair __attribute__((ext_vector_type(2), aligned(8)));
+    const pair a = *(const pair *)p, b = *(const pair *)(p + 2);
+    v[0] = a.x; v[1] = a.y; v[2] = b.x; v[3] = b.y; v[4] = p[4];
+}
+
 // ---------------------------------------------------------------------------
 // U_Q.cl:36-125
 // ---------------------------------------------------------------------------
@@ -79,7 +89,7 @@ __global__ void __launch_bounds__(256) k_uq(double *__restrict__ U_C, double *__
 // ---------------------------------------------------------------------------
 // Viscous.cl:23-643
 // ---------------------------------------------------------------------------
-__global__ void __launch_bounds__(128, 4) k_viscous(const double *__restrict__ U_C, double *__restrict__ Fo, double *__restrict__ Eo,
+__global__ void __launch_bounds__(128, 3) k_viscous(const double *__restrict__ U_C, double *__restrict__ Fo, double *__restrict__ Eo,
                                                  double *__restrict__ Go, double *__restrict__ Fvo, double *__restrict__ Evo,
                                                  double *__restrict__ Gvo, const int32_t *__restrict__ G,
                                                  const double *__restrict__ metric, const double *__restrict__ det,
@@ -88,8 +98,7 @@ __global__ void __launch_bounds__(128, 4) k_viscous(const double *__restrict__ U
     const int g = blockIdx.x * blockDim.x + threadIdx.x;
     if (g >= n) return;
     double U[5];
-#pragma unroll
-    for (int c = 0; c < 5; ++c) U[c] = U_C[(size_t)5 * g + c];
+    load5(U_C + (size_t)5 * g, U);
     const NodeRatios<double> nr = node_ratios(U);
     double Gr[4][3] = {}, sk[3], m[9];
 #pragma unroll
@@ -99,18 +108,21 @@ __global__ void __launch_bounds__(128, 4) k_viscous(const double *__restrict__ U
         int loc[7];
 #pragma unroll
         for (int s = 1; s < 6; ++s) loc[s] = G[GRID_N * idx[s] + G_LOC];
+        double V[7][5];
+#pragma unroll
+        for (int s = 0; s < 7; ++s) {
+            if (s == 3) continue;
+            load5(U_C + (size_t)5 * idx[s], V[s]);
+        }
         double dU[5];
 #pragma unroll
         for (int c = 0; c < 5; ++c) {
-            double f[7];
-#pragma unroll
-            for (int s = 0; s < 7; ++s) f[s] = U_C[(size_t)5 * idx[s] + c];
+            const double f[7] = {V[0][c], V[1][c], V[2][c], U[c], V[4][c], V[5][c], V[6][c]};
             dU[c] = loc_derivative(f, loc[3], loc[1], loc[2], loc[4], loc[5], false);
             pin_(dU[c]);
         }
         // magnitude of the MTS scale-similarity term of momentum component d+1 along d (Viscous.cl:493-495)
-        const double *um = U_C + (size_t)5 * idx[2], *up = U_C + (size_t)5 * idx[4];
-        sk[d] = fabs_(nr.r[d] - ((0.25 * um[1 + d] + 0.5 * U[1 + d] + 0.25 * up[1 + d]) * pinv_(0.25 * um[0] + 0.5 * U[0] + 0.25 * up[0])));
+        sk[d] = fabs_(nr.r[d] - ((0.25 * V[2][1 + d] + 0.5 * U[1 + d] + 0.25 * V[4][1 + d]) * pinv_(0.25 * V[2][0] + 0.5 * U[0] + 0.25 * V[4][0])));
         pin_(sk[d]);
 #pragma unroll
         for (int c = 3 * d; c < 3 * d + 3; ++c) m[c] = metric[(size_t)MET_N * g + c];
@@ -174,9 +186,16 @@ __global__ void __launch_bounds__(64 * 6, 3) k_weno(int j, double Mach, double d
         const double *k = metric + (size_t)MET_N * g + 9 + 9 * (2 * d + side) + 3 * d;
         const double detf = deter[(size_t)DET_N * g + 2 * d + side];
         const double *nf = d == 0 ? F : d == 1 ? E : Gf;
-        double h[5];
-        face_flux([&](int m, int c) { return Q_C[at[m] + c]; }, roe, k[0], k[1], k[2], detf, eps,
-                  [&](int m, int c) { return nf[at[m] + c]; }, h);
+        double q[6][5], h[5];
+#pragma unroll
+        for (int m = 0; m < 6; ++m) load5(Q_C + at[m], q[m]);
+        face_flux([&](int m, int c) { return q[m][c]; }, roe, k[0], k[1], k[2], detf, eps, h);
+        asm volatile("" ::: "memory");   // the node fluxes only now: with them loaded before, the registers do not hold both
+        double n6[6][5];
+#pragma unroll
+        for (int m = 0; m < 6; ++m) load5(nf + at[m], n6[m]);
+#pragma unroll
+        for (int c = 0; c < 5; ++c) h[c] += midpoint_correction(n6[0][c], n6[1][c], n6[2][c], n6[3][c], n6[4][c], n6[5][c]);
 #pragma unroll
         for (int c = 0; c < 5; ++c) face[wave][c][lane] = h[c];
         if (side == 0) {
@@ -184,11 +203,12 @@ __global__ void __launch_bounds__(64 * 6, 3) k_weno(int j, double Mach, double d
             int loc[7];
 #pragma unroll
             for (int s = 1; s < 6; ++s) loc[s] = G[GRID_N * idx[s] + G_LOC];
+            double V[7][5];
+#pragma unroll
+            for (int s = 0; s < 7; ++s) load5(nv + (size_t)5 * idx[s], V[s]);
 #pragma unroll
             for (int c = 0; c < 5; ++c) {
-                double fv[7];
-#pragma unroll
-                for (int s = 0; s < 7; ++s) fv[s] = nv[(size_t)5 * idx[s] + c];
+                const double fv[7] = {V[0][c], V[1][c], V[2][c], V[3][c], V[4][c], V[5][c], V[6][c]};
                 vis[d][c][lane] = loc_derivative(fv, loc[3], loc[1], loc[2], loc[4], loc[5], true);
             }
         }

@@ -383,18 +383,12 @@ __device__ __forceinline__ T midpoint_correction(T f0, T f1, T f2, T f3, T f4, T
     return T(57.0 / 11520.0) * (f0 + f5) - T(411.0 / 11520.0) * (f1 + f4) + T(354.0 / 11520.0) * (f2 + f3);
 }
 
-// Face flux F-hat = LLF + midpoint correction from the node fluxes nf(m, c) at offsets -2..+3; (k0, k1,
-// k2) the face metric row as stored by the reference, detf the face det.
-template <typename T, typename GetQ, typename GetF>
-__device__ __forceinline__ void face_flux(const GetQ &q, const T (&roe)[5], T k0, T k1, T k2, T detf, T eps, const GetF &nf,
-                                          T (&out)[5])
+// LLF face flux of a face metric row (k0, k1, k2) as stored by the reference; detf the face det.
+template <typename T, typename GetQ>
+__device__ __forceinline__ void face_flux(const GetQ &q, const T (&roe)[5], T k0, T k1, T k2, T detf, T eps, T (&llf)[5])
 {
     const T kn = sqrt_(k0 * k0 + k1 * k1 + k2 * k2), ik = inv_(kn);
-    T llf[5];
     face_llf(q, roe, pinv_(roe[4]), k0 * ik, k1 * ik, k2 * ik, detf * kn, eps, llf);
-#pragma unroll
-    for (int c = 0; c < 5; ++c)
-        out[c] = llf[c] + midpoint_correction(nf(0, c), nf(1, c), nf(2, c), nf(3, c), nf(4, c), nf(5, c));
 }
 
 // Viscous + SGS node fluxes (Viscous.cl:439-631, its mixed-time-scale model or the Smagorinsky
