@@ -1,13 +1,13 @@
 // Large device-to-host copies: chunks into a ring of pinned buffers, copied on to the caller's memory by a
 // few threads while the next chunks arrive. A copy straight into pageable memory moves 10 GB/s on an
-// MI355X host (the runtime pins the pages as it goes; 4 GB/s into fresh 4 kB pages), the link 57;
-// one thread's copy into fresh memory is no faster than that (5-12 GB/s, page faults), eight reach 50.
-// 151 MB into fresh memory: 15.2 ms straight, 3.7 ms so.
+// MI355X host (the runtime pins the pages as it goes), the link 57; one thread's copy into fresh memory is no
+// faster than that (page faults), four together reach 50. Into fresh memory, straight and so: 9 MB 0.52 and
+// 0.35 ms, 19 MB 1.08 and 0.54, 151 MB 14.2 and 3.6, 1.2 GB 113 and 26; eight or twelve threads are no faster, chunks of
+// 1 MB 5.0 ms at 151 MB.
 #include <sched.h>
 
 #include <algorithm>
 #include <atomic>
-#include <condition_variable>
 #include <cstring>
 #include <mutex>
 #include <system_error>
@@ -21,7 +21,7 @@ namespace {
 
 constexpr size_t CHUNK = (size_t)4 << 20, SLOTS = 8;
 constexpr size_t STAGED_FROM = 2 * CHUNK;   // smaller copies go straight
-constexpr unsigned THREADS = 8;
+constexpr unsigned THREADS = 4;
 constexpr size_t KEPT = 2;                  // rings kept for the next copy (32 MB of pinned memory each)
 
 struct Ring {
@@ -81,60 +81,58 @@ unsigned copy_threads()
     return std::min(THREADS, (unsigned)std::max(n, 1));
 }
 
-// One copy: `issued` chunks are on the stream, workers take them in order and mark them `done`.
+// One copy. The calling thread puts chunks on the stream as slots come free and watches them arrive (one
+// thread asks the runtime; eight waiting on events took 100 us a chunk); the workers take arrived chunks in
+// order and copy them out. All of them spin with yields: the copy alone is over in milliseconds.
 struct Copy {
     Ring &ring;
     char *dst;
     size_t bytes, chunks;
-    std::mutex m;
-    std::condition_variable cv;
-    size_t issued = 0, next = 0, done = 0;   // done: chunks copied out
-    std::vector<char> out;                   // per chunk: copied out
-    hipError_t err = hipSuccess;
+    std::atomic<size_t> arrived{0}, next{0};
+    std::atomic<bool> failed{false};
+    std::vector<std::atomic<char>> out;   // per chunk: copied out
 
-    Copy(Ring &r, void *d, size_t n) : ring(r), dst((char *)d), bytes(n), chunks((n + CHUNK - 1) / CHUNK), out(chunks, 0) {}
+    Copy(Ring &r, void *d, size_t n)
+        : ring(r), dst((char *)d), bytes(n), chunks((n + CHUNK - 1) / CHUNK), out(chunks)
+    {
+    }
 
     void work()
     {
-        (void)hipSetDevice(ring.device);
         for (;;) {
-            size_t c;
-            {
-                std::unique_lock<std::mutex> lock(m);
-                cv.wait(lock, [&] { return err != hipSuccess || next >= chunks || next < issued; });
-                if (err != hipSuccess || next >= chunks) return;
-                c = next++;
+            const size_t c = next.fetch_add(1);
+            if (c >= chunks) return;
+            while (arrived.load(std::memory_order_acquire) <= c) {
+                if (failed.load()) return;
+                std::this_thread::yield();
             }
-            const hipError_t e = hipEventSynchronize(ring.ev[c % SLOTS]);
             const size_t off = c * CHUNK;
-            if (e == hipSuccess) std::memcpy(dst + off, ring.mem + (c % SLOTS) * CHUNK, std::min(CHUNK, bytes - off));
-            std::lock_guard<std::mutex> lock(m);
-            if (e != hipSuccess) err = e;
-            out[c] = 1;
-            ++done;
-            cv.notify_all();
+            std::memcpy(dst + off, ring.mem + (c % SLOTS) * CHUNK, std::min(CHUNK, bytes - off));
+            out[c].store(1, std::memory_order_release);
         }
     }
 
-    // puts every chunk on the stream, each once its slot is free
-    void issue(const char *src, hipStream_t st)
+    hipError_t run(const char *src, hipStream_t st)
     {
-        for (size_t c = 0; c < chunks; ++c) {
-            {
-                std::unique_lock<std::mutex> lock(m);
-                cv.wait(lock, [&] { return err != hipSuccess || c < SLOTS || out[c - SLOTS]; });
-                if (err != hipSuccess) return;
+        size_t issued = 0, here = 0;
+        hipError_t e = hipSuccess;
+        while (here < chunks && e == hipSuccess) {
+            if (issued < chunks && (issued < SLOTS || out[issued - SLOTS].load(std::memory_order_acquire))) {
+                const size_t off = issued * CHUNK;
+                e = hipMemcpyAsync(ring.mem + (issued % SLOTS) * CHUNK, src + off, std::min(CHUNK, bytes - off),
+                                   hipMemcpyDeviceToHost, st);
+                if (e == hipSuccess) e = hipEventRecord(ring.ev[issued % SLOTS], st);
+                if (e == hipSuccess) ++issued;
             }
-            const size_t off = c * CHUNK;
-            hipError_t e = hipMemcpyAsync(ring.mem + (c % SLOTS) * CHUNK, src + off, std::min(CHUNK, bytes - off),
-                                          hipMemcpyDeviceToHost, st);
-            if (e == hipSuccess) e = hipEventRecord(ring.ev[c % SLOTS], st);
-            std::lock_guard<std::mutex> lock(m);
-            if (e != hipSuccess) err = e;
-            else issued = c + 1;
-            cv.notify_all();
-            if (e != hipSuccess) return;
+            if (e == hipSuccess && here < issued) {
+                const hipError_t q = hipEventQuery(ring.ev[here % SLOTS]);
+                if (q == hipSuccess) arrived.store(++here, std::memory_order_release);
+                else if (q != hipErrorNotReady) e = q;
+            }
+            if (here < issued && issued == chunks) std::this_thread::yield();
         }
+        if (e != hipSuccess) failed.store(true);
+        return e;
     }
 };
 
@@ -159,6 +157,12 @@ int copy_to_host(cfdx_ctx *ctx, void *dst, const void *src, size_t bytes, const 
         CFDX_HIP(hipStreamSynchronize(ctx->stream), what);
         return CFDX_OK;
     }
+    // the work queued so far may take long: it is waited for asleep, before the threads start to spin
+    const hipError_t ready = hipStreamSynchronize(ctx->stream);
+    if (ready != hipSuccess) {
+        ring_give(ring);
+        return hip_fail(ready, what);
+    }
     Copy c(*ring, dst, bytes);
     std::vector<std::thread> threads;
     try {
@@ -173,12 +177,12 @@ int copy_to_host(cfdx_ctx *ctx, void *dst, const void *src, size_t bytes, const 
         CFDX_HIP(hipStreamSynchronize(ctx->stream), what);
         return CFDX_OK;
     }
-    c.issue((const char *)src, ctx->stream);
+    const hipError_t e = c.run((const char *)src, ctx->stream);
     for (auto &t : threads) t.join();
-    if (c.err != hipSuccess) {
+    if (e != hipSuccess) {
         (void)hipStreamSynchronize(ctx->stream);   // no copy into the ring is left when it is given back
         ring_give(ring);
-        return hip_fail(c.err, what);
+        return hip_fail(e, what);
     }
     ring_give(ring);
     return CFDX_OK;
