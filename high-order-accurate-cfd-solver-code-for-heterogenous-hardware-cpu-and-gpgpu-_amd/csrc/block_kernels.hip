@@ -774,22 +774,30 @@ __global__ void __launch_bounds__(TX *TY) k_update(const BlockDev *__restrict__ 
     each_tile<LOOP>(all, tile);
 }
 
-// maxima over the per-wave monitor values: out[0..2] = max |du|, |dv|, |de|
-__global__ void __launch_bounds__(256) k_mon_reduce(const double *__restrict__ mon, uint32_t count, double *__restrict__ out)
+// maxima over the per-wave monitor values: out[0..2] = max |du|, |dv|, |de|; one workgroup, four triples of
+// each thread in flight (bound by memory latency)
+constexpr int MON_THREADS = 1024;
+__global__ void __launch_bounds__(MON_THREADS) k_mon_reduce(const double *__restrict__ mon, uint32_t count, double *__restrict__ out)
 {
-    __shared__ double sh[3][256];
-    double a = 0.0, b = 0.0, c = 0.0;
-    for (uint32_t q = threadIdx.x; q < count; q += 256) {
-        a = fmax(a, mon[3 * q]); b = fmax(b, mon[3 * q + 1]); c = fmax(c, mon[3 * q + 2]);
+    __shared__ double sh[3][MON_THREADS / 64];
+    double m[3] = {0.0, 0.0, 0.0};
+#pragma unroll 4
+    for (uint32_t q = threadIdx.x; q < count; q += MON_THREADS) {
+#pragma unroll
+        for (int r = 0; r < 3; ++r) m[r] = fmax(m[r], mon[3 * (size_t)q + r]);
     }
-    sh[0][threadIdx.x] = a; sh[1][threadIdx.x] = b; sh[2][threadIdx.x] = c;
+#pragma unroll
+    for (int r = 0; r < 3; ++r) {
+#pragma unroll
+        for (int o = 32; o > 0; o >>= 1) m[r] = fmax(m[r], __shfl_xor(m[r], o));
+        if ((threadIdx.x & 63) == 0) sh[r][threadIdx.x / 64] = m[r];
+    }
     __syncthreads();
-    for (int o = 128; o > 0; o >>= 1) {
-        if ((int)threadIdx.x < o)
-            for (int r = 0; r < 3; ++r) sh[r][threadIdx.x] = fmax(sh[r][threadIdx.x], sh[r][threadIdx.x + o]);
-        __syncthreads();
+    if (threadIdx.x < 3) {
+        double x = 0.0;
+        for (int w = 0; w < MON_THREADS / 64; ++w) x = fmax(x, sh[threadIdx.x][w]);
+        out[threadIdx.x] = x;
     }
-    if (threadIdx.x < 3) out[threadIdx.x] = sh[threadIdx.x][0];
 }
 
 // owned node o (i-fastest over ni x nj x nk) -> stored index
@@ -1268,7 +1276,7 @@ void prims(const BlockDev &B, int precision, hipStream_t st, double *out)
 
 void monitor_reduce(const double *mon, uint32_t count, double *out, hipStream_t st)
 {
-    hipLaunchKernelGGL(k_mon_reduce, dim3(1), dim3(256), 0, st, mon, count, out);
+    hipLaunchKernelGGL(k_mon_reduce, dim3(1), dim3(MON_THREADS), 0, st, mon, count, out);
 }
 
 uint32_t tiles_of(const BlockDev &B, int kind, const TileCfg &cfg)
