@@ -580,8 +580,8 @@ struct FluxTotals {
 };
 
 template <typename S, bool VISC, int K>
-__global__ void __launch_bounds__(256, 4) k_flux(const BlockDev *__restrict__ blks, FluxTotals T, uint32_t nblk, uint32_t slots,
-                                                 int mode, uint32_t shell_tiles)
+__global__ void __launch_bounds__(256, 4) k_flux(const BlockDev *__restrict__ blks, FluxTotals T, uint32_t nblk, int mode,
+                                                 uint32_t shell_tiles)
 {
     constexpr int IA = FACE_I_TILES[0][0], IB = FACE_I_TILES[0][1], JA = FACE_JK_TILES[0][0], JB = FACE_JK_TILES[0][1];
     constexpr int TX = NODE_TILES[0][0], TY = NODE_TILES[0][1];
@@ -1094,34 +1094,49 @@ void face_jk(const LaunchList &L, hipStream_t st)
     }
 }
 
-template <typename S>
-void launch_flux(const LaunchList &L, int mode, hipStream_t st, bool any_visc)
+// The grid of k_flux over a list: every kind's tiles per XCD rounded up to the same whole number of chunks. A
+// launch holds fewer than 2^32 threads; lists past that (thin blocks of tens of millions of nodes, whose
+// tiles of 256 points are nearly empty) run the kernels apart.
+constexpr uint64_t MAX_GRID = ((uint64_t)1 << 32) / 256 - 1;
+struct FluxGrid {
+    uint32_t chunk, shell_tiles;
+    uint64_t wgs;
+};
+FluxGrid flux_grid(const LaunchList &L, bool any_visc)
 {
-    FluxTotals T;
     uint32_t most = 0;
-    for (int q = 0; q < 4; ++q) {
-        T.prefix[q] = L.prefix[q];
-        T.total[q] = L.total[q];
-        if (q > 0 || any_visc) most = std::max(most, L.total[q]);
-    }
-    uint32_t slots = (most + 7) / 8;
-    T.chunk = std::min(FLUX_CHUNK, slots);
-    slots = (slots + T.chunk - 1) / T.chunk * T.chunk;
-    const uint32_t shell_tiles = L.bc_face && any_visc ? L.shell_tiles : 0u;
-    const dim3 g(8 * (any_visc ? 4u : 3u) * slots + ((L.nblk * shell_tiles + 7) & ~7u));
-    auto go = [&](auto kernel) {
-        hipLaunchKernelGGL(kernel, g, dim3(256), 0, st, L.blks, T, L.nblk, slots, mode, shell_tiles);
-    };
-    if (!any_visc) go(k_flux<S, false, LIST_PLAIN>);   // the sweeps alone take the blocks' own switch
-    else if (L.bc_face) go(k_flux<S, true, LIST_BOUNDED>);
-    else if (L.stream) go(k_flux<S, true, LIST_STREAM>);
-    else go(k_flux<S, true, LIST_PLAIN>);
+    for (int q = any_visc ? 0 : 1; q < 4; ++q) most = std::max(most, L.total[q]);
+    FluxGrid g;
+    const uint32_t share = most / 8 + (most % 8 != 0);
+    g.chunk = std::max(std::min(FLUX_CHUNK, share), 1u);
+    const uint64_t slots = (uint64_t)(share + g.chunk - 1) / g.chunk * g.chunk;
+    g.shell_tiles = L.bc_face && any_visc ? L.shell_tiles : 0u;
+    g.wgs = (uint64_t)8 * (any_visc ? 4 : 3) * slots + (((uint64_t)L.nblk * g.shell_tiles + 7) & ~(uint64_t)7);
+    return g;
 }
 
 bool stage_forks(const LaunchList &L, const Overlap *ov)
 {
     const TileCfg &t = L.tiles;
-    return ov && (L.grid_cap || t.face[0] || t.face[1] || t.face[2] || t.node);
+    return ov && (L.grid_cap || t.face[0] || t.face[1] || t.face[2] || t.node || flux_grid(L, true).wgs > MAX_GRID);
+}
+
+template <typename S>
+void launch_flux(const LaunchList &L, int mode, hipStream_t st, bool any_visc)
+{
+    const FluxGrid fg = flux_grid(L, any_visc);
+    FluxTotals T;
+    for (int q = 0; q < 4; ++q) {
+        T.prefix[q] = L.prefix[q];
+        T.total[q] = L.total[q];
+    }
+    T.chunk = fg.chunk;
+    const dim3 g((uint32_t)fg.wgs);
+    auto go = [&](auto kernel) { hipLaunchKernelGGL(kernel, g, dim3(256), 0, st, L.blks, T, L.nblk, mode, fg.shell_tiles); };
+    if (!any_visc) go(k_flux<S, false, LIST_PLAIN>);   // the sweeps alone take the blocks' own switch
+    else if (L.bc_face) go(k_flux<S, true, LIST_BOUNDED>);
+    else if (L.stream) go(k_flux<S, true, LIST_STREAM>);
+    else go(k_flux<S, true, LIST_PLAIN>);
 }
 
 template <typename S>
