@@ -117,14 +117,17 @@ __global__ void k_opcount(Ops *out, ViscParams vp)
         take(out[2]);
     }
     {
-        Cnt dU[5][3], U[5], m[9], KS[3], fv[3][5];
-        for (int c = 0; c < 5; ++c) {
-            U[c] = in(1.0 + 0.1 * c);
-            for (int d = 0; d < 3; ++d) dU[c][d] = in(0.01 * (c + 1) * (d + 2));
-        }
+        Cnt U[5], m[9], sk[3], G[4][3] = {}, fv[3][5];
+        for (int c = 0; c < 5; ++c) U[c] = in(1.0 + 0.1 * c);
         for (int c = 0; c < 9; ++c) m[c] = in(c % 4 == 0 ? 1.0 : 0.05);
-        for (int d = 0; d < 3; ++d) KS[d] = in(1e-4 * (d + 1));
-        viscous_node(dU, U, in(0.9), in(0.1), in(0.05), m, in(1.2), KS, vp, fv);
+        const NodeRatios<Cnt> nr = node_ratios(U);
+        for (int d = 0; d < 3; ++d) {
+            Cnt dU[5];
+            for (int c = 0; c < 5; ++c) dU[c] = in(0.01 * (c + 1) * (d + 2));
+            add_gradient(dU, nr, m[3 * d], m[3 * d + 1], m[3 * d + 2], G);
+            sk[d] = in(1e-2 * (d + 1));
+        }
+        viscous_fluxes(G, U, nr, in(0.9), in(0.1), in(0.05), m, in(1.2), sk, vp, fv);
         take(out[3]);
     }
 }
@@ -135,8 +138,8 @@ __global__ void k_opcount(Ops *out, ViscParams vp)
 // Operations written out in double in the node kernels (block_kernels.hip), counted by hand:
 //   visc_node: per direction and component the central difference (8 (f+1 - f-1) - (f+2 - f-2))
 //     / 12 = 5 operations (75 for 5 components x 3 directions); per direction the MTS
-//     scale-similarity term a = U/U0 - (weighted mean)/(weighted mean), a^2 = 14 operations
-//     (42); 1 / U0 = 1; the node velocity U_m / U_0 away from the sides = 3 (total 121).
+//     scale-similarity term U/U0 - (weighted mean) * 1/(weighted mean) = 14 operations (42);
+//     1 / U0 = 1; the node velocity U_m / U_0 away from the sides = 3 (total 121).
 //   update_node: face-flux differences 2 x 15 = 30; viscous divergence 4 components x 3
 //     directions x (5 + 1) = 72; RK stage 5 x {2, 6, 6} (modes 0, 1, 2; mean 4.67) = 23.3 per
 //     stage; primitive recovery (1/det, rho, 1/rho, u v w, e, p) = 20; at the last stage the RK

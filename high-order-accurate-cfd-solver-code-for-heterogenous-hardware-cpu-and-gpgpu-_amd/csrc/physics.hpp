@@ -570,23 +570,6 @@ __device__ __forceinline__ T viscous_fluxes(const T (&G)[4][3], const T (&U)[5],
     return mu;
 }
 
-// The same from all differences at once. KS[3]: the scale-similarity terms, squared.
-template <typename T>
-__device__ __forceinline__ T viscous_node(const T (&dU)[5][3], const T (&U)[5], T u, T v, T w, const T (&m)[9], T D,
-                                          const T (&KS)[3], const ViscParams &vp, T (&fvis)[3][5])
-{
-    const NodeRatios<T> n = node_ratios(U);
-    T G[4][3] = {};
-    T sk[3];
-#pragma unroll
-    for (int d = 0; d < 3; ++d) {
-        const T dUd[5] = {dU[0][d], dU[1][d], dU[2][d], dU[3][d], dU[4][d]};
-        add_gradient(dUd, n, m[3 * d], m[3 * d + 1], m[3 * d + 2], G);
-        sk[d] = sqrt_(KS[d]);
-    }
-    return viscous_fluxes(G, U, n, u, v, w, m, D, sk, vp, fvis);
-}
-
 // One-direction derivative of Viscous.cl:285-435 (weno_form = false) or Weno.cl:2732-2856
 // (weno_form = true) selected by the loc codes; f[0..6] at offsets -3..+3. Branches are
 // taken in source order, a later match overwriting an earlier one; with no match the
