@@ -9,10 +9,11 @@
 #include <algorithm>
 #include <atomic>
 #include <cstring>
+#include <exception>
 #include <mutex>
-#include <system_error>
+#include <new>
 #include <thread>
-#include <vector>
+#include <utility>
 
 #include "ctx.hpp"
 
@@ -38,20 +39,17 @@ struct Ring {
 };
 
 std::mutex rings_mutex;
-std::vector<Ring *> rings;   // not in use
+Ring *rings[KEPT] = {};   // not in use
 
 Ring *ring_take(int device)
 {
     {
         std::lock_guard<std::mutex> lock(rings_mutex);
-        for (size_t q = 0; q < rings.size(); ++q)
-            if (rings[q]->device == device) {
-                Ring *r = rings[q];
-                rings.erase(rings.begin() + (long)q);
-                return r;
-            }
+        for (Ring *&kept : rings)
+            if (kept && kept->device == device) return std::exchange(kept, nullptr);
     }
-    Ring *r = new Ring;
+    Ring *r = new (std::nothrow) Ring;
+    if (!r) return nullptr;
     r->device = device;
     hipError_t e = hipHostMalloc((void **)&r->mem, CHUNK * SLOTS, hipHostMallocDefault);
     for (auto &v : r->ev)
@@ -66,10 +64,11 @@ void ring_give(Ring *r)
 {
     {
         std::lock_guard<std::mutex> lock(rings_mutex);
-        if (rings.size() < KEPT) {
-            rings.push_back(r);
-            return;
-        }
+        for (Ring *&kept : rings)
+            if (!kept) {
+                kept = r;
+                return;
+            }
     }
     delete r;
 }
@@ -90,12 +89,9 @@ struct Copy {
     size_t bytes, chunks;
     std::atomic<size_t> arrived{0}, next{0};
     std::atomic<bool> failed{false};
-    std::vector<std::atomic<char>> out;   // per chunk: copied out
+    std::atomic<size_t> out[SLOTS] = {};   // per slot: chunks copied out of it
 
-    Copy(Ring &r, void *d, size_t n)
-        : ring(r), dst((char *)d), bytes(n), chunks((n + CHUNK - 1) / CHUNK), out(chunks)
-    {
-    }
+    Copy(Ring &r, void *d, size_t n) : ring(r), dst((char *)d), bytes(n), chunks((n + CHUNK - 1) / CHUNK) {}
 
     void work()
     {
@@ -108,7 +104,7 @@ struct Copy {
             }
             const size_t off = c * CHUNK;
             std::memcpy(dst + off, ring.mem + (c % SLOTS) * CHUNK, std::min(CHUNK, bytes - off));
-            out[c].store(1, std::memory_order_release);
+            out[c % SLOTS].store(c / SLOTS + 1, std::memory_order_release);
         }
     }
 
@@ -117,7 +113,7 @@ struct Copy {
         size_t issued = 0, here = 0;
         hipError_t e = hipSuccess;
         while (here < chunks && e == hipSuccess) {
-            if (issued < chunks && (issued < SLOTS || out[issued - SLOTS].load(std::memory_order_acquire))) {
+            if (issued < chunks && out[issued % SLOTS].load(std::memory_order_acquire) == issued / SLOTS) {
                 const size_t off = issued * CHUNK;
                 e = hipMemcpyAsync(ring.mem + (issued % SLOTS) * CHUNK, src + off, std::min(CHUNK, bytes - off),
                                    hipMemcpyDeviceToHost, st);
@@ -140,10 +136,10 @@ struct Copy {
 
 void staging_trim()
 {
-    std::vector<Ring *> gone;
+    Ring *gone[KEPT];
     {
         std::lock_guard<std::mutex> lock(rings_mutex);
-        gone.swap(rings);
+        for (size_t q = 0; q < KEPT; ++q) gone[q] = std::exchange(rings[q], nullptr);
     }
     for (Ring *r : gone) delete r;
 }
@@ -164,21 +160,21 @@ int copy_to_host(cfdx_ctx *ctx, void *dst, const void *src, size_t bytes, const 
         return hip_fail(ready, what);
     }
     Copy c(*ring, dst, bytes);
-    std::vector<std::thread> threads;
+    std::thread threads[THREADS];
+    unsigned started = 0;
     try {
-        threads.reserve(nt);
-        for (unsigned q = 0; q < nt; ++q) threads.emplace_back([&c] { c.work(); });
+        for (; started < nt; ++started) threads[started] = std::thread([&c] { c.work(); });
     } catch (const std::exception &) {
         // fewer threads than asked for: those that started do the work
     }
-    if (threads.empty()) {
+    if (!started) {
         ring_give(ring);
         CFDX_HIP(hipMemcpyAsync(dst, src, bytes, hipMemcpyDeviceToHost, ctx->stream), what);
         CFDX_HIP(hipStreamSynchronize(ctx->stream), what);
         return CFDX_OK;
     }
     const hipError_t e = c.run((const char *)src, ctx->stream);
-    for (auto &t : threads) t.join();
+    for (unsigned q = 0; q < started; ++q) threads[q].join();
     if (e != hipSuccess) {
         (void)hipStreamSynchronize(ctx->stream);   // no copy into the ring is left when it is given back
         ring_give(ring);
