@@ -110,18 +110,44 @@ int64_t stored_nodes(const cfdx_block_desc *d)
     return (int64_t)dims[0] * dims[1] * dims[2];
 }
 
+// How the arrays of a block lie in memory: the stored row pitch in nodes, the nodes before a stored row's first
+// ghost, and the length of an array.
+struct RowLayout {
+    int pitch, lead;
+    int64_t n;
+};
+
+// In a block that streams (STREAM_BYTES) the owned nodes of a row begin and end on 64-byte pieces of the flux type (8
+// doubles, 16 floats): the pitch is rounded up, and a bounded direction's ghosts are preceded by as many nodes as
+// complete a piece with them. Rows end to end, a wave's 64 nodes touch a piece more and share two with their
+// neighbours. FP64, us a step end to end and so: 385x128x32 1286 and 1239, 262x128x32 881 and 848; mixed: 385x128x32 767
+// and 703; C-grid 384x128x32 FP64 1332 and 1306, mixed 859 and 843. Blocks that the cache holds are better end to end
+// (C-grids 192x96x24 FP64 372 and 379, 128x64x16 mixed 112 and 116), and so are short rows, where the pieces cost more
+// than a twelfth of the memory.
+RowLayout row_layout(const cfdx_block_desc *d, bool aligned = true)
+{
+    int dims[3], off[3];
+    padded_dims(d, dims, off);
+    const int unit = (int)(64 / flux_size(d->precision)), pitch = (dims[0] + unit - 1) / unit * unit;
+    const int64_t rows = (int64_t)dims[1] * dims[2];
+    const bool streams = cfdx::blk::stage_bytes((uint64_t)rows * dims[0], d->precision == CFDX_MIXED) > cfdx::blk::STREAM_BYTES;
+    if (!aligned || !streams || (pitch - dims[0]) * 12 > dims[0] || rows * pitch >= (int64_t(1) << 29))
+        return {dims[0], 0, rows * dims[0]};
+    return {pitch, off[0] ? unit - off[0] : 0, rows * pitch};
+}
+
 // the block descriptor and the single-block prefix table after the arrays
 size_t tail_bytes() { return ((sizeof(BlockDev) + 255) / 256) * 256 + 256; }
 
-int64_t bytes_of(const cfdx_block_desc *d)
+int64_t bytes_of(const cfdx_block_desc *d, const RowLayout &R)
 {
-    const int64_t n = stored_nodes(d);
+    const int64_t n = R.n;
     // 33 double arrays (geometry 22, U0 5, Us 5, mu 1) + 32 flux-type arrays (P 5, Fv 12, FH 15)
     // + in a mixed block float copies of the 22 geometry arrays + one byte of loc code per node
-    // for a bounded block
+    // for a bounded block; 256 bytes of slack for the lead of each of the three types
     const int64_t codes = d->periodic == 7 ? 0 : ((n + 255) / 256) * 256;
     const int64_t geo32 = d->precision == CFDX_MIXED ? 22 * 4 : 0;
-    return n * (33 * 8 + 32 * (int64_t)flux_size(d->precision) + geo32) + codes + 256;
+    return n * (33 * 8 + 32 * (int64_t)flux_size(d->precision) + geo32) + codes + 4 * 256;
 }
 
 int check_desc(const cfdx_block_desc *d)
@@ -152,16 +178,16 @@ int check_desc(const cfdx_block_desc *d)
 
 // loc codes of a bounded block: 0 interior, 1 node on a side (boundary condition node), 100 ghost;
 // a ghost across a wake cut stands for its mirror node and takes the mirror's code
-std::vector<uint8_t> loc_codes(const cfdx_block_desc *d)
+std::vector<uint8_t> loc_codes(const cfdx_block_desc *d, int pitch)
 {
     int dims[3], off[3];
     padded_dims(d, dims, off);
     const int n[3] = {d->ni, d->nj, d->nk};
     const bool cut = !(d->periodic & 2) && d->bc[2] == CFDX_BC_WALL_CUT;
     auto wall_col = [&](int i) { return i >= d->cut_i0 && i <= d->cut_i1; };
-    std::vector<uint8_t> c((size_t)dims[0] * dims[1] * dims[2], 100);
+    std::vector<uint8_t> c((size_t)pitch * dims[1] * dims[2], 100);
     auto at = [&](int i, int j, int k) {
-        return (size_t)(i + off[0]) + (size_t)dims[0] * ((size_t)(j + off[1]) + (size_t)dims[1] * (size_t)(k + off[2]));
+        return (size_t)(i + off[0]) + (size_t)pitch * ((size_t)(j + off[1]) + (size_t)dims[1] * (size_t)(k + off[2]));
     };
     for (int k = 0; k < n[2]; ++k)
         for (int j = 0; j < n[1]; ++j)
@@ -426,7 +452,7 @@ extern "C" int64_t cfdx_block_bytes(const cfdx_block_desc *d)
     if (!d) return cfdx::fail(CFDX_E_INVALID, "block_bytes: null descriptor");
     const int rc = check_desc(d);
     if (rc != CFDX_OK) return rc;
-    return bytes_of(d) + (int64_t)tail_bytes();
+    return bytes_of(d, row_layout(d)) + (int64_t)tail_bytes();
 }
 
 extern "C" int cfdx_block_padded(const cfdx_block_desc *desc, int32_t dims[3], int32_t off[3])
@@ -444,13 +470,18 @@ extern "C" int cfdx_block_create(cfdx_ctx *ctx, const cfdx_block_desc *desc, cfd
     if (!desc || !out) return cfdx::fail(CFDX_E_INVALID, "block_create: null argument");
     *out = nullptr;
     CFDX_TRY(check_desc(desc));
-    const long long n = stored_nodes(desc);
+    RowLayout R = row_layout(desc);
     cfdx_block *b = new cfdx_block;
     b->ctx = ctx;
     cfdx::ctx_retain(ctx);
     b->desc = *desc;
-    b->bytes = (size_t)bytes_of(desc);
+    b->bytes = (size_t)bytes_of(desc, R);
     b->mem = cfdx::pool_take(ctx->device, b->bytes + tail_bytes(), &b->alloc);
+    if (!b->mem) {   // a block that only fits with its rows end to end
+        R = row_layout(desc, false);
+        b->bytes = (size_t)bytes_of(desc, R);
+        b->mem = cfdx::pool_take(ctx->device, b->bytes + tail_bytes(), &b->alloc);
+    }
     if (!b->mem) {
         cfdx::ctx_release(ctx);
         delete b;
@@ -467,11 +498,11 @@ extern "C" int cfdx_block_create(cfdx_ctx *ctx, const cfdx_block_desc *desc, cfd
         return cfdx::hip_fail(e, "block_create");
     }
     BlockDev &B = b->B;
-    B.ni = desc->ni; B.nj = desc->nj; B.nk = desc->nk; B.n = (uint32_t)n;
+    B.ni = desc->ni; B.nj = desc->nj; B.nk = desc->nk; B.n = (uint32_t)R.n;
     {
         int dims[3];
         padded_dims(desc, dims, B.off);
-        B.pi = dims[0];
+        B.pi = R.pitch;
         B.pj = dims[1];
         for (int q = 0; q < 6; ++q) B.bc[q] = desc->bc[q];
         B.cut_i0 = desc->cut_i0;
@@ -479,7 +510,10 @@ extern "C" int cfdx_block_create(cfdx_ctx *ctx, const cfdx_block_desc *desc, cfd
         B.cos_aoa = std::cos(desc->aoa);
         B.sin_aoa = std::sin(desc->aoa);
     }
-    char *p = (char *)b->mem;
+    const size_t n = (size_t)R.n;
+    // each type's arrays one after the other, the first R.lead nodes past a multiple of 64 bytes
+    auto start = [&](char *q, size_t size) { return (char *)(((uintptr_t)q + 63) & ~(uintptr_t)63) + R.lead * size; };
+    char *p = start((char *)b->mem, sizeof(double));
     auto takeD = [&]() { double *r = (double *)p; p += n * sizeof(double); return r; };
     auto takeS = [&]() { void *r = p; p += n * flux_size(desc->precision); return r; };
     B.det = takeD();
@@ -489,19 +523,21 @@ extern "C" int cfdx_block_create(cfdx_ctx *ctx, const cfdx_block_desc *desc, cfd
     for (auto &a : B.U0) a = takeD();
     for (auto &a : B.Us) a = takeD();
     B.mu = takeD();
+    p = start(p, flux_size(desc->precision));
     for (auto &a : B.P) a = takeS();
     for (auto &r : B.Fv) for (auto &a : r) a = takeS();
     for (auto &r : B.FH) for (auto &a : r) a = takeS();
     B.geo32 = nullptr;
     if (desc->precision == CFDX_MIXED) {
+        p = start(p, sizeof(float));
         B.geo32 = (const float *)p;
-        p += (size_t)22 * n * sizeof(float);
+        p += 22 * n * sizeof(float);
     }
     B.strip = 0;
     B.stream = 0;
     B.code = nullptr;
     if (desc->periodic != 7) {
-        const std::vector<uint8_t> codes = loc_codes(desc);
+        const std::vector<uint8_t> codes = loc_codes(desc, R.pitch);
         B.code = (const uint8_t *)p;
         e = hipMemcpyAsync((void *)B.code, codes.data(), codes.size(), hipMemcpyHostToDevice, ctx->stream);
         if (e == hipSuccess) e = hipStreamSynchronize(ctx->stream);
@@ -574,14 +610,16 @@ extern "C" int cfdx_block_set_geometry(cfdx_block *b, const double *det, const c
                     }
                 }
             }
-    std::vector<double> h((size_t)22 * n);
+    const size_t np = b->B.n, pitch = (size_t)b->B.pi;
+    std::vector<double> h(22 * np);
     for (long long g = 0; g < n; ++g) {
-        h[g] = det[g];
-        for (int c = 0; c < 9; ++c) h[(1 + c) * n + g] = metric[g].node[c];
+        const size_t s = (size_t)(g % ni) + pitch * (size_t)(g / ni);
+        h[s] = det[g];
+        for (int c = 0; c < 9; ++c) h[(1 + c) * np + s] = metric[g].node[c];
         for (int d = 0; d < 3; ++d)
-            for (int c = 0; c < 3; ++c) h[(10 + 3 * d + c) * n + g] = metric[g].face[2 * d][3 * d + c];
+            for (int c = 0; c < 3; ++c) h[(10 + 3 * d + c) * np + s] = metric[g].face[2 * d][3 * d + c];
         const double *dd = &deter[g].ip;
-        for (int d = 0; d < 3; ++d) h[(19 + d) * n + g] = dd[2 * d];
+        for (int d = 0; d < 3; ++d) h[(19 + d) * np + s] = dd[2 * d];
     }
     CFDX_HIP(hipMemcpyAsync((void *)b->B.det, h.data(), h.size() * 8, hipMemcpyHostToDevice, b->ctx->stream), "set_geometry copy");
     cfdx::blk::geometry_finalize(b->B, b->ctx->stream);
@@ -594,7 +632,22 @@ extern "C" int cfdx_block_set_geometry_soa(cfdx_block *b, const double *geo)
 {
     if (!b || !geo) return cfdx::fail(CFDX_E_INVALID, "set_geometry_soa: null argument");
     CFDX_TRY(enter_block(b));
-    CFDX_HIP(hipMemcpyAsync((void *)b->B.det, geo, (size_t)22 * b->B.n * 8, hipMemcpyHostToDevice, b->ctx->stream), "set_geometry_soa copy");
+    int dims[3], off[3];
+    padded_dims(&b->desc, dims, off);
+    const size_t rows = (size_t)dims[1] * dims[2], len = rows * dims[0];
+    if (b->B.pi == dims[0]) {
+        CFDX_HIP(hipMemcpyAsync((void *)b->B.det, geo, 22 * len * 8, hipMemcpyHostToDevice, b->ctx->stream), "set_geometry_soa copy");
+    } else {
+        // a few arrays at a time to the viscous node fluxes (scratch between steps), from there to their rows
+        const int some = b->B.geo32 ? 6 : 11;
+        double *tmp = (double *)(((uintptr_t)b->B.Fv[0][0] + 7) & ~(uintptr_t)7);
+        for (int a = 0; a < 22; a += some) {
+            const int c = std::min(some, 22 - a);
+            CFDX_HIP(hipMemcpyAsync(tmp, geo + a * len, c * len * 8, hipMemcpyHostToDevice, b->ctx->stream), "set_geometry_soa copy");
+            cfdx::blk::spread_rows(tmp, (double *)b->B.det + (size_t)a * b->B.n, c * rows, (uint32_t)dims[0], (uint32_t)b->B.pi, b->ctx->stream);
+            CFDX_TRY(cfdx::check_launch("k_spread_rows"));
+        }
+    }
     cfdx::blk::geometry_finalize(b->B, b->ctx->stream);
     CFDX_TRY(cfdx::check_launch("geometry_finalize"));
     // finiteness checked on the device; the counter lives in the face-flux scratch
@@ -768,7 +821,7 @@ extern "C" int cfdx_block_rhs_noalloc(cfdx_block *b, const cfdx_params *params, 
 {
     if (!b || !L_dev) return cfdx::fail(CFDX_E_INVALID, "block_rhs_noalloc: null argument");
     CFDX_TRY(check_params(params));
-    const long long n = b->B.n;
+    const long long n = stored_nodes(&b->desc);
     if (n > RHS_NOALLOC_NODES)
         return cfdx::fail(CFDX_E_CAPACITY,
                           "block_rhs_noalloc: %lld stored nodes exceed the limit of %lld, 64 MiB of results "

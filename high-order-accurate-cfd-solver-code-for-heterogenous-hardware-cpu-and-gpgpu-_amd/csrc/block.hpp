@@ -38,8 +38,8 @@ struct TileCfg {
 // P, Fv and FH hold the flux type (double or float); everything else is double.
 struct BlockDev {
     int ni, nj, nk;             // owned nodes
-    uint32_t n;                 // stored (padded) nodes: the length of every array
-    int pi, pj;                 // padded sizes along i and j (index strides)
+    uint32_t n;                 // the length of every array
+    int pi, pj;                 // stored rows: their pitch, and how many to a plane (index strides)
     int off[3];                 // ghost layers before the first owned node along i, j, k (3, or 0 if periodic)
     const uint8_t *code;        // bounded blocks: per stored node 0 interior, 1 boundary node, 100 ghost
     int bc[6];                  // side conditions (CFDX_BC_*) of i-, i+, j-, j+, k-, k+
@@ -108,27 +108,30 @@ __host__ __device__ inline uint32_t shell_wave(const BlockDev &B, uint32_t s, ui
     return s < rows ? 4 * s + w : 4 * rows + (s - rows) * (shell_column_tile(B) / 64) + w;
 }
 
-// How the node kernels of a list access memory.
-enum : int {
-    LIST_PLAIN,     // periodic blocks
-    LIST_STREAM,    // periodic blocks, non-temporal accesses to what a kernel touches once
-    LIST_BOUNDED    // some block has a bounded direction: shell tiles beside the node tiles
-};
+// How the kernels of a list go over its blocks: with shell tiles beside the node tiles if some block has a bounded
+// direction, and with non-temporal accesses to what a kernel touches once if the list streams.
+enum : int { LIST_PLAIN, LIST_STREAM, LIST_BOUNDED, LIST_BOUNDED_STREAM };
+constexpr bool list_streams(int k) { return (k & 1) != 0; }
+constexpr bool list_bounded(int k) { return (k & 2) != 0; }
 
 // Bytes of a stored node that a stage reads and writes (FP64: 22 geometry arrays, U0, Us, P, Fv, FH; mixed:
 // the float geometry, det, U0, Us and the 32 float arrays).
-inline uint64_t stage_bytes(const BlockDev &B) { return (uint64_t)B.n * (B.geo32 ? 304 : 512); }
+inline uint64_t stage_bytes(uint64_t n, bool mixed) { return n * (mixed ? 304 : 512); }
+inline uint64_t stage_bytes(const BlockDev &B) { return stage_bytes(B.n, B.geo32 != nullptr); }
 
-// Whether a block's rows take non-temporal accesses well: whole 64-byte pieces. With others the hint
-// drops lines that the neighbouring rows still need (FP64 161x131x127 1.5 % slower, 255x200x160 2.5 %, mixed 4 and
-// 5 %; the C-grids, rows of ni + 6 nodes, 14 % at 128x64x16 to 1 % at 384x128x32).
-inline bool rows_stream(const BlockDev &B) { return !B.code && (uint64_t)B.pi * (B.geo32 ? 4 : 8) % 64 == 0; }
-
-// The size past which a list of blocks streams: below it a stage's arrays stay in the 256 MB last-level
+// The size past which a block or a list streams: below it a stage's arrays stay in the 256 MB last-level
 // cache (and the L2s) from one stage to the next, and the hint gives that up. FP64: 64^3 197 us a step
 // with the hint, 177 without; 80^3 (262 MB) 449 and 391; 96^3 (453 MB) 708 and 731; 256^3 12.88 and 13.09 ms.
 // Mixed: 64^3 125 and 112 us, 96^3 (269 MB) 400 and 369, 112^3 (427 MB) 622 and 643, 128^3 889 and 937.
-constexpr uint64_t STREAM_BYTES = (uint64_t)320 << 20;
+// C-grids, FP64: 192x96x24 (288 MB) 423 and 378, 256x128x32 (575 MB) 889 and 904, 384x128x32 1284 and 1306; mixed:
+// 256x128x32 (341 MB) 588 and 572, 384x128x32 (508 MB) 829 and 843.
+// Past it, rows that are not whole 64-byte pieces cost as well (row_layout): below, the pieces that two rows share
+// are found in the cache, and end to end the arrays take less of it.
+constexpr uint64_t STREAM_BYTES = (uint64_t)384 << 20;
+
+// Whether a block's rows take non-temporal accesses: whole 64-byte pieces. With others the hint drops lines that
+// the neighbouring rows still need (FP64 161x131x127 1.5 % slower, 255x200x160 2.5 %, mixed 4 and 5 %).
+inline bool rows_stream(const BlockDev &B) { return (uint64_t)B.pi * (B.geo32 ? 4 : 8) % 64 == 0; }
 inline bool streams_past_cache(uint64_t bytes, bool rows) { return rows && bytes > STREAM_BYTES; }
 
 // One launch over a list of blocks.
@@ -143,7 +146,7 @@ struct LaunchList {
     uint32_t bc_face_d[3] = {};       // the same per direction (0: no block bounded in that direction)
     uint32_t bc_planes = 0;           // largest nk of the blocks bounded along i
     uint32_t shell_tiles = 0;         // most shell tiles of a bounded block
-    bool stream = false;              // periodic blocks past the cache: non-temporal accesses
+    bool stream = false;              // past the cache: non-temporal accesses
     double *Lout = nullptr;           // mode 3 (a single block): the right-hand side, 5 x owned nodes
 };
 
@@ -167,6 +170,8 @@ bool stage_forks(const LaunchList &L, const Overlap *ov);
 void geometry_finalize(const BlockDev &B, hipStream_t st);
 // P and U0 of the owned nodes from double primitives staged component-major in owned order
 void base(const BlockDev &B, int precision, hipStream_t st, const double *stage);
+// rows of w doubles, end to end in src, to rows of a pitch in dst
+void spread_rows(const double *src, double *dst, size_t rows, uint32_t w, uint32_t pitch, hipStream_t st);
 void prims(const BlockDev &B, int precision, hipStream_t st, double *out);
 // *count += the number of workgroups that found a value that is not finite in p[0..n)
 void count_nonfinite(const double *p, size_t n, unsigned *count, hipStream_t st);

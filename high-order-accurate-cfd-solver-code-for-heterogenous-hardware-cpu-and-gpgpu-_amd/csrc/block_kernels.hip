@@ -359,7 +359,7 @@ constexpr int VISC_LDS = TY >= 4 ? 5 * (TY + 4) * (TX + 4) : 1;
 template <typename S, int TX, int TY, int K>
 __device__ __forceinline__ void visc_tile(const BlockDev &B, uint32_t lt, int mode, double *plane)
 {
-    constexpr bool BND = K == LIST_BOUNDED, NT = K == LIST_STREAM;
+    constexpr bool BND = list_bounded(K), NT = list_streams(K);
     constexpr int PC = TX + 4, PR = TY + 4;
     int i0, j0, k;
     node_tile(B, lt, TX, TY, i0, j0, k);
@@ -400,11 +400,11 @@ __device__ __forceinline__ void visc_shell_tile(const BlockDev *__restrict__ blk
 // blocks, nblk x shell_tiles shell tiles of TX * TY shell nodes each (block = id / shell_tiles),
 // dispatched last in plain order so that they spread over the XCDs at the end of the launch.
 template <typename S, int TX, int TY, int K, bool LOOP>
-__global__ void __launch_bounds__(TX *TY, ((TY >= 4 && !(LOOP && K == LIST_BOUNDED)) || sizeof(S) == 4 ? 4 : 3))
+__global__ void __launch_bounds__(TX *TY, ((TY >= 4 && !(LOOP && list_bounded(K))) || sizeof(S) == 4 ? 4 : 3))
     k_visc(const BlockDev *__restrict__ blks, const uint32_t *__restrict__ prefix, uint32_t nblk, uint32_t total, int mode,
            uint32_t shell_tiles)
 {
-    constexpr bool BND = K == LIST_BOUNDED;
+    constexpr bool BND = list_bounded(K);
     __shared__ double plane[VISC_LDS<TX, TY>];
     const uint32_t all = total + (BND ? nblk * shell_tiles : 0u);
     auto tile = [&](uint32_t wg) {
@@ -588,7 +588,7 @@ __global__ void __launch_bounds__(256, 4) k_flux(const BlockDev *__restrict__ bl
     constexpr int L0 = VISC ? VISC_LDS<TX, TY> * (int)sizeof(double) : 0, L1 = FACE_LDS<S, IA, IB> * (int)sizeof(S),
                   L2 = FACE_LDS<S, JA, JB> * (int)sizeof(S);
     __shared__ __align__(16) char lds[L0 > L1 ? (L0 > L2 ? L0 : L2) : (L1 > L2 ? L1 : L2)];
-    constexpr bool BND = K == LIST_BOUNDED;
+    constexpr bool BND = list_bounded(K);
     constexpr uint32_t KINDS = VISC ? 4 : 3;
     uint32_t wg = blockIdx.x;
     if (VISC && BND) {
@@ -743,7 +743,7 @@ __global__ void __launch_bounds__(TX *TY) k_update(const BlockDev *__restrict__ 
                                                    uint32_t nblk, uint32_t total, int mode, uint32_t shell_tiles,
                                                    double *Lout)
 {
-    constexpr bool BND = K == LIST_BOUNDED, NT = K == LIST_STREAM;
+    constexpr bool BND = list_bounded(K), NT = list_streams(K);
     const uint32_t shell = BND ? nblk * shell_tiles : 0u, first = (shell + 7) & ~7u, all = first + total;
     auto tile = [&](uint32_t wg) {
         // residual monitor of the step (Solver.cpp:546-573): |du|, |dv|, |de| against the RK base
@@ -1038,7 +1038,7 @@ void launch_node_k(const LaunchList &L, uint32_t cap, hipStream_t st, bool visc_
 {
     constexpr int TX = NODE_TILES[V][0], TY = NODE_TILES[V][1];
     static_assert(TX * TY == 256, "node tiles have 256 threads");
-    const uint32_t shell_tiles = K == LIST_BOUNDED ? L.shell_tiles : 0u;
+    const uint32_t shell_tiles = list_bounded(K) ? L.shell_tiles : 0u;
     // one workgroup per shell tile too
     const uint32_t shell = L.nblk * shell_tiles, all = L.total[0] + (visc_kernel ? shell : (shell + 7) & ~7u);
     const bool loop = cap && cap < all;
@@ -1055,7 +1055,8 @@ void launch_node_k(const LaunchList &L, uint32_t cap, hipStream_t st, bool visc_
 template <typename S, int V>
 void launch_node(const LaunchList &L, uint32_t cap, hipStream_t st, bool visc_kernel, int mode)
 {
-    if (L.bc_face) launch_node_k<S, V, LIST_BOUNDED>(L, cap, st, visc_kernel, mode);
+    if (L.bc_face && L.stream) launch_node_k<S, V, LIST_BOUNDED_STREAM>(L, cap, st, visc_kernel, mode);
+    else if (L.bc_face) launch_node_k<S, V, LIST_BOUNDED>(L, cap, st, visc_kernel, mode);
     else if (L.stream) launch_node_k<S, V, LIST_STREAM>(L, cap, st, visc_kernel, mode);
     else launch_node_k<S, V, LIST_PLAIN>(L, cap, st, visc_kernel, mode);
 }
@@ -1134,6 +1135,7 @@ void launch_flux(const LaunchList &L, int mode, hipStream_t st, bool any_visc)
     const dim3 g((uint32_t)fg.wgs);
     auto go = [&](auto kernel) { hipLaunchKernelGGL(kernel, g, dim3(256), 0, st, L.blks, T, L.nblk, mode, fg.shell_tiles); };
     if (!any_visc) go(k_flux<S, false, LIST_PLAIN>);   // the sweeps alone take the blocks' own switch
+    else if (L.bc_face && L.stream) go(k_flux<S, true, LIST_BOUNDED_STREAM>);
     else if (L.bc_face) go(k_flux<S, true, LIST_BOUNDED>);
     else if (L.stream) go(k_flux<S, true, LIST_STREAM>);
     else go(k_flux<S, true, LIST_PLAIN>);
@@ -1269,6 +1271,20 @@ __global__ void __launch_bounds__(256) k_unit_normals(double *__restrict__ geo, 
             }
         }
     }
+}
+
+__global__ void __launch_bounds__(256) k_spread_rows(const double *__restrict__ src, double *__restrict__ dst, size_t n,
+                                                     uint32_t w, uint32_t pitch)
+{
+    for (size_t q = (size_t)blockIdx.x * blockDim.x + threadIdx.x; q < n; q += (size_t)gridDim.x * blockDim.x)
+        dst[q / w * pitch + q % w] = src[q];
+}
+
+void spread_rows(const double *src, double *dst, size_t rows, uint32_t w, uint32_t pitch, hipStream_t st)
+{
+    const size_t n = rows * w;
+    const unsigned nb = (unsigned)std::min<size_t>((n + 255) / 256, 8192);
+    hipLaunchKernelGGL(k_spread_rows, dim3(nb), dim3(256), 0, st, src, dst, n, w, pitch);
 }
 
 void geometry_finalize(const BlockDev &B, hipStream_t st)

@@ -31,9 +31,10 @@ __device__ __forceinline__ void node_coords(const MapArgs &a, int ni, int nj, in
 
 __global__ void k_geom(BlockDev B, MapArgs a)
 {
-    const uint32_t g = blockIdx.x * blockDim.x + threadIdx.x;
-    if (g >= B.n) return;
-    const int i = (int)(g % (uint32_t)B.ni), j = (int)((g / (uint32_t)B.ni) % (uint32_t)B.nj), k = (int)(g / ((uint32_t)B.ni * B.nj));
+    const uint32_t o = blockIdx.x * blockDim.x + threadIdx.x, no = (uint32_t)B.ni * B.nj * B.nk;
+    if (o >= no) return;
+    const int i = (int)(o % (uint32_t)B.ni), j = (int)((o / (uint32_t)B.ni) % (uint32_t)B.nj), k = (int)(o / ((uint32_t)B.ni * B.nj));
+    const uint32_t g = (uint32_t)i + (uint32_t)B.pi * ((uint32_t)j + (uint32_t)B.nj * (uint32_t)k);
     const double w0 = 2.0 * M_PI / a.L[0], w1 = 2.0 * M_PI / a.L[1], w2 = 2.0 * M_PI / a.L[2];
     const double h0 = a.L[0] / B.ni, h1 = a.L[1] / B.nj, h2 = a.L[2] / B.nk;
     const double s1 = i * h0, s2 = j * h1, s3 = k * h2;
@@ -70,9 +71,10 @@ __device__ __forceinline__ int wrap(int i, int n) { return i < 0 ? i + n : (i >=
 // +1/2-face metrics of each direction from the node values along it (periodic wrap)
 __global__ void k_half(BlockDev B)
 {
-    const uint32_t g = blockIdx.x * blockDim.x + threadIdx.x;
-    if (g >= B.n) return;
-    const int i = (int)(g % (uint32_t)B.ni), j = (int)((g / (uint32_t)B.ni) % (uint32_t)B.nj), k = (int)(g / ((uint32_t)B.ni * B.nj));
+    const uint32_t o = blockIdx.x * blockDim.x + threadIdx.x, no = (uint32_t)B.ni * B.nj * B.nk;
+    if (o >= no) return;
+    const int i = (int)(o % (uint32_t)B.ni), j = (int)((o / (uint32_t)B.ni) % (uint32_t)B.nj), k = (int)(o / ((uint32_t)B.ni * B.nj));
+    const uint32_t g = (uint32_t)i + (uint32_t)B.pi * ((uint32_t)j + (uint32_t)B.nj * (uint32_t)k);
     for (int d = 0; d < 3; ++d) {
         uint32_t s[6];
         for (int o = -2; o <= 3; ++o) {
@@ -80,7 +82,7 @@ __global__ void k_half(BlockDev B)
             if (d == 0) ii = wrap(i + o, B.ni);
             else if (d == 1) jj = wrap(j + o, B.nj);
             else kk = wrap(k + o, B.nk);
-            s[o + 2] = (uint32_t)ii + (uint32_t)B.ni * ((uint32_t)jj + (uint32_t)B.nj * (uint32_t)kk);
+            s[o + 2] = (uint32_t)ii + (uint32_t)B.pi * ((uint32_t)jj + (uint32_t)B.nj * (uint32_t)kk);
         }
         auto interp = [&](const double *f) {
             return (1.0 / 256.0) * (3.0 * (f[s[0]]) - 25.0 * (f[s[1]]) + 150.0 * (f[s[2]]) + 150.0 * (f[s[3]]) - 25.0 * (f[s[4]])
@@ -97,12 +99,12 @@ struct InitArgs {
     double mach, beta, xc, yc;
 };
 
-// primitives (rho, u, v, w, p) in double into Us, for k_base to turn into P and U0
+// primitives (rho, u, v, w, p) in double into Us, component-major in owned order, for k_base to turn into P and U0
 __global__ void k_init(BlockDev B, InitArgs a)
 {
-    const uint32_t g = blockIdx.x * blockDim.x + threadIdx.x;
-    if (g >= B.n) return;
-    const int i = (int)(g % (uint32_t)B.ni), j = (int)((g / (uint32_t)B.ni) % (uint32_t)B.nj), k = (int)(g / ((uint32_t)B.ni * B.nj));
+    const uint32_t o = blockIdx.x * blockDim.x + threadIdx.x, no = (uint32_t)B.ni * B.nj * B.nk;
+    if (o >= no) return;
+    const int i = (int)(o % (uint32_t)B.ni), j = (int)((o / (uint32_t)B.ni) % (uint32_t)B.nj), k = (int)(o / ((uint32_t)B.ni * B.nj));
     double x[3], s[3];
     node_coords(a.map, B.ni, B.nj, B.nk, i, j, k, x, s);
     const double M = a.mach, pinf = 1.0 / (1.4 * M * M);
@@ -123,7 +125,8 @@ __global__ void k_init(BlockDev B, InitArgs a)
         p = pinf + (1.0 / 16.0) * (cos(2.0 * x[0]) + cos(2.0 * x[1])) * (cos(2.0 * x[2]) + 2.0);
         rho = 1.4 * M * M * p;
     }
-    B.Us[0][g] = rho; B.Us[1][g] = u; B.Us[2][g] = v; B.Us[3][g] = w; B.Us[4][g] = p;
+    double *s5 = B.Us[0];
+    s5[o] = rho; s5[no + o] = u; s5[2 * (size_t)no + o] = v; s5[3 * (size_t)no + o] = w; s5[4 * (size_t)no + o] = p;
 }
 
 // Stable-step radius max over nodes of r_c + r_v, from the RK base U0 = det Q (valid between
@@ -196,7 +199,7 @@ __global__ void __launch_bounds__(RED) k_cfl_final(double *part, int nparts)
 void init_geometry(const BlockDev &B, const double L[3], double amp, const double ph[3], hipStream_t st)
 {
     MapArgs a{{L[0], L[1], L[2]}, amp, {ph[0], ph[1], ph[2]}};
-    const unsigned nb = (unsigned)((B.n + 255) / 256);
+    const unsigned nb = (unsigned)(((uint32_t)B.ni * B.nj * B.nk + 255) / 256);
     hipLaunchKernelGGL(k_geom, dim3(nb), dim3(256), 0, st, B, a);
     hipLaunchKernelGGL(k_half, dim3(nb), dim3(256), 0, st, B);
 }
@@ -205,7 +208,7 @@ void init_state(const BlockDev &B, const double L[3], double amp, const double p
                 double xc, double yc, hipStream_t st)
 {
     InitArgs a{{{L[0], L[1], L[2]}, amp, {ph[0], ph[1], ph[2]}}, kind, mach, beta, xc, yc};
-    const unsigned nb = (unsigned)((B.n + 255) / 256);
+    const unsigned nb = (unsigned)(((uint32_t)B.ni * B.nj * B.nk + 255) / 256);
     hipLaunchKernelGGL(k_init, dim3(nb), dim3(256), 0, st, B, a);
 }
 
