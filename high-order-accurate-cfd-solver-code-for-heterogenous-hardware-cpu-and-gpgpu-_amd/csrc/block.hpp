@@ -12,7 +12,8 @@ namespace blk {
 
 // Tile shapes compiled into the kernels; a launch list picks one of each at run time (the
 // autotuner times them on the actual grids). All tiles have 256 threads.
-//   face sweep along i: (TA lines across = j, TB faces along i)
+//   face sweep along i: (TA lines across = j, TB faces along i); variant 0: the next 256 faces of the lines one
+//   after the other (line_tile), four lines of 64
 //   face sweeps along j and k: (TA lines across = i, TB faces along j or k)
 //   node kernels: (TX along i, TY along j) at one k
 constexpr int N_FACE_I = 3, N_FACE_JK = 4, N_NODE = 4;

@@ -447,9 +447,78 @@ __device__ __forceinline__ uint32_t tile_node(const BlockDev &B, int along, int 
 template <typename S>
 constexpr bool STAGE_ROE = std::is_same<S, float>::value;
 
-// Values of LDS a face tile stages: Q, the node flux and (mixed form) the Roe inputs of its points.
+// Values of LDS a point of a face tile takes: Q, the node flux and (mixed form) the Roe inputs.
+template <typename S>
+constexpr int POINT_VALUES = STAGE_ROE<S> ? 15 : 10;
 template <typename S, int TA, int TB>
-constexpr int FACE_LDS = (STAGE_ROE<S> ? 15 : 10) * (TB + 5) * TA;
+constexpr int FACE_LDS = POINT_VALUES<S> * (TB + 5) * TA;
+
+// Phase 1: the values of the point at stored node x, handed to put(value, its place).
+template <typename S, int DIR, typename Put>
+__device__ __forceinline__ void stage_point(const BlockDev &B, uint32_t x, const Put &put)
+{
+    const S rho = ld((const S *)B.P[0], x), u = ld((const S *)B.P[1], x), v = ld((const S *)B.P[2], x), w = ld((const S *)B.P[3], x),
+            pr = ld((const S *)B.P[4], x);
+    S q[5], f[5];
+    prim_to_q(rho, u, v, w, pr, q);
+    node_flux_e(rho, u, v, w, pr, q[4] + pr, ld(geo<S>(B, 1 + 3 * DIR), x), ld(geo<S>(B, 2 + 3 * DIR), x),
+                ld(geo<S>(B, 3 + 3 * DIR), x), ld(geo<S>(B, 0), x), f);
+#pragma unroll
+    for (int c = 0; c < 5; ++c) {
+        put(c, q[c]);
+        put(5 + c, f[c]);
+    }
+    if constexpr (STAGE_ROE<S>) {
+        put(10, rho); put(11, u); put(12, v); put(13, w);
+        put(14, enthalpy(rho, u, v, w, pr));
+    }
+}
+
+// Phase 2: the flux of the face at stored node gl; get(m, v) is value v of its stencil point m (0..5).
+template <typename S, int DIR, typename Get>
+__device__ __forceinline__ void face_at(const BlockDev &B, uint32_t gl, const Get &get)
+{
+    auto q = [&](int m, int c) { return get(m, c); };
+    S roe[5], irho;
+    if constexpr (STAGE_ROE<S>) {
+        // the face's two centre nodes are stencil points 2 and 3
+        irho = roe_average(get(2, 10), get(2, 11), get(2, 12), get(2, 13), get(2, 14), get(3, 10), get(3, 11), get(3, 12), get(3, 13),
+                           get(3, 14), roe);
+    } else {
+        // from the conserved states of the two centre nodes
+        S qa[5], qb[5], ia, ib, ua, va, wa, ha, ub, vb, wb, hb;
+#pragma unroll
+        for (int c = 0; c < 5; ++c) { qa[c] = q(2, c); qb[c] = q(3, c); }
+        pinv2_(qa[0], qb[0], ia, ib);
+        q_roe_inputs(qa, ia, ua, va, wa, ha);
+        q_roe_inputs(qb, ib, ub, vb, wb, hb);
+        irho = roe_average(qa[0], ua, va, wa, ha, qb[0], ub, vb, wb, hb, roe);
+    }
+    // unit face normal and det_f |k| (the stored face arrays after geometry_finalize)
+    S fg[4];
+    if (!B.stream) {
+#pragma unroll
+        for (int c = 0; c < 3; ++c) fg[c] = ld(geo<S>(B, 10 + 3 * DIR + c), gl);
+        fg[3] = ld(geo<S>(B, 19 + DIR), gl);
+    } else {
+#pragma unroll
+        for (int c = 0; c < 3; ++c) fg[c] = ldx<true>(geo<S>(B, 10 + 3 * DIR + c), gl);
+        fg[3] = ldx<true>(geo<S>(B, 19 + DIR), gl);
+    }
+    S llf[5];
+    face_llf(q, roe, irho, fg[0], fg[1], fg[2], fg[3], S(B.eps), llf);
+    S fh[5];
+#pragma unroll
+    for (int c = 0; c < 5; ++c)
+        fh[c] = S(llf[c] + midpoint_correction(get(0, 5 + c), get(1, 5 + c), get(2, 5 + c), get(3, 5 + c), get(4, 5 + c), get(5, 5 + c)));
+    if (!B.stream) {
+#pragma unroll
+        for (int c = 0; c < 5; ++c) st((S *)B.FH[DIR][c], gl, fh[c]);
+    } else {
+#pragma unroll
+        for (int c = 0; c < 5; ++c) stx<true>((S *)B.FH[DIR][c], gl, fh[c]);
+    }
+}
 
 // The faces of tile lt of block B along DIR; sq: FACE_LDS<S, TA, TB> values of LDS.
 template <typename S, int DIR, int TA, int TB>
@@ -457,8 +526,6 @@ __device__ __forceinline__ void face_tile(const BlockDev &B, uint32_t lt, S *sq)
 {
     static_assert(TA * TB == 256, "face tiles have 256 threads");
     constexpr int NP = TB + 5;
-    S *const sf = sq + 5 * NP * TA;
-    S *const sp = sq + 10 * NP * TA;   // STAGE_ROE only
     const int tid = threadIdx.x;
     const int n_along = DIR == 0 ? B.ni : DIR == 1 ? B.nj : B.nk;
     const int n_across = DIR == 0 ? B.nj : B.ni;
@@ -471,7 +538,6 @@ __device__ __forceinline__ void face_tile(const BlockDev &B, uint32_t lt, S *sq)
     int b0, a0, fixed;
     if (DIR == 0) { b0 = (lt % ntb) * TB; a0 = ((lt / ntb) % nta) * TA; fixed = lt / (ntb * nta); }
     else { a0 = (lt % nta) * TA; b0 = ((lt / nta) % ntb) * TB; fixed = lt / (nta * ntb); }
-    const S *P0 = (const S *)B.P[0], *P1 = (const S *)B.P[1], *P2 = (const S *)B.P[2], *P3 = (const S *)B.P[3], *P4 = (const S *)B.P[4];
 
     __syncthreads();   // the previous tile's LDS fully consumed
     for (int p = tid; p < NP * TA; p += 256) {
@@ -484,82 +550,93 @@ __device__ __forceinline__ void face_tile(const BlockDev &B, uint32_t lt, S *sq)
         if (s > nfa - b0 + 4) continue;
         const int along = along_shift(B, DIR, b0 - sh, s - 2, n_along);
         const uint32_t x = tile_node<DIR>(B, along, a0 + a, fixed);
-        const S rho = ld(P0, x), u = ld(P1, x), v = ld(P2, x), w = ld(P3, x), pr = ld(P4, x);
-        S q[5], f[5];
-        prim_to_q(rho, u, v, w, pr, q);
-        node_flux_e(rho, u, v, w, pr, q[4] + pr, ld(geo<S>(B, 1 + 3 * DIR), x), ld(geo<S>(B, 2 + 3 * DIR), x),
-                    ld(geo<S>(B, 3 + 3 * DIR), x), ld(geo<S>(B, 0), x), f);
-#pragma unroll
-        for (int c = 0; c < 5; ++c) {
-            sq[lds_at<DIR, TA, TB>(c, s, a)] = q[c];
-            sf[lds_at<DIR, TA, TB>(c, s, a)] = f[c];
-        }
-        if constexpr (STAGE_ROE<S>) {
-            sp[lds_at<DIR, TA, TB>(0, s, a)] = rho; sp[lds_at<DIR, TA, TB>(1, s, a)] = u;
-            sp[lds_at<DIR, TA, TB>(2, s, a)] = v; sp[lds_at<DIR, TA, TB>(3, s, a)] = w;
-            sp[lds_at<DIR, TA, TB>(4, s, a)] = enthalpy(rho, u, v, w, pr);
-        }
+        stage_point<S, DIR>(B, x, [&](int v, S y) { sq[lds_at<DIR, TA, TB>(v, s, a)] = y; });
     }
     __syncthreads();
 
     const int b = DIR == 0 ? tid % TB : tid / TA;
     const int a = DIR == 0 ? tid / TB : tid % TA;
     if (b0 + b < nfa && a0 + a < n_across) {
-        auto q = [&](int m, int c) { return sq[lds_at<DIR, TA, TB>(c, b + m, a)]; };
-        const uint32_t gl = tile_node<DIR>(B, b0 + b - sh, a0 + a, fixed);
-        S roe[5], irho;
-        if constexpr (STAGE_ROE<S>) {
-            // the face's two centre nodes are stencil points 2 and 3
-            auto at = [&](int c, int m) { return sp[lds_at<DIR, TA, TB>(c, b + m, a)]; };
-            irho = roe_average(at(0, 2), at(1, 2), at(2, 2), at(3, 2), at(4, 2), at(0, 3), at(1, 3), at(2, 3), at(3, 3), at(4, 3), roe);
-        } else {
-            // from the conserved states of the two centre nodes
-            S qa[5], qb[5], ia, ib, ua, va, wa, ha, ub, vb, wb, hb;
-#pragma unroll
-            for (int c = 0; c < 5; ++c) { qa[c] = q(2, c); qb[c] = q(3, c); }
-            pinv2_(qa[0], qb[0], ia, ib);
-            q_roe_inputs(qa, ia, ua, va, wa, ha);
-            q_roe_inputs(qb, ib, ub, vb, wb, hb);
-            irho = roe_average(qa[0], ua, va, wa, ha, qb[0], ub, vb, wb, hb, roe);
-        }
-        // unit face normal and det_f |k| (the stored face arrays after geometry_finalize)
-        S fg[4];
-        if (!B.stream) {
-#pragma unroll
-            for (int c = 0; c < 3; ++c) fg[c] = ld(geo<S>(B, 10 + 3 * DIR + c), gl);
-            fg[3] = ld(geo<S>(B, 19 + DIR), gl);
-        } else {
-#pragma unroll
-            for (int c = 0; c < 3; ++c) fg[c] = ldx<true>(geo<S>(B, 10 + 3 * DIR + c), gl);
-            fg[3] = ldx<true>(geo<S>(B, 19 + DIR), gl);
-        }
-        S llf[5];
-        face_llf(q, roe, irho, fg[0], fg[1], fg[2], fg[3], S(B.eps), llf);
-        S fh[5];
-#pragma unroll
-        for (int c = 0; c < 5; ++c)
-            fh[c] = S(llf[c] + midpoint_correction(sf[lds_at<DIR, TA, TB>(c, b, a)], sf[lds_at<DIR, TA, TB>(c, b + 1, a)],
-                                                   sf[lds_at<DIR, TA, TB>(c, b + 2, a)], sf[lds_at<DIR, TA, TB>(c, b + 3, a)],
-                                                   sf[lds_at<DIR, TA, TB>(c, b + 4, a)], sf[lds_at<DIR, TA, TB>(c, b + 5, a)]));
-        if (!B.stream) {
-#pragma unroll
-            for (int c = 0; c < 5; ++c) st((S *)B.FH[DIR][c], gl, fh[c]);
-        } else {
-#pragma unroll
-            for (int c = 0; c < 5; ++c) stx<true>((S *)B.FH[DIR][c], gl, fh[c]);
-        }
+        face_at<S, DIR>(B, tile_node<DIR>(B, b0 + b - sh, a0 + a, fixed),
+                        [&](int m, int v) { return sq[lds_at<DIR, TA, TB>(v, b + m, a)]; });
     }
+}
+
+// Variant 0 of the i sweep: a tile is the next line_faces() faces of the block's lines one after the other, whatever
+// their length, so that no tile but the last is partly empty. (Tiles of 4 lines by 64 faces gave the 385 faces of a
+// bounded line of 384 nodes 7 tiles, and 97 faces 2; us a step with those and with these, FP64 and mixed: C-grids
+// 128x64x16 146 and 141, 107 and 103; 384x128x32 1279 and 1257, 825 and 807; 97x83x61 353 and 344, 226 and 221; sizes of
+// whole tiles 0-0.5 %.) The stencil points of its faces are the points of the lines' own sequence, row = nf + 5 to
+// a line, from that of its first face on.
+constexpr int LINE_POINTS = 336;
+__device__ __host__ __forceinline__ uint32_t line_faces(uint32_t nf)
+{
+    // 256 faces reach over 16 lines of 17, 256 + 16 x 5 points; shorter lines: n faces touch up to n / nf + 2
+    return nf >= 17 ? 256u : (LINE_POINTS - 10) * nf / (nf + 5);
+}
+
+template <typename S>
+__device__ __forceinline__ void line_tile(const BlockDev &B, uint32_t lt, S *sq)
+{
+    const uint32_t tid = threadIdx.x, nf = faces_along(B, 0), row = nf + 5, lines = (uint32_t)B.nj * (uint32_t)B.nk;
+    const int sh = B.off[0] ? 1 : 0;
+    const uint32_t faces = line_faces(nf), F0 = lt * faces, count = min(faces, nf * lines - F0);
+    const uint32_t l0 = F0 / nf, f0 = F0 - l0 * nf;               // first line, and its first face here
+    const uint32_t last = (f0 + count - 1) / nf;                  // lines after it
+    const uint32_t points = last * row + (f0 + count - 1 - last * nf) + 6 - f0;
+    const int j0 = (int)(l0 % (uint32_t)B.nj), k0 = (int)(l0 / (uint32_t)B.nj);
+    // item x of len to a line, counted from the first line: lines after it (into s) and the item of that line. Past
+    // the first line x is below LINE_POINTS, where the product with the reciprocal is exact.
+    auto split = [](uint32_t &x, uint32_t len, float inv) -> uint32_t {
+        if (x < len) return 0;
+        x -= len;
+        const uint32_t s = (uint32_t)(((float)x + 0.5f) * inv);
+        x -= s * len;
+        return s + 1;
+    };
+    auto node = [&](uint32_t s, int i) -> uint32_t {
+        int j = j0 + (int)s, k = k0;
+        while (j >= B.nj) { j -= B.nj; ++k; }
+        return node_index(B, i, j, k);
+    };
+    const float inv_row = 1.0f / (float)row, inv_nf = 1.0f / (float)nf;
+
+    __syncthreads();   // the previous tile's LDS fully consumed
+    for (uint32_t p = tid; p < points; p += 256) {
+        uint32_t x = f0 + p;
+        const uint32_t s = split(x, row, inv_row);
+        stage_point<S, 0>(B, node(s, along_shift(B, 0, (int)x - sh, -2, B.ni)), [&](int v, S y) { sq[v * LINE_POINTS + p] = y; });
+    }
+    __syncthreads();
+
+    if (tid < count) {
+        uint32_t f = f0 + tid;
+        const uint32_t s = split(f, nf, inv_nf), p = s * row + f - f0;
+        face_at<S, 0>(B, node(s, (int)f - sh), [&](int m, int v) { return sq[v * LINE_POINTS + p + m]; });
+    }
+}
+
+// Tile lt of the sweep along DIR: variant 0 of the i sweep is a line tile, every other a rectangular one.
+template <int DIR, int TA, int TB>
+constexpr bool LINE_TILE = DIR == 0 && TA == FACE_I_TILES[0][0] && TB == FACE_I_TILES[0][1];
+template <typename S, int DIR, int TA, int TB>
+constexpr int SWEEP_LDS = LINE_TILE<DIR, TA, TB> ? POINT_VALUES<S> *LINE_POINTS : FACE_LDS<S, TA, TB>;
+template <typename S, int DIR, int TA, int TB>
+__device__ __forceinline__ void sweep_tile(const BlockDev &B, uint32_t lt, S *lds)
+{
+    if constexpr (LINE_TILE<DIR, TA, TB>) line_tile<S>(B, lt, lds);
+    else face_tile<S, DIR, TA, TB>(B, lt, lds);
 }
 
 template <typename S, int DIR, int TA, int TB, bool LOOP>
 __global__ void __launch_bounds__(256, (TA == 64 ? 3 : 4)) k_face(const BlockDev *__restrict__ blks, const uint32_t *__restrict__ prefix,
                                               uint32_t nblk, uint32_t total)
 {
-    __shared__ S lds[FACE_LDS<S, TA, TB>];
+    __shared__ S lds[SWEEP_LDS<S, DIR, TA, TB>];
     auto tile = [&](uint32_t wg) {
         const uint32_t t = xcd_tile(wg, total);
         const BlockDev &B = blks[find_block(prefix, nblk, t)];
-        face_tile<S, DIR, TA, TB>(B, t - B.tile0[1 + DIR], lds);
+        sweep_tile<S, DIR, TA, TB>(B, t - B.tile0[1 + DIR], lds);
     };
     each_tile<LOOP>(total, tile);
 }
@@ -585,7 +662,7 @@ __global__ void __launch_bounds__(256, 4) k_flux(const BlockDev *__restrict__ bl
 {
     constexpr int IA = FACE_I_TILES[0][0], IB = FACE_I_TILES[0][1], JA = FACE_JK_TILES[0][0], JB = FACE_JK_TILES[0][1];
     constexpr int TX = NODE_TILES[0][0], TY = NODE_TILES[0][1];
-    constexpr int L0 = VISC ? VISC_LDS<TX, TY> * (int)sizeof(double) : 0, L1 = FACE_LDS<S, IA, IB> * (int)sizeof(S),
+    constexpr int L0 = VISC ? VISC_LDS<TX, TY> * (int)sizeof(double) : 0, L1 = SWEEP_LDS<S, 0, IA, IB> * (int)sizeof(S),
                   L2 = FACE_LDS<S, JA, JB> * (int)sizeof(S);
     __shared__ __align__(16) char lds[L0 > L1 ? (L0 > L2 ? L0 : L2) : (L1 > L2 ? L1 : L2)];
     constexpr bool BND = list_bounded(K);
@@ -609,11 +686,11 @@ __global__ void __launch_bounds__(256, 4) k_flux(const BlockDev *__restrict__ bl
     if (kind == 0) {
         if (B.viscous) visc_tile<S, TX, TY, K>(B, lt, mode, (double *)lds);
     } else if (kind == 1) {
-        face_tile<S, 0, IA, IB>(B, lt, (S *)lds);
+        sweep_tile<S, 0, IA, IB>(B, lt, (S *)lds);
     } else if (kind == 2) {
-        face_tile<S, 1, JA, JB>(B, lt, (S *)lds);
+        sweep_tile<S, 1, JA, JB>(B, lt, (S *)lds);
     } else {
-        face_tile<S, 2, JA, JB>(B, lt, (S *)lds);
+        sweep_tile<S, 2, JA, JB>(B, lt, (S *)lds);
     }
 }
 
@@ -1319,6 +1396,10 @@ uint32_t tiles_of(const BlockDev &B, int kind, const TileCfg &cfg)
     auto f = [&](const int (&t)[2], int along, int across, int fix) {
         return (uint32_t)(((across + t[0] - 1) / t[0]) * ((along + t[1] - 1) / t[1]) * fix);
     };
+    if (kind == 1 && cfg.face[0] == 0) {
+        const uint32_t nf = (uint32_t)faces_along(B, 0), faces = line_faces(nf);
+        return (nf * (uint32_t)B.nj * (uint32_t)B.nk + faces - 1) / faces;
+    }
     if (kind == 1) return f(FACE_I_TILES[cfg.face[0]], faces_along(B, 0), B.nj, B.nk);
     if (kind == 2) return f(FACE_JK_TILES[cfg.face[1]], faces_along(B, 1), B.ni, B.nk);
     return f(FACE_JK_TILES[cfg.face[2]], faces_along(B, 2), B.ni, B.nj);

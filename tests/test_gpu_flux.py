@@ -144,3 +144,38 @@ def test_groups_of_a_batch_give_the_bits_of_each_block_alone(ctx, graph, tiles):
     q.close()
     for b in blocks:
         b.close()
+
+
+@pytest.mark.parametrize("precision", [cfdx.FP64, cfdx.MIXED], ids=["fp64", "mixed"])
+@pytest.mark.parametrize("side", ["periodic", "bounded"])
+def test_line_tiles_give_the_bits_of_rectangular_ones(ctx, side, precision):
+    """The i sweep's default tiles take 256 faces (fewer on lines of under 17) of the lines one after the other:
+    line lengths about the points where the faces of a tile change, its lines end, or it holds many."""
+    prm = cfdx.default_params(mach=0.3, reyl=900.0)
+
+    def make(ni):
+        shape = (ni, 5 if ni > 100 else 11, 7)
+        if side == "periodic":
+            return periodic(ctx, shape, precision, prm)
+        d = cfdx.BlockDesc(*shape[:1], shape[1] + 4, shape[2], 6, precision)
+        d.bc[0], d.bc[1] = cfdx.BC_EXTRAP, cfdx.BC_OUTFLOW
+        xyz, geo = cfdx.box_geometry(d, (0.1 * ni, 1.1, 0.9), 0.005, (0.3, 1.2, 2.1))
+        b = cfdx.Block.of(d, ctx=ctx)
+        b.set_geometry_soa(geo)
+        b.configure(0.3, 0.0, prm)
+        b.set_flow(perturbed(xyz[cfdx.owned_index(d)], 0.3, 2.0))
+        b.configure(0.3, 0.5 * b.cfl_dt(0.5), prm)
+        return b
+
+    low = 3 if side == "periodic" else 7
+    for ni in (low, low + 1, 12, 15, 16, 17, 18, 51, 63, 64, 65, 127, 128, 255, 256, 257, 511):
+        out = []
+        for variant in (0, 1, 2):
+            b = make(ni)
+            b.set_tiles((variant, 0, 0, 0, 4))
+            b.step(2, 0.3, b.dt, prm)
+            out.append(b.get_flow())
+            b.close()
+        for f in FIELDS:
+            assert np.isfinite(out[0][f]).all(), (ni, f)
+            assert np.array_equal(out[0][f], out[1][f]) and np.array_equal(out[0][f], out[2][f]), (ni, f)
