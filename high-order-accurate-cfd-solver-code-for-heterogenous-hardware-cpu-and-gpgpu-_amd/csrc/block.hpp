@@ -117,8 +117,8 @@ constexpr bool list_bounded(int k) { return (k & 2) != 0; }
 
 // Bytes of a stored node that a stage reads and writes (FP64: 22 geometry arrays, U0, Us, P, Fv, FH; mixed:
 // the float geometry, det, U0, Us and the 32 float arrays).
-inline uint64_t stage_bytes(uint64_t n, bool mixed) { return n * (mixed ? 304 : 512); }
-inline uint64_t stage_bytes(const BlockDev &B) { return stage_bytes(B.n, B.geo32 != nullptr); }
+__host__ __device__ inline uint64_t stage_bytes(uint64_t n, bool mixed) { return n * (mixed ? 304 : 512); }
+__host__ __device__ inline uint64_t stage_bytes(const BlockDev &B) { return stage_bytes(B.n, B.geo32 != nullptr); }
 
 // The size past which a block or a list streams: below it a stage's arrays stay in the 256 MB last-level
 // cache (and the L2s) from one stage to the next, and the hint gives that up. FP64: 64^3 197 us a step

@@ -520,6 +520,15 @@ __device__ __forceinline__ void face_at(const BlockDev &B, uint32_t gl, const Ge
     }
 }
 
+// Lines to a row of the j and k sweeps' tiles: the sweeps go over the lines of all rows one after the other, so that
+// the last tile of a row is not partly empty (a tile takes TA lines, 97 nodes would be seven tiles of 16; us a step with
+// those and with these, FP64 and mixed: 97x83x61 344 and 337, 222 and 218; 50x70x90 255 and 230, 154 and 147; rows of whole
+// tiles are unchanged). Blocks that stream keep a tile's lines in a row, on whole pieces of memory.
+__device__ __host__ __forceinline__ int line_row(const BlockDev &B, int TA)
+{
+    return stage_bytes(B) > STREAM_BYTES ? (B.ni + TA - 1) / TA * TA : B.ni;
+}
+
 // The faces of tile lt of block B along DIR; sq: FACE_LDS<S, TA, TB> values of LDS.
 template <typename S, int DIR, int TA, int TB>
 __device__ __forceinline__ void face_tile(const BlockDev &B, uint32_t lt, S *sq)
@@ -528,37 +537,54 @@ __device__ __forceinline__ void face_tile(const BlockDev &B, uint32_t lt, S *sq)
     constexpr int NP = TB + 5;
     const int tid = threadIdx.x;
     const int n_along = DIR == 0 ? B.ni : DIR == 1 ? B.nj : B.nk;
-    const int n_across = DIR == 0 ? B.nj : B.ni;
     // face f of a line is the +1/2 face of along-coordinate f - sh (sh = 1 in a bounded
     // direction: the first face lies between the first owned node and its ghost)
     const int nfa = faces_along(B, DIR), sh = B.off[DIR] ? 1 : 0;
-    const uint32_t nta = (n_across + TA - 1) / TA, ntb = (nfa + TB - 1) / TB;
     // tiles run along the lines' direction before the fixed coordinate, so that the next tile of
     // an XCD re-reads the stencil halo planes of this one from its L2
-    int b0, a0, fixed;
-    if (DIR == 0) { b0 = (lt % ntb) * TB; a0 = ((lt / ntb) % nta) * TA; fixed = lt / (ntb * nta); }
-    else { a0 = (lt % nta) * TA; b0 = ((lt / nta) % ntb) * TB; fixed = lt / (nta * ntb); }
+    const uint32_t ntb = (nfa + TB - 1) / TB, nta = DIR == 0 ? (B.nj + TA - 1) / TA : (B.ni + TA - 1) / TA;
+    const int tb = DIR == 0 ? tid % TB : tid / TA, ta = DIR == 0 ? tid / TB : tid % TA;
+    int b0, a0, fixed, across = 0;
+    bool line;
+    if (DIR == 0) {
+        b0 = (lt % ntb) * TB; a0 = ((lt / ntb) % nta) * TA; fixed = lt / (ntb * nta);
+        line = a0 + ta < B.nj;
+    } else {
+        // a row of tiles takes the next nta * TA lines, whose across coordinate i runs on from one fixed coordinate
+        // to the next after row lines
+        const int row = line_row(B, TA), nfix = DIR == 1 ? B.nk : B.nj;
+        const uint32_t r = lt / (nta * ntb), rest = lt - r * (nta * ntb), tile_b = rest / nta, a = rest - tile_b * nta;
+        b0 = tile_b * TB;
+        a0 = 0;
+        fixed = (int)r;
+        across = (int)(a * TA) + ta;
+        if (row != (int)(nta * TA)) {
+            const uint32_t l0 = (r * nta + a) * TA;
+            fixed = (int)(l0 / (uint32_t)row);
+            across = (int)(l0 - (uint32_t)fixed * (uint32_t)row) + ta;
+            while (across >= row) { across -= row; ++fixed; }
+        }
+        line = across < B.ni && fixed < nfix;
+    }
 
     __syncthreads();   // the previous tile's LDS fully consumed
     for (int p = tid; p < NP * TA; p += 256) {
         const int s = DIR == 0 ? p % NP : p / TA;
-        const int a = DIR == 0 ? p / NP : p % TA;
-        if (a0 + a >= n_across) continue;
+        const int a = DIR == 0 ? p / NP : ta;
+        if (DIR == 0 ? a0 + a >= B.nj : !line) continue;
         // the points past the stencil of the tile's last computed face feed no face: skip them
         // (a bounded line ends 3 ghost nodes past its last owned node; a periodic line shorter
         // than the tile would wrap more than once)
         if (s > nfa - b0 + 4) continue;
         const int along = along_shift(B, DIR, b0 - sh, s - 2, n_along);
-        const uint32_t x = tile_node<DIR>(B, along, a0 + a, fixed);
+        const uint32_t x = tile_node<DIR>(B, along, DIR == 0 ? a0 + a : across, fixed);
         stage_point<S, DIR>(B, x, [&](int v, S y) { sq[lds_at<DIR, TA, TB>(v, s, a)] = y; });
     }
     __syncthreads();
 
-    const int b = DIR == 0 ? tid % TB : tid / TA;
-    const int a = DIR == 0 ? tid / TB : tid % TA;
-    if (b0 + b < nfa && a0 + a < n_across) {
-        face_at<S, DIR>(B, tile_node<DIR>(B, b0 + b - sh, a0 + a, fixed),
-                        [&](int m, int v) { return sq[lds_at<DIR, TA, TB>(v, b + m, a)]; });
+    if (b0 + tb < nfa && line) {
+        face_at<S, DIR>(B, tile_node<DIR>(B, b0 + tb - sh, DIR == 0 ? a0 + ta : across, fixed),
+                        [&](int m, int v) { return sq[lds_at<DIR, TA, TB>(v, tb + m, ta)]; });
     }
 }
 
@@ -1401,8 +1427,13 @@ uint32_t tiles_of(const BlockDev &B, int kind, const TileCfg &cfg)
         return (nf * (uint32_t)B.nj * (uint32_t)B.nk + faces - 1) / faces;
     }
     if (kind == 1) return f(FACE_I_TILES[cfg.face[0]], faces_along(B, 0), B.nj, B.nk);
-    if (kind == 2) return f(FACE_JK_TILES[cfg.face[1]], faces_along(B, 1), B.ni, B.nk);
-    return f(FACE_JK_TILES[cfg.face[2]], faces_along(B, 2), B.ni, B.nj);
+    // rows of tiles over the block's lines, nta tiles to a row
+    auto rows = [&](const int (&t)[2], int along, int fix) {
+        const uint32_t nta = (uint32_t)((B.ni + t[0] - 1) / t[0]), lines = (uint32_t)line_row(B, t[0]) * (uint32_t)fix;
+        return (lines + nta * t[0] - 1) / (nta * t[0]) * nta * (uint32_t)((along + t[1] - 1) / t[1]);
+    };
+    if (kind == 2) return rows(FACE_JK_TILES[cfg.face[1]], faces_along(B, 1), B.nk);
+    return rows(FACE_JK_TILES[cfg.face[2]], faces_along(B, 2), B.nj);
 }
 
 }  // namespace blk
