@@ -316,8 +316,8 @@ def tuned_tiles(cfdx, cdef, precision, mach, prm):
 
 
 def graph_steps(cfdx, block, ctx, tiles=None):
-    """A one-block batch around `block` whose step(n) replays a captured RK3-step graph: the
-    library's graph path for a single block. The block keeps its
+    """A one-block batch around `block`: step(n) launches the stages of the default tiles directly and
+    replays a captured RK3-step graph with tiles whose stage forks onto a second stream. The block keeps its
     state and run parameters; remove it (q.remove, q.close) to step it directly again."""
     q = cfdx.Batch(block.precision, ctx)
     q.add(block)
@@ -327,8 +327,8 @@ def graph_steps(cfdx, block, ctx, tiles=None):
 
 
 def time_block(block, ctx, mach, dt, prm, steps, warmup, profile_steps, cfdx=None, tiles=None):
-    """Warm-up, K timed steps bracketed by HIP events on the block's stream (replayed as a
-    captured graph when cfdx is given, see graph_steps), then a separate per-kernel-class
+    """Warm-up, K timed steps bracketed by HIP events on the block's stream (through a
+    one-block batch when cfdx is given, see graph_steps), then a separate per-kernel-class
     timing pass of direct steps."""
     q = graph_steps(cfdx, block, ctx, tiles) if cfdx is not None else None
     step = (lambda n: q.step(n, True)) if q else (lambda n: block.step(n, mach, dt, prm))
@@ -389,7 +389,7 @@ def dropin_path(cfdx, case, mach, dt, prm, block_value, steps: int = 3):
 
 def timed_run(cfdx, name, precision, steps, warmup, tune, profile_steps=2, ctx=None, host_case=None, keep_flow=True):
     """One workload's timed block: tuned tiles, CFL-0.5 dt from the initial state, `warmup`
-    untimed and `steps` timed RK3 steps replayed from the captured step graph (device time from
+    untimed and `steps` timed RK3 steps of a one-block batch (device time from
     HIP events on the block's stream), then the per-kernel-class timing pass."""
     spec, cdef, pkw, viscous = workload(name)
     prm = cfdx.default_params(**pkw) if viscous else cfdx.euler_params()
@@ -439,7 +439,7 @@ def c2_leg(cfdx, steps, warmup, tune, profile_steps=2):
 def batched_c4(cfdx, steps: int, warmup: int, nblocks: int = 64, grid_cap: int = 0):
     """C4: the 64 seeded periodic cubes (edge U{32,48,64,96,128}, isentropic vortex / TGV ~
     Bernoulli(1/2), Mach U(0.1,0.6), Re U(500,5000)), set up on the device; mixed precision, one
-    batched launch per kernel class replayed from a hipGraph of one RK3 step, tuned tiles. Also
+    batched step (cache-sized groups of blocks), tuned tiles. Also
     times the same solves in plain FP64 one block after another."""
     from cfdx import tune, workloads
     ctx = cfdx.Ctx(0)
@@ -748,7 +748,7 @@ def main() -> int:
         "data": "synthetic",
         "config": dict(spec, parallelism="single GPU, one block (one GPU's share of a 512^3 run split 2x2x2)"
                        if args.workload == "ns256" else "single GPU, one block", precision=args.precision,
-                       stepping="captured RK3-step graph replays (one-block batch)"),
+                       stepping="one-block batch (captured RK3-step graph where the tuned tiles fork)"),
         "roofline": {"bound": bound or "valu", "achieved": alg_gbs, "peak": HBM_PEAK_GBS, "unit": "GB/s",
                      "frac": alg_gbs / HBM_PEAK_GBS,
                      "traffic": counters["hbm_bytes_per_step"] if counters else None,

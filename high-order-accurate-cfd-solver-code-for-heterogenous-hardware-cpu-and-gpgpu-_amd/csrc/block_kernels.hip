@@ -1,11 +1,13 @@
-// Structured-block kernels. Each block is one periodic ni x nj x nk grid held in HBM as
+// Structured-block kernels. Each block is one ni x nj x nk grid, periodic or bounded, held in HBM as
 // structure-of-arrays; a launch covers a list of blocks (one for cfdx_block_step, many for a
 // batch), every workgroup taking one tile of one block through a prefix table of tile counts.
+//   k_flux        a stage's viscous tiles and face tiles in one launch (default tile shapes); apart:
 //   k_visc        node kernel: Fv, Ev, Gv (+ mu) from the stage vector U (Viscous.cl)
 //   k_face<DIR>   one thread per face (i+1/2 along DIR): characteristic WCNS reconstruction,
 //                 LLF and the 6th-order midpoint correction (Weno.cl), LDS-staged tiles
 //   k_update      flux differences + viscous divergence -> L, SSP-RK3 stage j, primitives
 //                 (Weno.cl:3060-3135)
+//   k_bc_ij, k_bc side conditions of bounded blocks after each stage
 // Each face flux is computed once and shared by its two nodes (the reference computes it
 // twice, once from each side, with identical operands).
 // S is the flux arithmetic / storage type: double (plain form) or float (mixed form). The RK
@@ -668,10 +670,12 @@ __global__ void __launch_bounds__(256, (TA == 64 ? 3 : 4)) k_face(const BlockDev
 }
 
 // The viscous node tiles and the three face sweeps of a stage in one launch (tile variants 0). They
-// depend on nothing of each other, and apart each launch ends with a tail and a gap: at 64^3 the
-// five launches of a stage take 87 us (FP64) and 59 us (mixed), the two that are left 71 and 42 us;
-// at 128^3 511 us against 546 apart (FP64) and 294 against 325 (mixed), at 256^3 4.19 ms against 4.26 and
-// 2.40 against 2.43. Each XCD takes its own contiguous share of every kind of tile and runs through them
+// depend on nothing of each other, and apart each launch ends with a tail and a gap: when it was made, a stage of 64^3
+// took 87 us in five launches and 71 in two (FP64; mixed 59 and 42), 128^3 546 and 511 (325 and 294), 256^3 4.26 ms and
+// 4.19 (2.43 and 2.40); now 57 us (37), 510 (286) and 4.25 ms (2.38). At 256^3 it takes 2.78 ms FP64 and 1.59 mixed, moves
+// 11.0 and 5.9 GB through the L2 and issues 8.6e8 and 8.0e8 wave instructions: FP64 65-70 % of the issue slots at the 1.9
+// GHz that the card's power limit leaves, 3.96 TB/s; mixed all of them (an FP32 instruction takes an issue slot like an
+// FP64 one). Each XCD takes its own contiguous share of every kind of tile and runs through them
 // FLUX_CHUNK tiles of a kind at a time: with the kinds alternating tile by tile they fall into step
 // with the CUs (each CU draws tiles of one kind; 256^3 8 % slower in FP64, 23 % mixed), 4 and 16 are
 // best, a kind's whole share at a time 1 % slower at 256^3 FP64 and 3 % at 128^3 mixed.
@@ -721,7 +725,8 @@ __global__ void __launch_bounds__(256, 4) k_flux(const BlockDev *__restrict__ bl
 }
 
 // ---------------------------------------------------------------------------
-// update kernel: L and the SSP-RK3 stage (Weno.cl:3060-3135), in double.
+// update kernel: L and the SSP-RK3 stage (Weno.cl:3060-3135), in double. Bound by memory: 256^3 FP64 1.41 ms, 7.0
+// GB (6.4 with every value once), 5.0 TB/s; mixed 0.81 ms, 4.3 GB, 5.3 TB/s (a copy of 4 GiB: 4.7).
 //   mode 0..2: RK stage j; mode 3: write L only, to Lout (owned order, component-major)
 // ---------------------------------------------------------------------------
 // L and the SSP-RK3 stage of one node; mdu / mdv / mde: the node's monitor values (mode 2 with

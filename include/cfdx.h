@@ -300,7 +300,7 @@ int cfdx_block_set_tiles(cfdx_block *b, const cfdx_tiles *t);
 int cfdx_block_get_tiles(cfdx_block *b, cfdx_tiles *t);
 
 /* Batches: blocks of different sizes and run parameters stepped together. Each kernel class is
- * one launch over the tiles of every block; a step can be replayed from a captured hipGraph.
+ * one launch over the tiles of a group of blocks that the last-level cache holds.
  * A batch references its blocks (it does not own them); all share its precision and device. */
 /* Static operation count of the scheme's arithmetic (no counterpart in the reference; for
  * measurement): the device physics run once on a counting number type. out[6 g + c], groups g =
