@@ -725,7 +725,7 @@ extern "C" int cfdx_block_cfl_dt(cfdx_block *b, double cfl, double *dt)
     if (!b || !dt || !(cfl > 0)) return cfdx::fail(CFDX_E_INVALID, "cfl_dt: null argument or cfl <= 0");
     CFDX_TRY(enter_block(b));
     // per-workgroup maxima in the face-flux scratch (at most 1025 doubles)
-    double *part = (double *)b->B.FH[0][0];
+    double *part = (double *)(((uintptr_t)b->B.FH[0][0] + 7) & ~(uintptr_t)7);
     const int np = cfdx::blk::cfl_parts(b->B);
     cfdx::blk::cfl_radius(b->B, part, b->ctx->stream);
     CFDX_TRY(cfdx::check_launch("cfl_radius"));
