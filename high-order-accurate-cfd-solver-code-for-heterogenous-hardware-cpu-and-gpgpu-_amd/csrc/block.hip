@@ -504,7 +504,8 @@ extern "C" int cfdx_block_create(cfdx_ctx *ctx, const cfdx_block_desc *desc, cfd
         padded_dims(desc, dims, B.off);
         B.pi = R.pitch;
         B.pj = dims[1];
-        for (int q = 0; q < 6; ++q) B.bc[q] = desc->bc[q];
+        // the conditions of a periodic direction are ignored: none of them reaches a kernel
+        for (int q = 0; q < 6; ++q) B.bc[q] = B.off[q / 2] ? desc->bc[q] : 0;
         B.cut_i0 = desc->cut_i0;
         B.cut_i1 = desc->cut_i1;
         B.cos_aoa = std::cos(desc->aoa);
