@@ -50,3 +50,34 @@ def test_conditions_of_a_periodic_direction_are_ignored(ctx, periodic, bc, preci
     assert np.array_equal(L0, L1)
     for f in FIELDS:
         assert np.array_equal(f0[f], f1[f]), f
+
+
+@PRECISIONS
+@pytest.mark.parametrize("periodic", [4, 0, 6], ids=["bounded-ij", "bounded-ijk", "bounded-i"])
+def test_a_uniform_state_has_no_derivative_at_the_sides(ctx, periodic, precision):
+    """A uniform state on a uniform grid: every difference of two points is exactly 0, so every one-sided form and
+    the central one give exactly 0, and with them the viscous fluxes, their divergence and the whole right-hand
+    side. (Weighted sums of the values leave rounding of the state's own size, 1e-17 of it.) The primitives are numbers
+    of 32 bits: a mixed block rounds those of its side nodes to them."""
+    d = desc((12, 10, 9), periodic, (cfdx.BC_EXTRAP,) * 6, precision)
+    for q in range(3):
+        if (periodic >> q) & 1:
+            d.bc[2 * q] = d.bc[2 * q + 1] = 0
+    dims, _ = cfdx.padded(d)
+    geo = np.zeros((22, int(np.prod(dims))))
+    geo[0] = 0.07                             # det
+    for c, m in zip((1, 5, 9), (2.3, 3.1, 1.7)):
+        geo[c] = m                            # zeta_x, eta_y, xi_z
+        geo[c + 9] = m                        # the same on the faces of that direction
+    geo[19:] = 0.07
+    prm = cfdx.default_params(mach=0.4, reyl=300.0)
+    f = cfdx.freestream(d.ni * d.nj * d.nk, 0.4, 3.0)
+    for c, x in zip(("rho", "u", "v", "w", "p"), (1.125, 0.6875, 0.3125, -0.1875, 3.25)):
+        f[c] = x
+    b = cfdx.Block.of(d, ctx=ctx)
+    b.set_geometry_soa(geo)
+    b.configure(0.4, 0.0, prm)
+    b.set_flow(f)
+    L = b.rhs(prm)
+    b.close()
+    assert (L == 0).all(), np.abs(L).max()
