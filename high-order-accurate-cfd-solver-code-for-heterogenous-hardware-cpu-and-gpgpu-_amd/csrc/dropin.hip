@@ -131,8 +131,9 @@ __global__ void __launch_bounds__(128, 3) k_viscous(const double *__restrict__ U
             dU[c] = loc_derivative(f, loc[3], loc[1], loc[2], loc[4], loc[5], false);
             pin_(dU[c]);
         }
-        // magnitude of the MTS scale-similarity term of momentum component d+1 along d (Viscous.cl:493-495)
-        sk[d] = fabs_(nr.r[d] - ((0.25 * V[2][1 + d] + 0.5 * U[1 + d] + 0.25 * V[4][1 + d]) * pinv_(0.25 * V[2][0] + 0.5 * U[0] + 0.25 * V[4][0])));
+        // magnitude of the MTS scale-similarity term of momentum component d+1 along d (Viscous.cl:493-495): a small
+        // difference of two quotients, so both are correctly rounded divisions
+        sk[d] = fabs_(U[1 + d] / U[0] - (0.25 * V[2][1 + d] + 0.5 * U[1 + d] + 0.25 * V[4][1 + d]) / (0.25 * V[2][0] + 0.5 * U[0] + 0.25 * V[4][0]));
         pin_(sk[d]);
 #pragma unroll
         for (int c = 3 * d; c < 3 * d + 3; ++c) m[c] = metric[(size_t)MET_N * g + c];

@@ -183,3 +183,30 @@ def test_block_steps_small_periodic(ctx, orc, shape):
         err = cases.rel_err(cases.flow_matrix(b.get_flow()), want)
         b.close()
         assert err.max() <= TOL, (shape, v, err)
+
+
+def test_dropin_scale_similarity_of_equal_velocities(ctx):
+    """The scale-similarity term of direction d is the node's momentum component d + 1 over its density less the same
+    quotient of the weighted sums along d. Where the two quotients are the same number (U_{1+d} / U_0 constant along d, all
+    sums exact in double) they are the same double, the term is exactly 0, and with Re = inf the mixed-time-scale model
+    gives no flux at all."""
+    n = 6
+    rng = np.random.default_rng(4)
+    case = cases.periodic(n, n, n)
+    s = rng.integers(1, 6, (n, n, n)).astype(float)            # [k, j, i]: the det that scales the whole state
+    a = [rng.integers(-(1 << 20), 1 << 20, (n, n)).astype(float) for _ in range(3)]
+    U = np.empty((n, n, n, 5))
+    U[..., 0] = s * 1234567.0
+    U[..., 1] = s * a[0][:, :, None]                           # u of (k, j)
+    U[..., 2] = s * a[1][:, None, :]                           # v of (k, i)
+    U[..., 3] = s * a[2][None, :, :]                           # w of (j, i)
+    U[..., 4] = s * 8.0e6
+    rows = len(case["Grid_P"])
+    U_C = np.ones((rows, 5))
+    U_C[1:n ** 3 + 1] = U.reshape(-1, 5)
+    d = {k: ctx.to_device(np.ascontiguousarray(case[k])) for k in ("Grid_P", "metric", "det", "FLOW")}
+    out = [ctx.zeros((rows, 5)) for _ in range(6)]
+    prm = cfdx.default_params(reyl=math.inf, mach=0.3)
+    ctx.viscous(ctx.to_device(U_C), *out, d["Grid_P"], d["metric"], d["det"], d["FLOW"], rows, prm)
+    flux = np.abs(np.stack([o.numpy() for o in out[3:]])[:, 1:]).max()
+    assert flux == 0.0, flux
