@@ -387,7 +387,11 @@ int upload_batch(cfdx_batch *q)
         const size_t cap = std::max<size_t>(nb, 2 * q->cap);
         hipError_t e = hipMalloc((void **)&q->dB, cap * sizeof(BlockDev));
         if (e == hipSuccess) e = hipMalloc((void **)&q->dprefix, 4 * 2 * cap * sizeof(uint32_t));
-        if (e != hipSuccess) { q->cap = 0; return cfdx::fail(CFDX_E_NOMEM, "batch: descriptor allocation failed"); }
+        if (e != hipSuccess) {
+            (void)hipGetLastError();
+            q->cap = 0;
+            return cfdx::fail(CFDX_E_NOMEM, "batch: descriptor allocation failed");
+        }
         q->cap = cap;
     }
     // descriptors group by group; a group of n blocks has n + 1 prefix entries of each kind, so 2 x cap

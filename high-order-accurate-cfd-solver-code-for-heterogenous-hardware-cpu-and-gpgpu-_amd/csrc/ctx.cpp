@@ -50,7 +50,10 @@ void *pool_take(int device, size_t bytes, size_t *got)
     if (hipMalloc(&ptr, bytes) != hipSuccess) {
         (void)hipGetLastError();
         pool_trim(device);
-        if (hipMalloc(&ptr, bytes) != hipSuccess) return nullptr;
+        if (hipMalloc(&ptr, bytes) != hipSuccess) {
+            (void)hipGetLastError();
+            return nullptr;
+        }
     }
     *got = bytes;
     return ptr;
@@ -244,7 +247,10 @@ extern "C" int cfdx_device_alloc(cfdx_ctx *ctx, size_t bytes, void **dptr)
     if (!dptr) return cfdx::fail(CFDX_E_INVALID, "device_alloc: null out");
     *dptr = nullptr;
     hipError_t e = hipMalloc(dptr, bytes ? bytes : 1);
-    if (e != hipSuccess) return cfdx::fail(CFDX_E_NOMEM, "hipMalloc(%zu): %s", bytes, hipGetErrorString(e));
+    if (e != hipSuccess) {
+        (void)hipGetLastError();
+        return cfdx::fail(CFDX_E_NOMEM, "hipMalloc(%zu): %s", bytes, hipGetErrorString(e));
+    }
     return CFDX_OK;
 }
 

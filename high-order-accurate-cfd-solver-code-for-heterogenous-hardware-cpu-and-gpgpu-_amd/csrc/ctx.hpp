@@ -44,8 +44,11 @@ void staging_trim();
 
 namespace cfdx {
 
+// Reports a failed call. The runtime keeps an error until it is read: it is read here, so that a later
+// check_launch does not report it again.
 inline int hip_fail(hipError_t e, const char *what)
 {
+    (void)hipGetLastError();
     return fail(CFDX_E_HIP, "%s: %s (%d)", what, hipGetErrorString(e), (int)e);
 }
 

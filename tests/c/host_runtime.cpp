@@ -1,0 +1,137 @@
+/* The library's host sources (csrc/ctx.cpp, host_copy.cpp, common.cpp) on a HIP runtime of plain host memory that keeps
+ * the books: what is allocated on which device, and the last error, which like the real one's stays until it is read.
+ * No GPU, and no HIP library is linked. One check a run, named by the argument; "ok" if it holds. */
+#include <cstdio>
+#include <cstdlib>
+#include <cstring>
+#include <map>
+#include <mutex>
+#include <vector>
+
+#include "ctx.hpp"
+
+namespace {
+constexpr int DEVICES = 4;
+std::mutex mu;
+std::map<void *, size_t> device_mem, host_mem;
+size_t device_free = (size_t)1 << 30;
+size_t host_allocs = 0;                     // hipHostMalloc calls so far
+thread_local int current = 0;
+thread_local hipError_t last = hipSuccess;
+
+hipError_t done(hipError_t e)
+{
+    if (e != hipSuccess && e != hipErrorNotReady) last = e;
+    return e;
+}
+
+#define CHECK(cond, ...)                        \
+    do {                                        \
+        if (!(cond)) {                          \
+            std::printf("failed: " __VA_ARGS__); \
+            std::printf(" (%s)\n", #cond);      \
+            std::exit(1);                       \
+        }                                       \
+    } while (0)
+}  // namespace
+
+extern "C" {
+hipError_t hipGetLastError()
+{
+    const hipError_t e = last;
+    last = hipSuccess;
+    return e;
+}
+const char *hipGetErrorString(hipError_t e) { return e == hipSuccess ? "no error" : "an error"; }
+hipError_t hipGetDeviceCount(int *n) { *n = DEVICES; return hipSuccess; }
+hipError_t hipSetDevice(int d) { current = d; return done(d >= 0 && d < DEVICES ? hipSuccess : hipErrorInvalidDevice); }
+hipError_t hipMalloc(void **p, size_t n)
+{
+    std::lock_guard<std::mutex> lock(mu);
+    if (n > device_free) return done(hipErrorOutOfMemory);
+    *p = std::malloc(16);
+    device_mem[*p] = n;
+    device_free -= n;
+    return hipSuccess;
+}
+hipError_t hipFree(void *p)
+{
+    std::lock_guard<std::mutex> lock(mu);
+    const auto it = device_mem.find(p);
+    if (it == device_mem.end()) return done(hipErrorInvalidValue);
+    device_free += it->second;
+    device_mem.erase(it);
+    std::free(p);
+    return hipSuccess;
+}
+hipError_t hipMemGetInfo(size_t *f, size_t *t)
+{
+    *f = device_free;
+    *t = (size_t)1 << 30;
+    return hipSuccess;
+}
+hipError_t hipHostMalloc(void **p, size_t n, unsigned)
+{
+    std::lock_guard<std::mutex> lock(mu);
+    *p = std::malloc(n);
+    host_mem[*p] = n;
+    ++host_allocs;
+    return hipSuccess;
+}
+hipError_t hipHostFree(void *p)
+{
+    std::lock_guard<std::mutex> lock(mu);
+    host_mem.erase(p);
+    std::free(p);
+    return hipSuccess;
+}
+hipError_t hipMemcpyAsync(void *d, const void *s, size_t n, hipMemcpyKind, hipStream_t)
+{
+    std::memcpy(d, s, n);
+    return hipSuccess;
+}
+hipError_t hipStreamCreateWithFlags(hipStream_t *s, unsigned) { *s = (hipStream_t)std::malloc(1); return hipSuccess; }
+hipError_t hipStreamDestroy(hipStream_t s) { std::free((void *)s); return hipSuccess; }
+hipError_t hipStreamSynchronize(hipStream_t) { return hipSuccess; }
+hipError_t hipEventCreate(hipEvent_t *e) { *e = (hipEvent_t)std::malloc(1); return hipSuccess; }
+hipError_t hipEventCreateWithFlags(hipEvent_t *e, unsigned) { return hipEventCreate(e); }
+hipError_t hipEventDestroy(hipEvent_t e) { std::free((void *)e); return hipSuccess; }
+hipError_t hipEventRecord(hipEvent_t, hipStream_t) { return hipSuccess; }
+hipError_t hipEventQuery(hipEvent_t) { return hipSuccess; }
+hipError_t hipEventSynchronize(hipEvent_t) { return hipSuccess; }
+hipError_t hipEventElapsedTime(float *ms, hipEvent_t, hipEvent_t) { *ms = 0; return hipSuccess; }
+}
+
+namespace {
+cfdx_ctx *context(int device)
+{
+    cfdx_ctx *c = nullptr;
+    CHECK(cfdx_ctx_create(device, nullptr, &c) == CFDX_OK, "context on device %d", device);
+    return c;
+}
+
+// An allocation that does not fit is answered with a null pointer and leaves no error behind: the next launch check
+// of the thread, on work that did fit, passes.
+void pool()
+{
+    cfdx_ctx *c = context(0);
+    size_t got = 0;
+    CHECK(!cfdx::pool_take(0, (size_t)2 << 30, &got), "more than the device has");
+    void *p = cfdx::pool_take(0, (size_t)256 << 20, &got);
+    CHECK(p && got == (size_t)256 << 20, "what the device has");
+    CHECK(cfdx::check_launch("the next launch") == CFDX_OK, "%s", cfdx_last_error());
+    cfdx::pool_give(0, p, got);
+    void *d = nullptr;
+    CHECK(cfdx_device_alloc(c, (size_t)2 << 30, &d) == CFDX_E_NOMEM, "device_alloc past the memory");
+    CHECK(cfdx::check_launch("the next launch") == CFDX_OK, "%s", cfdx_last_error());
+    CHECK(cfdx_ctx_destroy(c) == CFDX_OK, "destroy");
+}
+}  // namespace
+
+int main(int argc, char **argv)
+{
+    const char *what = argc > 1 ? argv[1] : "";
+    if (!std::strcmp(what, "pool")) pool();
+    else CHECK(false, "no check named '%s'", what);
+    std::puts("ok");
+}
