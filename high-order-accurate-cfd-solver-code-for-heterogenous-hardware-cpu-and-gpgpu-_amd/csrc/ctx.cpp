@@ -96,14 +96,15 @@ size_t pool_cached(int device)
 extern "C" int cfdx_pool_trim(cfdx_ctx *ctx)
 {
     CFDX_TRY(cfdx::enter(ctx));
-    // the driver may give freed memory back a little later: wait for it (bounded), so that a
-    // cfdx_mem_info that follows counts it
+    // the driver may give freed memory back a little later (within 0.6 ms for 0.1 .. 6 GB): wait for it, so that a
+    // cfdx_mem_info that follows counts it, but no longer than 10 ms, since other threads' allocations may keep the
+    // figure down
     size_t before = 0, now = 0, total = 0;
     const size_t kept = cfdx::pool_cached(ctx->device);
     const bool known = hipMemGetInfo(&before, &total) == hipSuccess;
     cfdx::pool_trim(ctx->device);
     cfdx::staging_trim();
-    for (int q = 0; known && kept && q < 400; ++q) {
+    for (int q = 0; known && kept && q < 20; ++q) {
         if (hipMemGetInfo(&now, &total) != hipSuccess || now >= before + kept / 2) break;
         std::this_thread::sleep_for(std::chrono::microseconds(500));
     }

@@ -16,6 +16,8 @@ std::mutex mu;
 std::map<void *, size_t> device_mem, host_mem;
 size_t device_free = (size_t)1 << 30;
 size_t host_allocs = 0;                     // hipHostMalloc calls so far
+size_t looks = 0;                           // hipMemGetInfo calls so far
+bool taken = false;                         // another process takes what is freed: the free figure stays
 thread_local int current = 0;
 thread_local hipError_t last = hipSuccess;
 
@@ -66,7 +68,10 @@ hipError_t hipFree(void *p)
 }
 hipError_t hipMemGetInfo(size_t *f, size_t *t)
 {
-    *f = device_free;
+    static size_t shown = 0;
+    if (!taken) shown = device_free;
+    *f = shown;
+    ++looks;
     *t = (size_t)1 << 30;
     return hipSuccess;
 }
@@ -126,12 +131,28 @@ void pool()
     CHECK(cfdx::check_launch("the next launch") == CFDX_OK, "%s", cfdx_last_error());
     CHECK(cfdx_ctx_destroy(c) == CFDX_OK, "destroy");
 }
+
+// A trim whose memory is taken by others at once does not wait for the free figure to rise.
+void trim()
+{
+    cfdx_ctx *c = context(0);
+    size_t got = 0, f = 0, t = 0;
+    void *p = cfdx::pool_take(0, (size_t)200 << 20, &got);
+    cfdx::pool_give(0, p, got);
+    (void)hipMemGetInfo(&f, &t);
+    taken = true;
+    const size_t before = looks;
+    CHECK(cfdx_pool_trim(c) == CFDX_OK && cfdx::pool_cached(0) == 0, "trim");
+    CHECK(looks - before <= 32, "%zu looks at the free figure, half a millisecond apart", looks - before);
+    CHECK(cfdx_ctx_destroy(c) == CFDX_OK, "destroy");
+}
 }  // namespace
 
 int main(int argc, char **argv)
 {
     const char *what = argc > 1 ? argv[1] : "";
     if (!std::strcmp(what, "pool")) pool();
+    else if (!std::strcmp(what, "trim")) trim();
     else CHECK(false, "no check named '%s'", what);
     std::puts("ok");
 }
