@@ -80,6 +80,16 @@ unsigned copy_threads()
     return std::min(THREADS, (unsigned)std::max(n, 1));
 }
 
+// Whether the runtime knows the memory (pinned, managed or device memory): a copy into it needs no staging (151 MB
+// into pinned memory 2.78 ms, 57 GB/s; staged 3.55).
+bool known_memory(const void *p)
+{
+    hipPointerAttribute_t a{};
+    if (hipPointerGetAttributes(&a, p) == hipSuccess) return a.type != hipMemoryTypeUnregistered;
+    (void)hipGetLastError();
+    return false;
+}
+
 // One copy. The calling thread puts chunks on the stream as slots come free and watches them arrive (one
 // thread asks the runtime; eight waiting on events took 100 us a chunk); the workers take arrived chunks in
 // order and copy them out. All of them spin with yields: the copy alone is over in milliseconds.
@@ -146,9 +156,9 @@ void staging_trim()
 
 int copy_to_host(cfdx_ctx *ctx, void *dst, const void *src, size_t bytes, const char *what)
 {
-    const unsigned nt = bytes >= STAGED_FROM ? copy_threads() : 0;
+    const unsigned nt = bytes >= STAGED_FROM && !known_memory(dst) ? copy_threads() : 0;
     Ring *ring = nt > 1 ? ring_take(ctx->device) : nullptr;
-    if (!ring) {   // small, one CPU, or no pinned memory: straight
+    if (!ring) {   // small, into pinned memory, one CPU, or no pinned memory left for a ring: straight
         CFDX_HIP(hipMemcpyAsync(dst, src, bytes, hipMemcpyDeviceToHost, ctx->stream), what);
         CFDX_HIP(hipStreamSynchronize(ctx->stream), what);
         return CFDX_OK;

@@ -90,6 +90,17 @@ hipError_t hipHostFree(void *p)
     std::free(p);
     return hipSuccess;
 }
+// like the real one's older form: memory it does not know is an error
+hipError_t hipPointerGetAttributes(hipPointerAttribute_t *a, const void *p)
+{
+    std::lock_guard<std::mutex> lock(mu);
+    for (const auto &m : host_mem)
+        if ((const char *)p >= (const char *)m.first && (const char *)p < (const char *)m.first + m.second) {
+            a->type = hipMemoryTypeHost;
+            return hipSuccess;
+        }
+    return done(hipErrorInvalidValue);
+}
 hipError_t hipMemcpyAsync(void *d, const void *s, size_t n, hipMemcpyKind, hipStream_t)
 {
     std::memcpy(d, s, n);
@@ -146,6 +157,41 @@ void trim()
     CHECK(looks - before <= 32, "%zu looks at the free figure, half a millisecond apart", looks - before);
     CHECK(cfdx_ctx_destroy(c) == CFDX_OK, "destroy");
 }
+
+// The bytes of a device-to-host copy.
+void copy(cfdx_ctx *c, char *dst, const std::vector<char> &src)
+{
+    std::memset(dst, 0, src.size());
+    CHECK(cfdx_copy_to_host(c, dst, src.data(), src.size()) == CFDX_OK, "copy: %s", cfdx_last_error());
+    CHECK(std::memcmp(dst, src.data(), src.size()) == 0, "the bytes of a copy");
+}
+
+std::vector<char> bytes(size_t n)
+{
+    std::vector<char> b(n);
+    for (size_t q = 0; q < n; ++q) b[q] = (char)(q * 31 + (q >> 12));
+    return b;
+}
+
+// Large copies into pageable memory go through a pinned ring; into memory that is pinned already, also from the middle
+// of it on, they go straight. Neither leaves an error behind.
+void pinned()
+{
+    cfdx_ctx *c = context(0);
+    const std::vector<char> src = bytes((size_t)20 << 20);
+    void *p = nullptr;
+    (void)hipHostMalloc(&p, src.size() + 4096, 0);
+    const size_t own = host_allocs;
+    copy(c, (char *)p, src);
+    copy(c, (char *)p + 4096, src);
+    CHECK(host_allocs == own, "a ring was made for a copy into pinned memory");
+    std::vector<char> plain(src.size());
+    copy(c, plain.data(), src);
+    CHECK(host_allocs == own + 1, "%zu rings for a copy into pageable memory", host_allocs - own);
+    CHECK(cfdx::check_launch("the next launch") == CFDX_OK, "%s", cfdx_last_error());
+    (void)hipHostFree(p);
+    CHECK(cfdx_ctx_destroy(c) == CFDX_OK, "destroy");
+}
 }  // namespace
 
 int main(int argc, char **argv)
@@ -153,6 +199,7 @@ int main(int argc, char **argv)
     const char *what = argc > 1 ? argv[1] : "";
     if (!std::strcmp(what, "pool")) pool();
     else if (!std::strcmp(what, "trim")) trim();
+    else if (!std::strcmp(what, "pinned")) pinned();
     else CHECK(false, "no check named '%s'", what);
     std::puts("ok");
 }
