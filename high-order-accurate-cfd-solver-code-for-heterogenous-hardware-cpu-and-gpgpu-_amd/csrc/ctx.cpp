@@ -103,7 +103,7 @@ extern "C" int cfdx_pool_trim(cfdx_ctx *ctx)
     const size_t kept = cfdx::pool_cached(ctx->device);
     const bool known = hipMemGetInfo(&before, &total) == hipSuccess;
     cfdx::pool_trim(ctx->device);
-    cfdx::staging_trim();
+    cfdx::staging_trim(ctx->device);
     for (int q = 0; known && kept && q < 20; ++q) {
         if (hipMemGetInfo(&now, &total) != hipSuccess || now >= before + kept / 2) break;
         std::this_thread::sleep_for(std::chrono::microseconds(500));

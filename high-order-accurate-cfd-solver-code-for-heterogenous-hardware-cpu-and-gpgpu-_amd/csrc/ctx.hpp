@@ -37,9 +37,9 @@ void pool_trim(int device);
 size_t pool_cached(int device);
 
 // bytes of device memory to the host, after the work queued on the context's stream; returns when
-// they are there. Large copies go through pinned memory (host_copy.cpp).
+// they are there. Large copies go through pinned memory (host_copy.cpp), which staging_trim gives back.
 int copy_to_host(cfdx_ctx *ctx, void *dst, const void *src, size_t bytes, const char *what);
-void staging_trim();
+void staging_trim(int device);
 }  // namespace cfdx
 
 namespace cfdx {

@@ -23,12 +23,13 @@ namespace {
 constexpr size_t CHUNK = (size_t)4 << 20, SLOTS = 8;
 constexpr size_t STAGED_FROM = 2 * CHUNK;   // smaller copies go straight
 constexpr unsigned THREADS = 4;
-constexpr size_t KEPT = 2;                  // rings kept for the next copy (32 MB of pinned memory each)
+constexpr size_t KEPT = 2;                  // rings of a device kept for its next copy (32 MB of pinned memory each)
 
 struct Ring {
     char *mem = nullptr;
     hipEvent_t ev[SLOTS] = {};
     int device = 0;
+    Ring *next = nullptr;   // in the list of those not in use
 
     ~Ring()
     {
@@ -39,14 +40,24 @@ struct Ring {
 };
 
 std::mutex rings_mutex;
-Ring *rings[KEPT] = {};   // not in use
+Ring *rings = nullptr;   // not in use, at most KEPT of each device
+
+// the next ring of the device among those not in use, from *at on
+Ring **ring_of(int device, Ring **at)
+{
+    while (*at && (*at)->device != device) at = &(*at)->next;
+    return at;
+}
 
 Ring *ring_take(int device)
 {
     {
         std::lock_guard<std::mutex> lock(rings_mutex);
-        for (Ring *&kept : rings)
-            if (kept && kept->device == device) return std::exchange(kept, nullptr);
+        Ring **at = ring_of(device, &rings);
+        if (Ring *r = *at) {
+            *at = r->next;
+            return r;
+        }
     }
     Ring *r = new (std::nothrow) Ring;
     if (!r) return nullptr;
@@ -64,11 +75,12 @@ void ring_give(Ring *r)
 {
     {
         std::lock_guard<std::mutex> lock(rings_mutex);
-        for (Ring *&kept : rings)
-            if (!kept) {
-                kept = r;
-                return;
-            }
+        size_t kept = 0;
+        for (Ring **at = ring_of(r->device, &rings); *at; at = ring_of(r->device, &(*at)->next)) ++kept;
+        if (kept < KEPT) {
+            r->next = std::exchange(rings, r);
+            return;
+        }
     }
     delete r;
 }
@@ -144,14 +156,18 @@ struct Copy {
 
 }  // namespace
 
-void staging_trim()
+void staging_trim(int device)
 {
-    Ring *gone[KEPT];
+    Ring *gone = nullptr;
     {
         std::lock_guard<std::mutex> lock(rings_mutex);
-        for (size_t q = 0; q < KEPT; ++q) gone[q] = std::exchange(rings[q], nullptr);
+        for (Ring **at = ring_of(device, &rings); *at; at = ring_of(device, at)) {
+            Ring *r = *at;
+            *at = r->next;
+            r->next = std::exchange(gone, r);
+        }
     }
-    for (Ring *r : gone) delete r;
+    while (gone) delete std::exchange(gone, gone->next);
 }
 
 int copy_to_host(cfdx_ctx *ctx, void *dst, const void *src, size_t bytes, const char *what)

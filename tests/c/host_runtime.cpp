@@ -6,6 +6,7 @@
 #include <cstring>
 #include <map>
 #include <mutex>
+#include <thread>
 #include <vector>
 
 #include "ctx.hpp"
@@ -192,6 +193,37 @@ void pinned()
     (void)hipHostFree(p);
     CHECK(cfdx_ctx_destroy(c) == CFDX_OK, "destroy");
 }
+
+// Every device of a process keeps its rings: copies that go round the devices make one each, once. A trim gives those
+// of its device back and no others.
+void rings()
+{
+    cfdx_ctx *c[DEVICES];
+    for (int d = 0; d < DEVICES; ++d) c[d] = context(d);
+    const std::vector<char> src = bytes((size_t)9 << 20);
+    std::vector<char> dst(src.size());
+    for (int round = 0; round < 3; ++round)
+        for (cfdx_ctx *x : c) copy(x, dst.data(), src);
+    CHECK(host_allocs == DEVICES, "%zu rings for %d devices", host_allocs, DEVICES);
+    CHECK(cfdx_pool_trim(c[1]) == CFDX_OK, "trim");
+    CHECK(host_mem.size() == DEVICES - 1, "%zu rings after a trim of one device", host_mem.size());
+    for (cfdx_ctx *x : c) copy(x, dst.data(), src);
+    CHECK(host_allocs == DEVICES + 1, "%zu rings made", host_allocs);
+    for (cfdx_ctx *x : c) CHECK(cfdx_pool_trim(x) == CFDX_OK, "trim");
+    CHECK(host_mem.empty(), "%zu rings after every trim", host_mem.size());
+    // at most two of a device are kept, however many copies ran at once
+    std::vector<std::thread> t;
+    for (int q = 0; q < 6; ++q)
+        t.emplace_back([&src] {
+            cfdx_ctx *x = context(2);
+            std::vector<char> own(src.size());
+            for (int k = 0; k < 4; ++k) copy(x, own.data(), src);
+            CHECK(cfdx_ctx_destroy(x) == CFDX_OK, "destroy");
+        });
+    for (auto &x : t) x.join();
+    CHECK(host_mem.size() <= 2, "%zu rings kept", host_mem.size());
+    for (cfdx_ctx *x : c) CHECK(cfdx_ctx_destroy(x) == CFDX_OK, "destroy");
+}
 }  // namespace
 
 int main(int argc, char **argv)
@@ -200,6 +232,7 @@ int main(int argc, char **argv)
     if (!std::strcmp(what, "pool")) pool();
     else if (!std::strcmp(what, "trim")) trim();
     else if (!std::strcmp(what, "pinned")) pinned();
+    else if (!std::strcmp(what, "rings")) rings();
     else CHECK(false, "no check named '%s'", what);
     std::puts("ok");
 }

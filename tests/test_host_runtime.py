@@ -25,7 +25,7 @@ def program(tmp_path_factory):
     return exe
 
 
-@pytest.mark.parametrize("check", ["pool", "trim", "pinned"])
+@pytest.mark.parametrize("check", ["pool", "trim", "pinned", "rings"])
 def test_host_runtime(program, check):
     r = subprocess.run([program, check], capture_output=True, text=True, timeout=60)
     assert r.returncode == 0 and r.stdout.strip().endswith("ok"), r.stdout + r.stderr
