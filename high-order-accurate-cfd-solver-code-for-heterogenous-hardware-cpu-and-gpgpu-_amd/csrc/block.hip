@@ -306,9 +306,8 @@ int run_stage(cfdx_block *b, int mode, double *Lout = nullptr)
     L.Lout = Lout;
     if (mode == 2) b->mon_count = mon_triples(b->B, b->tiles);
     cfdx::blk::Overlap ov;
-    cfdx::blk::stage(L, b->desc.precision, mode, b->ctx->stream, b->B.viscous != 0, b->timing ? b->ev : nullptr,
-                     overlap_of(b->ctx, ov));
-    b->launches += (b->B.viscous ? 5 : 4);
+    b->launches += cfdx::blk::stage(L, b->desc.precision, mode, b->ctx->stream, b->B.viscous != 0,
+                                    b->timing ? b->ev : nullptr, overlap_of(b->ctx, ov));
     CFDX_TRY(cfdx::check_launch("block stage"));
     if (b->timing) {
         float t[5] = {0, 0, 0, 0, 0};

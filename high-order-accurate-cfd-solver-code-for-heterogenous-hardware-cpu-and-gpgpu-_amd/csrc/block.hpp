@@ -157,12 +157,13 @@ struct LaunchList {
 // ov (optional, ignored when timing with ev): the viscous node kernel and the face sweeps run together:
 // in one launch with the default tile shapes and grid, else the viscous kernel on ov->aux, forked from
 // st before the sweeps and joined back before the update
+// Returns the number of kernels launched.
 struct Overlap {
     hipStream_t aux;
     hipEvent_t fork, join;
 };
-void stage(const LaunchList &L, int precision, int mode, hipStream_t st, bool any_visc, hipEvent_t *ev,
-           const Overlap *ov = nullptr);
+int stage(const LaunchList &L, int precision, int mode, hipStream_t st, bool any_visc, hipEvent_t *ev,
+          const Overlap *ov = nullptr);
 // whether stage() puts the viscous kernel on the second stream: other tile shapes than the defaults or a
 // capped grid, with the overlap on
 bool stage_forks(const LaunchList &L, const Overlap *ov);

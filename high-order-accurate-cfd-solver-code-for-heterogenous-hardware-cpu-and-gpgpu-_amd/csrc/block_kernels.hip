@@ -1128,17 +1128,23 @@ __global__ void __launch_bounds__(BC_IJ) k_bc_ij(const BlockDev *__restrict__ bl
     bc_node<S>(B, 1, (int)((r / (uint32_t)nk) >> 2), (int)(first + c), (int)(r % (uint32_t)nk), (int)((r / (uint32_t)nk) & 3u), mode);
 }
 
+// The kernels launched.
 template <typename S>
-void launch_bc(const LaunchList &L, int mode, hipStream_t st)
+int launch_bc(const LaunchList &L, int mode, hipStream_t st)
 {
+    int n = 0;
     const bool ij = L.bc_face_d[0] && L.bc_face_d[1];
     if (ij) {
         const uint32_t js = (8 * L.bc_face_d[1] + BC_IJ - 1) / BC_IJ;
         hipLaunchKernelGGL(k_bc_ij<S>, dim3(L.bc_planes + js, L.nblk), dim3(BC_IJ), 0, st, L.blks, L.bc_planes, mode);
+        ++n;
     }
     for (int d = ij ? 2 : 0; d < 3; ++d)
-        if (L.bc_face_d[d])
+        if (L.bc_face_d[d]) {
             hipLaunchKernelGGL(k_bc<S>, dim3((4 * L.bc_face_d[d] + 255) / 256, L.nblk, 2), dim3(256), 0, st, L.blks, d, mode);
+            ++n;
+        }
+    return n;
 }
 
 // ---------------------------------------------------------------------------
@@ -1263,13 +1269,14 @@ void launch_flux(const LaunchList &L, int mode, hipStream_t st, bool any_visc)
 }
 
 template <typename S>
-void launch_stage(const LaunchList &L, int mode, hipStream_t st, bool any_visc, hipEvent_t *ev, const Overlap *ov)
+int launch_stage(const LaunchList &L, int mode, hipStream_t st, bool any_visc, hipEvent_t *ev, const Overlap *ov)
 {
     auto rec = [&](int s) { if (ev) (void)hipEventRecord(ev[s], st); };
     rec(0);
     // the viscous node kernel reads the stage vector, primitives and geometry and writes Fv and mu;
     // the face sweeps read the primitives and geometry and write F-hat: independent until the update
     const bool overlap = ov && !ev, together = overlap && !stage_forks(L, ov);
+    int n = together ? 2 : any_visc ? 5 : 4;   // kernels launched
     hipStream_t vs = st;
     if (together) {
         launch_flux<S>(L, mode, st, any_visc);
@@ -1292,14 +1299,15 @@ void launch_stage(const LaunchList &L, int mode, hipStream_t st, bool any_visc, 
     rec(4);
     if (vs != st) (void)hipStreamWaitEvent(st, ov->join, 0);
     node_kernel<S>(L, L.grid_cap, st, false, mode);
-    if (L.bc_face && mode <= 2) launch_bc<S>(L, mode, st);
+    if (L.bc_face && mode <= 2) n += launch_bc<S>(L, mode, st);
     rec(5);
+    return n;
 }
 
-void stage(const LaunchList &L, int precision, int mode, hipStream_t st, bool any_visc, hipEvent_t *ev, const Overlap *ov)
+int stage(const LaunchList &L, int precision, int mode, hipStream_t st, bool any_visc, hipEvent_t *ev, const Overlap *ov)
 {
-    if (precision == CFDX_MIXED) launch_stage<float>(L, mode, st, any_visc, ev, ov);
-    else launch_stage<double>(L, mode, st, any_visc, ev, ov);
+    return precision == CFDX_MIXED ? launch_stage<float>(L, mode, st, any_visc, ev, ov)
+                                   : launch_stage<double>(L, mode, st, any_visc, ev, ov);
 }
 
 void base(const BlockDev &B, int precision, hipStream_t st, const double *stage)

@@ -262,7 +262,7 @@ int cfdx_block_rhs(cfdx_block *b, const cfdx_params *params, double *L_host);
 int cfdx_block_rhs_noalloc(cfdx_block *b, const cfdx_params *params, double *L_dev);
 
 /* Device time in ms of the kernels of the last cfdx_block_step, per kernel class,
- * measured with HIP events on the context stream when timing is on. */
+ * measured with HIP events on the context stream when timing is on, and the kernels it launched. */
 int cfdx_block_set_timing(cfdx_block *b, int on);
 int cfdx_block_timing(cfdx_block *b, double *ms_visc, double *ms_face, double *ms_update, int *launches);
 
