@@ -285,7 +285,9 @@ int cfdx_block_timing_split(cfdx_block *b, double ms[5]);
 /* Tile shapes. Every kernel class has a few compiled tile variants; kind 0 = face sweep along i
  * (shape = lines across j, faces along i), kind 1 = face sweeps along j and k (lines across i,
  * faces along j or k), kind 2 = node kernels (nodes along i, along j). cfdx_tile_variants gives
- * the count and, if shapes is not NULL, 2 * count shape numbers. A block or batch launches the
+ * the count and, if shapes is not NULL, 2 * count shape numbers; variant 0 of kind 0 is named by its
+ * 4 x 64 faces, but takes the next 256 faces (fewer on lines of under 17) of the lines one after the
+ * other, not a rectangle of them. A block or batch launches the
  * variants its cfdx_tiles names (variants 0 and strips of 4 rows by default); results do not
  * depend on them. */
 typedef struct {
