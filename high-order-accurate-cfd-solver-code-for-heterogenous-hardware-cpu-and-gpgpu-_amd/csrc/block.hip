@@ -255,7 +255,7 @@ int upload_single(cfdx_block *b)
     if (b->uploaded == b->version) return CFDX_OK;
     BlockDev B = b->B;
     B.strip = (uint32_t)b->tiles.strip;
-    B.stream = cfdx::blk::streams_past_cache(cfdx::blk::stage_bytes(B), cfdx::blk::rows_stream(B));
+    B.stream = cfdx::blk::streams_past_cache(B);
     uint32_t pre[8];
     for (int kind = 0; kind < 4; ++kind) {
         B.tile0[kind] = 0;
@@ -275,7 +275,7 @@ LaunchList single_list(cfdx_block *b)
     L.blks = b->dB;
     L.nblk = 1;
     L.tiles = b->tiles;
-    L.stream = cfdx::blk::streams_past_cache(cfdx::blk::stage_bytes(b->B), cfdx::blk::rows_stream(b->B));
+    L.stream = cfdx::blk::streams_past_cache(b->B);
     bc_extent(b->B, L);
     for (int kind = 0; kind < 4; ++kind) {
         L.prefix[kind] = b->dprefix + 2 * kind;
@@ -339,6 +339,7 @@ void drop_graph(cfdx_batch *q)
 // 1305 -> 1183 (three a group, 239 MB) and 2272 -> 2025 (two, 268 MB; three, 402 MB: 2240; one: 2135); three 128^3 2837 ->
 // 2614 and 4800 -> 4652; twenty-four 32^3 mixed in one list of 239 MB 376, eight a group 430.
 constexpr uint64_t GROUP_BYTES = (uint64_t)256 << 20;
+static_assert(GROUP_BYTES <= cfdx::blk::STREAM_BYTES, "a group of several blocks does not stream");
 std::vector<std::vector<size_t>> group_blocks(const std::vector<cfdx_block *> &blocks)
 {
     std::vector<size_t> order(blocks.size());
@@ -407,13 +408,9 @@ int upload_batch(cfdx_batch *q)
         L.nblk = (uint32_t)packed[g].size();
         L.grid_cap = q->grid_cap;
         L.tiles = q->tiles;
-        uint64_t bytes = 0;
-        bool rows = true;
-        for (size_t i : packed[g]) {
-            bytes += cfdx::blk::stage_bytes(q->blocks[i]->B);
-            rows = rows && cfdx::blk::rows_stream(q->blocks[i]->B);
-        }
-        L.stream = cfdx::blk::streams_past_cache(bytes, rows);
+        // a group of several blocks stays in the cache; a block past it is a group of its own
+        const BlockDev &B0 = q->blocks[packed[g][0]]->B;
+        L.stream = packed[g].size() == 1 && cfdx::blk::streams_past_cache(B0);
         uint32_t tot[4] = {0, 0, 0, 0};
         for (size_t n = 0; n < packed[g].size(); ++n) {
             BlockDev B = q->blocks[packed[g][n]]->B;

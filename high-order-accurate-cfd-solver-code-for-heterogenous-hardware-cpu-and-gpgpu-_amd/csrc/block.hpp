@@ -130,10 +130,12 @@ __host__ __device__ inline uint64_t stage_bytes(const BlockDev &B) { return stag
 // are found in the cache, and end to end the arrays take less of it.
 constexpr uint64_t STREAM_BYTES = (uint64_t)384 << 20;
 
-// Whether a block's rows take non-temporal accesses: whole 64-byte pieces. With others the hint drops lines that
-// the neighbouring rows still need (FP64 161x131x127 1.5 % slower, 255x200x160 2.5 %, mixed 4 and 5 %).
-inline bool rows_stream(const BlockDev &B) { return (uint64_t)B.pi * (B.geo32 ? 4 : 8) % 64 == 0; }
-inline bool streams_past_cache(uint64_t bytes, bool rows) { return rows && bytes > STREAM_BYTES; }
+// Whether a block takes non-temporal accesses: past that size, with rows of whole 64-byte pieces. With others the hint
+// drops lines that the neighbouring rows still need (FP64 161x131x127 1.5 % slower, 255x200x160 2.5 %, mixed 4 and 5 %).
+inline bool streams_past_cache(const BlockDev &B)
+{
+    return (uint64_t)B.pi * (B.geo32 ? 4 : 8) % 64 == 0 && stage_bytes(B) > STREAM_BYTES;
+}
 
 // One launch over a list of blocks.
 struct LaunchList {

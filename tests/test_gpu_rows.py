@@ -78,6 +78,46 @@ def test_rows_of_a_large_block_give_the_bits_of_a_small_one(ctx, name, precision
     assert np.array_equal(LL.reshape(5, times, -1), np.broadcast_to(L[:, None, :], (5, times, f.size)))
 
 
+@pytest.mark.parametrize("precision", [cfdx.FP64, cfdx.MIXED], ids=["fp64", "mixed"])
+@pytest.mark.parametrize("batch", [False, True], ids=["block", "batch"])
+def test_streaming_accesses_give_the_bits_of_plain_ones(ctx, batch, precision):
+    """Rows that are whole 64-byte pieces as they are: the small block is stepped with plain accesses, the one that
+    repeats it along k past the last-level cache with non-temporal ones, by itself and in a batch with others."""
+    d, xyz, geo = box(64, 43, (0,) * 6, 7, precision)
+    prm = cfdx.default_params(mach=0.4, reyl=900.0)
+    flow = perturbed(xyz[cfdx.owned_index(d)], 0.4, 2.0)
+    times = (384 << 20) // ((304 if precision == cfdx.MIXED else 512) * 64 * 43 * NK) + 1
+    big = cfdx.BlockDesc.from_buffer_copy(d)
+    big.nk = NK * times
+    out, dt = [], None
+    for x, n in ((d, 1), (big, times)):
+        b = cfdx.Block.of(x, ctx=ctx)
+        b.set_geometry_soa(np.tile(geo.reshape(22, 1, -1), (1, n, 1)).reshape(-1))
+        b.configure(0.4, 0.0, prm)
+        b.set_flow(np.tile(flow, n))
+        dt = dt or 0.5 * b.cfl_dt(0.5)
+        b.configure(0.4, dt, prm)
+        if batch:
+            others = [cfdx.Block(s, 12, 10, precision=precision, ctx=ctx) for s in (16, 21)]
+            q = cfdx.Batch(precision, ctx)
+            for o in others:
+                o.init_case(grid="box", length=(2 * math.pi,) * 3, init="tgv", mach=0.4)
+                o.configure(0.4, 1e-3, prm)
+                q.add(o)
+            q.add(b)
+            q.step(2, False)
+        else:
+            b.step(2, 0.4, dt, prm)
+        out.append(b.get_flow())
+        if batch:
+            q.close()
+            for o in others:
+                o.close()
+        b.close()
+    for c in FIELDS:
+        assert np.array_equal(out[1][c].reshape(times, -1), np.broadcast_to(out[0][c], (times, flow.size))), c
+
+
 def test_geometry_built_on_the_device_in_long_rows(ctx):
     """The sinusoidal map and its Taylor-Green state, from the host's arrays and from the device's set-up: the
     same formulas through two libraries' sines, a few ulp apart in the metrics (1e-15), and the right-hand side
