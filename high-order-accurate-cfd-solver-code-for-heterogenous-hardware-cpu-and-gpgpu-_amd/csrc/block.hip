@@ -337,7 +337,10 @@ void drop_graph(cfdx_batch *q)
 // with room. us a step of all blocks in one list and in groups, mixed and FP64: eight cubes of 32^3 .. 128^3
 // 2205 -> 1910 and 3730 -> 3560; the four C-grids of the served ladder 1949 -> 1758 and 2959 -> 2776; twelve 64^3
 // 1305 -> 1183 (three a group, 239 MB) and 2272 -> 2025 (two, 268 MB; three, 402 MB: 2240; one: 2135); three 128^3 2837 ->
-// 2614 and 4800 -> 4652; twenty-four 32^3 mixed in one list of 239 MB 376, eight a group 430.
+// 2614 and 4800 -> 4652; twenty-four 32^3 mixed in one list of 239 MB 376, eight a group 430. Lists not far past the size
+// (small blocks, one list and groups): 39 cubes of 32^3 mixed (370 MB) 633 and 553, 21 FP64 (336 MB) 632 and 552; C-grids
+// of 128x64x16, eight mixed (348 MB) 643 and 581, five FP64 (366 MB) 615 and 559. Just past it one list can
+// be the better: seventeen C-grids of 96x32x8 FP64 (257 MB) 438 and 460.
 constexpr uint64_t GROUP_BYTES = (uint64_t)256 << 20;
 static_assert(GROUP_BYTES <= cfdx::blk::STREAM_BYTES, "a group of several blocks does not stream");
 std::vector<std::vector<size_t>> group_blocks(const std::vector<cfdx_block *> &blocks)

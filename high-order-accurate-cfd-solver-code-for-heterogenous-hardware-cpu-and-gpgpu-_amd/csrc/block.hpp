@@ -90,9 +90,10 @@ __host__ __device__ inline uint32_t shell_columns(const BlockDev &B)
 
 // Shell tiles: 256 nodes of the rows, 64 or 256 of the columns. A column node's neighbours share no cache line
 // with the next node's, so a wave's loads take 32 lines each and few columns are bound by the address rate of
-// the few CUs they are on: up to COLUMNS_SPREAD nodes they go over four times the CUs. C-grids, FP64 and mixed, us
-// a step with 256 and with 64: 128x64x16 (3840 column nodes) 176 and 136, 153 and 113; 192x96x24 (8832) 371 and 269,
-// 369 and 263; 256x128x32 (15872) 915 and 572, 921 and 579.
+// the few CUs they are on: up to COLUMNS_SPREAD nodes they go over four times the CUs. C-grids, us a step with 256
+// and with 64, FP64: 128x64x16 (3840 column nodes) 168 and 146, 192x96x24 (8832) 352 and 347, 192x96x28 (10304) 427 and 426,
+// 224x112x28 (12096) 634 and 637, 256x112x30 (12960) 722 and 725, 256x128x32 (15872) 857 and 863; mixed: 132 and 104, 258 and
+// 241, 282 and 268, 359 and 354, 438 and 435, 552 and 549. The line lies where the two types' gain and loss meet.
 constexpr uint32_t SHELL_TILE = 256, COLUMNS_SPREAD = 12288;
 __host__ __device__ inline uint32_t shell_column_tile(const BlockDev &B) { return shell_columns(B) <= COLUMNS_SPREAD ? 64u : 256u; }
 __host__ __device__ inline uint32_t shell_row_tiles(const BlockDev &B) { return (shell_rows(B) + SHELL_TILE - 1) / SHELL_TILE; }

@@ -408,7 +408,7 @@ __device__ __forceinline__ void visc_shell_tile(const BlockDev *__restrict__ blk
 }
 
 // Node tiles of the list first (tile ids through the XCD remap), then, for lists with bounded
-// blocks, nblk x shell_tiles shell tiles of TX * TY shell nodes each (block = id / shell_tiles),
+// blocks, nblk x shell_tiles shell tiles of up to TX * TY shell nodes each (SHELL_TILE; block = id / shell_tiles),
 // dispatched last in plain order so that they spread over the XCDs at the end of the launch.
 template <typename S, int TX, int TY, int K, bool LOOP>
 __global__ void __launch_bounds__(TX *TY, ((TY >= 4 && !(LOOP && list_bounded(K))) || sizeof(S) == 4 ? 4 : 3))
@@ -679,12 +679,13 @@ __global__ void __launch_bounds__(256, (TA == 64 ? 3 : 4)) k_face(const BlockDev
 }
 
 // The viscous node tiles and the three face sweeps of a stage in one launch (tile variants 0). They
-// depend on nothing of each other, and apart each launch ends with a tail and a gap: when it was made, a stage of 64^3
-// took 87 us in five launches and 71 in two (FP64; mixed 59 and 42), 128^3 546 and 511 (325 and 294), 256^3 4.26 ms and
-// 4.19 (2.43 and 2.40); now 57 us (37), 510 (286) and 4.25 ms (2.38). At 256^3 it takes 2.78 ms FP64 and 1.59 mixed, moves
-// 11.0 and 5.9 GB through the L2 and issues 8.6e8 and 8.0e8 wave instructions: FP64 65-70 % of the issue slots at the 1.9
-// GHz that the card's power limit leaves, 3.96 TB/s; mixed all of them (an FP32 instruction takes an issue slot like an
-// FP64 one). Each XCD takes its own contiguous share of every kind of tile and runs through them
+// depend on nothing of each other, and apart each launch ends with a tail and a gap. Untimed steps of the same build, apart
+// and together, us, FP64: 64^3 213 and 176, 96^3 766 and 686, 128^3 1615 and 1548, 160^3 3153 and 3088, 256^3 12745 and
+// 12880, 320^3 25227 and 25608; mixed: 146 and 111, 407 and 354, 938 and 872, 1809 and 1776, 7234 and 7206, 14009 and
+// 14136: from 256^3 on it no longer pays, by 1 to 1.5 % in FP64. At 256^3 it takes 2.9 ms FP64 and 1.6 mixed, moves 11.0
+// and 5.9 GB through the L2 (its kinds apart 11.2 and 6.1) and issues 8.6e8 and 7.9e8 wave instructions: FP64 62 % of the
+// issue slots at the 1.9 GHz that the card's power limit leaves, 3.8 TB/s; mixed all of them (an FP32 instruction takes
+// an issue slot like an FP64 one). Each XCD takes its own contiguous share of every kind of tile and runs through them
 // FLUX_CHUNK tiles of a kind at a time: with the kinds alternating tile by tile they fall into step
 // with the CUs (each CU draws tiles of one kind; 256^3 8 % slower in FP64, 23 % mixed), 4 and 16 are
 // best, a kind's whole share at a time 1 % slower at 256^3 FP64 and 3 % at 128^3 mixed.
@@ -1098,8 +1099,9 @@ __global__ void __launch_bounds__(256) k_bc(const BlockDev *__restrict__ blks, i
 // The side conditions of the i and j directions of blocks bounded in either, in one launch: i first, then
 // j, as k_bc one after the other. Workgroups 0 .. planes - 1 take the two i sides of a k plane each and,
 // after them, the j sides of the four columns at either end, the only ones that read what the i sides
-// wrote or write what they read; the other workgroups take the j sides of the columns between. (Two
-// launches of 6-7 us each on a C-grid of any size of the served ladder.)
+// wrote or write what they read; the other workgroups take the j sides of the columns between. 384x128x32: 15.6 us,
+// where two launches of 7.2 us each were: a plane's workgroup does its i sides and then its end columns, so the launch
+// saves the gap between two and no kernel time.
 constexpr int BC_IJ = 512, BC_END = 4;
 template <typename S>
 __global__ void __launch_bounds__(BC_IJ) k_bc_ij(const BlockDev *__restrict__ blks, uint32_t planes, int mode)
