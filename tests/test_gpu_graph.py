@@ -6,6 +6,8 @@ import numpy as np
 import pytest
 
 import cfdx
+from cfdx import serve
+from test_gpu_serve import small_stream
 from test_gpu_tiles import ragged
 
 pytestmark = pytest.mark.gpu
@@ -115,3 +117,23 @@ def test_a_destroyed_block_takes_the_graph_with_it(ctx):
     q.close()
     a.close()
     c.close()
+
+
+@pytest.mark.parametrize("clock", ["steps", "wall"])
+def test_served_requests_of_a_batch_that_captures(ctx, clock):
+    """A server whose batch has a capped grid captures its step again at every admission and retirement, on the wall
+    clock beside the set-up thread's own library calls: every result is that of the request alone."""
+    reqs = small_stream()
+    for r in reqs:
+        r.nsteps *= 3
+        if clock == "wall":
+            r.arrival *= 1e-3
+    srv = serve.Server(precision=cfdx.MIXED, ctx=ctx, reserve_bytes=0, chunk=4, graph=True, grid_cap=9)
+    res = srv.run(reqs, clock=clock)
+    srv.close()
+    assert sorted(res) == [r.rid for r in reqs] and srv.peak_active >= 2
+    for r in reqs:
+        want = serve.run_alone(r, cfdx.MIXED, ctx)
+        assert res[r.rid].dt == want.dt
+        for f in FIELDS[:5]:
+            assert np.array_equal(res[r.rid].flow[f], want.flow[f]), (r.rid, f)
